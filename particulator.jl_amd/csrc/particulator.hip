@@ -73,14 +73,17 @@ constexpr int NCOUNT = MAX_PROCS + 1;
 // run derives them on the device (tfinal = t + dt, then t = tfinal and step + 1 at the end
 // of the step: the same arithmetic as the host loop t += dt), so replays of one graph
 // advance the time.
+constexpr int MAX_SUB = 16;  // steps of one launch at most
 struct Clock {
     double t, dt, tfinal;
     uint32_t step, qpar;  // qpar: which work queue of each species is the input
     ull cursor;           // work items claimed by the push/select kernel
     ull ecur;             // queued collisions claimed by the sampling kernel
     ull nmark[PT_NSPECIES];  // population counts where the last secondary pass starts
-    uint32_t pass, pad2;     // 0: the step's main pass; > 0: passes over its secondaries
+    uint32_t pass;           // 0: the launch's main pass; > 0: passes over its secondaries
+    uint32_t nsub;           // steps of this launch
     ull tcur;                // items claimed in the current pass of the one-workgroup tail
+    double tf[MAX_SUB];      // their final times
 };
 
 // Work queues of the event rounds: per species two ping-pong queues of particles to
@@ -197,7 +200,9 @@ struct Shared {
     // memory each read would be a vector load whose wait also waits for every memory
     // operation issued before it)
     Field field0;
-    const double* fields_lds;  // several swarms: their E, B vectors in the dynamic LDS
+    const double* fields_lds;  // homogeneous fields: the swarms' E, B vectors in the dynamic LDS
+    double tf[MAX_SUB];  // the final times of the launch's steps (nsub of them)
+    int nsub, pad;
 };
 
 __device__ __forceinline__ void stage(const Params& P, double* lds, Shared& sh) {
@@ -211,6 +216,8 @@ __device__ __forceinline__ void stage(const Params& P, double* lds, Shared& sh) 
             const FieldFn& f = (q % 6) < 3 ? P.fields[q / 6].e : P.fields[q / 6].b;
             lds[P.lds_field_off + q] = f.v[q % 3];
         }
+    if (threadIdx.x < MAX_SUB) sh.tf[threadIdx.x] = P.clock->tf[threadIdx.x];
+    if (threadIdx.x == 0) sh.nsub = (int)P.clock->nsub;
     for (int s = 0; s < PT_NSPECIES; s++) {
         const DevTable& tb = P.tab[s];
         const SpeciesDev& S = P.sp[s];
@@ -324,7 +331,6 @@ __device__ __forceinline__ void deposit(const Params& P, BlockCounters& bc, doub
 // add_particle!, src/population.jl:103-113 (+ birth tallies of untracked species; the energy
 // of a particle born below the cut is left where it is born)
 constexpr ull NO_SLOT = ~0ull;
-constexpr int NCHILD = 2;
 
 // A slot of species sp2's store for each lane here with `want`: the lanes that call this
 // together and want a slot of the same species share one atomic on its counter and take
@@ -356,7 +362,7 @@ __device__ __forceinline__ ull claim_slots(const Shared& sh, int sp2, bool want)
 __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, const V3& x,
                                       const V3& p, double w, double t, double s, uint64_t puid,
                                       uint32_t step, uint32_t dend, int k, int swarm, bool main_pass,
-                                      double tfinal) {
+                                      uint32_t mark) {
     const SpLite& L = sh.sp[sp2];
     double E = kinenergy(sp2, p);
     bool store = true;
@@ -404,8 +410,7 @@ __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, cons
     L.uid[slot] = child_uid(P.seed, puid, step, dend, k);
     L.swarm[slot] = swarm;
     L.active[slot] = 1;
-    L.trem[slot] = tfinal - t;
-    L.draw[slot] = 0;
+    L.draw[slot] = mark;
     atomicAdd(&sh.bc.work[W_SECONDARIES], 1ull);
     if (main_pass) atomicAdd(&sh.bc.work[W_MAIN_SEC], 1ull);
     return slot;
@@ -427,9 +432,24 @@ __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, cons
 // a short window of consecutive slots: refills read whole cache lines and neighbouring
 // write-backs meet in L2.
 //
-// Collisions are sampled in the lane; the secondaries a lane creates are advanced by that
-// lane right after their parent (up to NCHILD pending per lane; the rest are left to the
-// tail passes, which skip every particle already at tfinal).
+// A launch carries its particles through up to MAX_SUB steps (MULTI): particles do not
+// interact, and a step's stream and rate bound depend on the particle alone, so a lane goes
+// on to the next step of its particle in registers, with the arithmetic of the step
+// boundary (droplow!'s cut, the times t += dt, setr!, a fresh stream) and without the record's
+// way to memory and back, the launches between steps and the wait for the step's slowest
+// wave.  10^7 electrons, 8 steps a launch: 2.50 -> 2.36 ms a step; 41,000 electrons: 253 ->
+// 168 us; a pencil beam of 2 x 10^6 photons, where the wait is for the electron with the most
+// collisions: 75 -> 26 ms (with the repeated pushes of E).
+//
+// Collisions are sampled in the lane.  The secondaries it stores go on a stack in LDS that
+// the wave's free lanes take from before new items; those that find it full are left to the
+// passes over the launch's secondaries (the `draw` column holds the step each was born in,
+// and the number of steps once it is done).
+//
+// Lanes reach their next collision at different times: of a wave's 64, about 40 end a push in
+// a collision and 24 at the end of a step.  When enough lanes could still reach theirs, they
+// push once more before the wave goes through the collision code (MORE_LANES; 10^7 electrons:
+// 2.39 -> 2.33 ms a step with 12 to 20 lanes, 2.45 with 28).
 // EVENT = true (collision rounds): a selected real collision of a sampler kind in
 // P.defer_mask is not sampled here; the particle is written back with its time left and
 // stream position and queued for that sampler kind (wave-aggregated appends), and the
@@ -440,6 +460,8 @@ __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, cons
 // and the sweep's 512-thread workgroups)
 __device__ __forceinline__ ull claim_chunk() { return blockDim.x > 256 ? 256ull : 128ull; }
 enum { SRC_RANGE = 0, SRC_QUEUE = 1 };
+// a further push round before the collisions, when at least MORE_LANES lanes can use it
+constexpr int MORE_ROUNDS = 1, MORE_LANES = 20;
 
 struct Loaded {
     V3 x, p;
@@ -506,8 +528,12 @@ struct RbebJob {
     double first;  // uniform number d0 of the stream when d0 is odd (a cached block's half)
     uint64_t uid;
     uint32_t d0, k;  // stream position before the loop, trips evaluated so far
+    uint32_t step, pad;
 };
-constexpr int COOP_WAVE_BYTES = 64 * (int)sizeof(RbebJob) + 64;
+// a wave's LDS area: the RBEB jobs and their rank table, then its stack of secondaries
+constexpr int STACK = 64;
+constexpr int COOP_JOB_BYTES = 64 * (int)sizeof(RbebJob) + 64;
+constexpr int COOP_WAVE_BYTES = COOP_JOB_BYTES + 8 * STACK;
 
 // The rejection loops of the wave's pending RBEB collisions (_rbeb_sample,
 // src/rbeb.jl:170-196), run by every lane of the wave together.  Trip k of a particle uses
@@ -516,8 +542,8 @@ constexpr int COOP_WAVE_BYTES = 64 * (int)sizeof(RbebJob) + 64;
 // a particle takes its first accepting trip.  Result and stream position are those of the
 // sequential loop; the wave runs about log(n) rounds instead of the longest particle's
 // trip count.  Called by the whole wave; `pending` lanes have written their job.
-__device__ __forceinline__ void rbeb_coop(const Params& P, char* wlds, int lane, uint64_t ltmask, uint32_t step,
-                                          bool& pending, double& wout, PhiloxStream& g) {
+__device__ __forceinline__ void rbeb_coop(const Params& P, char* wlds, int lane, uint64_t ltmask, bool& pending,
+                                          double& wout, PhiloxStream& g) {
     RbebJob* jobs = (RbebJob*)wlds;
     uint8_t* rank_lane = (uint8_t*)(wlds + 64 * sizeof(RbebJob));
     const uint32_t k0 = (uint32_t)P.seed, k1 = (uint32_t)(P.seed >> 32);
@@ -538,7 +564,7 @@ __device__ __forceinline__ void rbeb_coop(const Params& P, char* wlds, int lane,
             const RbebJob& J = jobs[ow];
             D = J.d0 + 2u * (J.k + (uint32_t)j);
             blk = (D + 1) >> 1;  // the block of the trip's second draw
-            uint32_t a = (uint32_t)J.uid, b = (uint32_t)(J.uid >> 32), c = step, e = blk;
+            uint32_t a = (uint32_t)J.uid, b = (uint32_t)(J.uid >> 32), c = J.step, e = blk;
             philox10(a, b, c, e, k0, k1);
             c0b = u01(a, b);
             c1b = u01(c, e);
@@ -652,11 +678,14 @@ __device__ __forceinline__ int swarm_of(const Params& P, int32_t sw) { return (s
 
 template <int SRC, bool EVENT, bool WALL = false, bool MLP = false>
 __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* wlds, const ull* rb, const ull* re,
-                                            ull* cursor, double tfinal, uint32_t step, bool main_pass,
-                                            int par) {
-    // range passes load a retiring lane's next item ahead (3b); a lane that retires ends its
-    // step without a collision, so it neither queues one (EVENT) nor runs a network (MLP)
+                                            ull* cursor, uint32_t step0, bool main_pass, int par) {
+    // range passes load a retiring lane's next item ahead (D); a lane that retires ends its
+    // last step without a collision, so it neither queues one (EVENT) nor runs a network (MLP)
     constexpr bool AHEAD = SRC == SRC_RANGE;
+    // range passes with every collision in place advance their particles through several
+    // steps; the others through one
+    constexpr bool MULTI = SRC == SRC_RANGE && !EVENT;
+    const int K = MULTI ? sh.nsub : 1;
     const ull n0 = re[0] - rb[0], n1 = re[1] - rb[1], n2 = re[2] - rb[2];
     const ull total = n0 + n1 + n2;
     const uint32_t foff = P.forcing_off;  // read once: the loop below does not reload it
@@ -666,6 +695,10 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
     const ull chunk = claim_chunk();
     ull cbeg = 0, cend = 0;
     bool drained = false;
+    // the wave's secondaries waiting to be advanced (LDS, last in first out)
+    uint64_t* const stk = (uint64_t*)(wlds + COOP_JOB_BYTES);
+    int nstk = 0;  // wave-uniform
+    int extra = 0;  // push rounds since the wave's last collision phase (wave-uniform)
     // lane state
     bool have = false;
     int sp = 0, swarm = 0;
@@ -677,141 +710,248 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
     g.init(0, 0, 0);
     uint32_t iters = 0, nev = 0;
     uint32_t n_events = 0, n_psteps = 0, n_tail = 0;  // the lane's work counts
-    bool active = false, oob = false, child = false;
-    int nch = 0;
-    int chsp[NCHILD];
-    ull chidx[NCHILD];
+    bool active = false, oob = false;
+    bool child = false;  // born in the step it is in (counted apart)
+    bool born = false;   // born in this launch: marked when it is done
+    bool pend = false;   // its push ended in a collision, which is still to be selected
+    bool new_r = false;  // its rate bound is to be recomputed
+    double cE = 0.0;     // kinetic energy at the pending collision
+    int ks = 0;          // the step it is in (0..K-1)
+    // the item loaded ahead for this lane
+    bool ahead = false;
+    int nsp = 0;
+    ull nidx = 0;
+    Loaded na;
+    na.act = 0;
+    // an item that was just read becomes the lane's particle if it has a step to do from
+    // step k0 on; `ch`: it was born in step k0
+    auto take = [&](int qs, ull qi, const Loaded& a, int k0, bool ch, bool bo) {
+        int k = k0;
+        double cr = sh.tf[k] - a.t;
+        if constexpr (MULTI) {
+            while (!(cr > EPS64) && ++k < K) {
+                cr = sh.tf[k] - a.t;
+                ch = false;
+            }
+        }
+        if (a.act == 0 || !(cr > EPS64)) return;
+        sp = qs;
+        idx = qi;
+        x = a.x;
+        p = a.p;
+        w = a.w;
+        t = a.t;
+        s = a.s;
+        uid = a.uid;
+        swarm = swarm_of(P, a.swarm);
+        trem = cr;
+        oob = false;
+        new_r = true;
+        ks = k;
+        g.init(P.seed, uid, step0 + (uint32_t)k);
+        iters = 0;
+        nev = 0;
+        active = true;
+        have = true;
+        child = ch;
+        born = bo;
+    };
     for (;;) {
-        // 1. pending secondaries of this lane
-        {
-            while (!have && nch > 0) {
-                nch--;
-                int csp = nch == 0 ? chsp[0] : chsp[1];
-                ull cidx = nch == 0 ? chidx[0] : chidx[1];
-                Loaded a = load_slot(sh.sp[csp], cidx);
-                if constexpr (AHEAD) wait_vmem();
-                double cr = tfinal - a.t;
-                if (a.act != 0 && cr > EPS64) {
-                    sp = csp;
-                    idx = cidx;
-                    x = a.x;
-                    p = a.p;
-                    w = a.w;
-                    t = a.t;
-                    s = a.s;
-                    uid = a.uid;
-                    swarm = swarm_of(P, a.swarm);
-                    trem = cr;
-                    oob = false;
-                    r = setr(sh.sp[sp], kinenergy(sp, p), swarm, oob);
-                    g.init(P.seed, uid, step);
-                    iters = 0;
-                    nev = 0;
-                    active = true;
-                    have = true;
-                    child = true;
+        const bool first = !MULTI || extra == 0;
+        // A. the end of a particle's step: droplow!'s cut, then its next step, or back to
+        //    memory.  A lane whose next item is loaded waits for the first push round after
+        //    a collision phase, when its loads have had that phase's time.
+        if (have && !pend && (!(trem > EPS64) || !active) && (first || !ahead)) {
+            const SpLite& L = sh.sp[sp];
+            // droplow!: the energy is computed only where |p|^2 does not settle the test
+            if (active && !(dot3(p, p) > L.ppcut_hi)) {
+                double Ek = kinenergy(sp, p);
+                if (Ek < L.cut) {
+                    active = false;
+                    deposit(P, sh.bc, Ek * w, x.z);
                 }
             }
-        }
-        // 2. free lanes take the next items of the wave's chunk, in lane order
-        uint64_t need = __ballot(!have);
-        while (need && !drained) {
-            if (cbeg >= cend) {
-                int fl = __ffsll((unsigned long long)__ballot(1)) - 1;
-                ull b = 0;
-                if (lane == fl) b = global_add(cursor, chunk);
-                b = __shfl(b, fl);
-                if (b >= total) {
-                    drained = true;
-                    break;
-                }
-                cbeg = b;
-                cend = b + chunk < total ? b + chunk : total;
+            // a collision at the very end of the step: the record gets the new rate bound
+            if (new_r) {
+                r = setr(L, kinenergy(sp, p), swarm, oob);
+                new_r = false;
             }
-            ull q = cbeg + (ull)__popcll(need & ltmask);
-            ull cnt = (ull)__popcll(need);
-            bool mine = !have && q < cend;
-            cbeg = cbeg + cnt < cend ? cbeg + cnt : cend;
-            if (mine) {
-                int qs;
-                ull qi;
-                if (q < n0) {
-                    qs = 0;
-                    qi = rb[0] + q;
-                } else if (q < n0 + n1) {
-                    qs = 1;
-                    qi = rb[1] + (q - n0);
-                } else {
-                    qs = 2;
-                    qi = rb[2] + (q - n0 - n1);
-                }
-                bool qchild = !main_pass;
-                if constexpr (SRC == SRC_QUEUE) {
-                    uint32_t e = P.q.work[qs][par][qi];
-                    qchild = (e & CHILD_BIT) != 0;
-                    qi = e & ~CHILD_BIT;
-                }
-                const SpLite& Lq = sh.sp[qs];
-                Loaded a = load_slot(Lq, qi);
-                double cr;
-                uint32_t d0 = 0;
-                if constexpr (SRC == SRC_QUEUE) {
-                    cr = Lq.trem[qi];
-                    d0 = Lq.draw[qi];
-                } else {
-                    if constexpr (AHEAD) wait_vmem();
-                    cr = tfinal - a.t;
-                }
-                // queued particles are active and always enter (one with no time left is
-                // only finished); range items enter when active with time left
-                if (SRC == SRC_QUEUE || (a.act != 0 && cr > EPS64)) {
-                    sp = qs;
-                    idx = qi;
-                    x = a.x;
-                    p = a.p;
-                    w = a.w;
-                    t = a.t;
-                    s = a.s;
-                    uid = a.uid;
-                    swarm = swarm_of(P, a.swarm);
-                    trem = cr;
-                    oob = false;
-                    if constexpr (SRC == SRC_QUEUE) {
-                        r = PF(Lq.f[PT_R], qi);  // set by the sampler (setr! of apply!) or at birth
-                    } else {
-                        r = setr(Lq, kinenergy(qs, p), swarm, oob);
+            if (oob) atomicAdd(&sh.bc.flags[FLAG_RANGE], 1ull);
+            n_events += nev;
+            if (child)
+                n_tail++;
+            else
+                n_psteps++;
+            bool cont = false;
+            if constexpr (MULTI) {
+                if (active) {
+                    while (++ks < K) {
+                        trem = sh.tf[ks] - t;
+                        if (trem > EPS64) {
+                            cont = true;
+                            break;
+                        }
                     }
-                    g.init(P.seed, uid, step);
-                    g.resume(d0);
-                    iters = 0;
-                    nev = 0;
-                    active = true;
-                    have = true;
-                    child = qchild;
                 }
             }
-            need = __ballot(!have);
+            if (cont) {
+                // the next step's advance_init!: a new rate bound and random stream
+                g.init(P.seed, uid, step0 + (uint32_t)ks);
+                iters = 0;
+                nev = 0;
+                oob = false;
+                child = false;
+                new_r = true;
+            } else {
+                // the item loaded ahead: its loads are waited for here, before the stores
+                // below, so that the wait is not a wait for those stores too
+                if (AHEAD && ahead) wait_vmem();
+                __builtin_amdgcn_sched_barrier(0);
+                // the particle's record: 72 contiguous bytes (w unchanged), written in whole
+                // sectors, four of the five stores 16 bytes wide
+                {
+                    PT_GLOBAL pair2* w2 = rec_pairs(L, idx);
+                    const pair2 v0 = {x.x, x.y}, v1 = {x.z, p.x}, v2 = {p.y, p.z}, v4 = {s, r};
+                    w2[0] = v0;
+                    w2[1] = v1;
+                    w2[2] = v2;
+                    PF(L.f[PT_T], idx) = t;
+                    w2[4] = v4;
+                }
+                if (!active) L.active[idx] = 0;
+                if (MULTI && born && K > 1) L.draw[idx] = (uint32_t)K;
+                have = false;
+                if (AHEAD && ahead) {
+                    ahead = false;
+                    take(nsp, nidx, na, 0, !main_pass, false);
+                }
+            }
         }
-        // 3. the wave leaves when its items are claimed and no lane holds a particle
-        if (drained && __ballot(have) == 0) break;
-        // 3b. a lane whose push reaches the end of the step without a collision retires in
-        //     this iteration (6): it claims its next item now and loads it while the push,
-        //     the wave's collisions and the other lanes' work run, and takes it when it
-        //     writes its particle back.  Without this the load is issued when the lane is
-        //     free and used at once, so the lane waits for it, and, since memory operations
-        //     complete in order for that wait, also for the stores of the write-back just
-        //     before.
-        const double tnext0 = s / r;
-        bool ahead = false;  // an item is loaded for this lane: nsp, nidx, na
-        int nsp = 0;
-        ull nidx = 0;
-        Loaded na;
-        // read only where ahead is set; a default that is not a constant keeps the compiler
-        // from turning the test of the loaded byte into a lane mask right at the load
-        na.act = (uint32_t)iters;
+        // B. free lanes take the wave's waiting secondaries, then the next items of its chunk,
+        //    in lane order
+        if (first) {
+            uint64_t need = __ballot(!have);
+            while (need) {
+                const int rank = __popcll(need & ltmask), nfree = __popcll(need);
+                const int pop = nfree < nstk ? nfree : nstk;
+                bool mine = false, ch = !main_pass, bo = false;
+                int qs = 0, k0 = 0;
+                ull qi = 0;
+                if (!have && rank < pop) {
+                    const uint64_t e = stk[nstk - 1 - rank];
+                    qi = e & 0xFFFFFFFFull;
+                    qs = (int)(e >> 32) & 0xFF;
+                    k0 = (int)(e >> 40);
+                    ch = bo = true;
+                    mine = true;
+                }
+                nstk -= pop;
+                const int want = nfree - pop;
+                if (want > 0 && !drained) {
+                    if (cbeg >= cend) {
+                        int fl = __ffsll((unsigned long long)__ballot(1)) - 1;
+                        ull b = 0;
+                        if (lane == fl) b = global_add(cursor, chunk);
+                        b = __shfl(b, fl);
+                        if (b >= total) {
+                            drained = true;
+                        } else {
+                            cbeg = b;
+                            cend = b + chunk < total ? b + chunk : total;
+                        }
+                    }
+                    const ull q = cbeg + (ull)(rank - pop);
+                    if (!have && rank >= pop && q < cend) {
+                        if (q < n0) {
+                            qs = 0;
+                            qi = rb[0] + q;
+                        } else if (q < n0 + n1) {
+                            qs = 1;
+                            qi = rb[1] + (q - n0);
+                        } else {
+                            qs = 2;
+                            qi = rb[2] + (q - n0 - n1);
+                        }
+                        mine = true;
+                    }
+                    cbeg = cbeg + (ull)want < cend ? cbeg + (ull)want : cend;
+                }
+                if (__ballot(mine) == 0) break;
+                if (mine) {
+                    if constexpr (SRC == SRC_QUEUE) {
+                        // queued particles are active and always enter (one with no time left
+                        // is only finished); secondaries on the stack enter as in a range
+                        const bool queued = !bo;
+                        if (queued) {
+                            const uint32_t e = P.q.work[qs][par][qi];
+                            ch = (e & CHILD_BIT) != 0;
+                            qi = e & ~CHILD_BIT;
+                        }
+                        const SpLite& Lq = sh.sp[qs];
+                        const Loaded a = load_slot(Lq, qi);
+                        if (queued) {
+                            const double cr = Lq.trem[qi];
+                            const uint32_t d0 = Lq.draw[qi];
+                            sp = qs;
+                            idx = qi;
+                            x = a.x;
+                            p = a.p;
+                            w = a.w;
+                            t = a.t;
+                            s = a.s;
+                            uid = a.uid;
+                            swarm = swarm_of(P, a.swarm);
+                            trem = cr;
+                            oob = false;
+                            r = PF(Lq.f[PT_R], qi);  // set by the sampler (setr! of apply!) or at birth
+                            new_r = false;
+                            g.init(P.seed, uid, step0);
+                            g.resume(d0);
+                            iters = 0;
+                            nev = 0;
+                            active = true;
+                            have = true;
+                            child = ch;
+                            born = false;
+                        } else {
+                            take(qs, qi, a, 0, ch, false);
+                        }
+                    } else {
+                        const Loaded a = load_slot(sh.sp[qs], qi);
+                        // a pass over secondaries of several steps: the step each was born in,
+                        // or K when it has been advanced already
+                        if (MULTI && K > 1 && !main_pass && !bo) {
+                            k0 = (int)sh.sp[qs].draw[qi];
+                            bo = true;
+                        }
+                        wait_vmem();
+                        if (k0 < K) take(qs, qi, a, k0, ch, bo);
+                    }
+                }
+                need = __ballot(!have);
+            }
+            // C. the wave leaves when its items are claimed and no lane holds a particle
+            if (drained && nstk == 0 && __ballot(have) == 0) break;
+        }
+        // setr! for a particle that changed: after its collision, at the start of a step, or
+        // newly taken (one evaluation for all these lanes)
+        if (new_r) {
+            r = setr(sh.sp[sp], kinenergy(sp, p), swarm, oob);
+            new_r = false;
+        }
+        const double tnext = s / r;
+        // D. a lane whose push reaches the end of its last step without a collision retires at
+        //    the next A: it claims its next item now and loads it while the push, the wave's
+        //    collisions and the other lanes' work run, and takes it when it writes its particle
+        //    back.  Without this the load is issued when the lane is free and used at once, so
+        //    the lane waits for it, and, since memory operations complete in order for that
+        //    wait, also for the stores of the write-back just before.
         if constexpr (AHEAD) {
-            // (a lane with secondaries on its list takes them first, as it did before)
-            const bool ends = have && nch == 0 && trem > EPS64 && active && !(trem > tnext0);
+            // (waiting secondaries are taken first; a pass over secondaries of several steps
+            // reads their birth steps in B)
+            const bool ends = first && nstk == 0 && (main_pass || K == 1) && have && !pend && ks == K - 1 && trem > EPS64 && active &&
+                              !(trem > tnext);
+            bool got = false;
             uint64_t want = __ballot(ends);
             while (want && !drained) {
                 if (cbeg >= cend) {
@@ -828,7 +968,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                 }
                 const ull q = cbeg + (ull)__popcll(want & ltmask);
                 const ull cnt = (ull)__popcll(want);
-                const bool mine = ends && !ahead && q < cend;
+                const bool mine = ends && !got && q < cend;
                 cbeg = cbeg + cnt < cend ? cbeg + cnt : cend;
                 if (mine) {
                     if (q < n0) {
@@ -841,33 +981,26 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                         nsp = 2;
                         nidx = rb[2] + (q - n0 - n1);
                     }
-                    ahead = true;
+                    got = true;
                 }
-                want = __ballot(ends && !ahead);
+                want = __ballot(ends && !got);
             }
             // issued after the claim loop and read nowhere before the write-back: values
             // that a loop carried, or a flag tested here, would make the wave wait for the
             // loads at once
-            if (ahead) na = load_slot(sh.sp[nsp], nidx);
+            if (got) {
+                na = load_slot(sh.sp[nsp], nidx);
+                ahead = true;
+            }
         }
-        // 4. one push of this lane's particle and, at the end of it, the selection; a real
-        //    collision is finished in 6, after the wave's RBEB rejection loops (5)
-        ull* qc = nullptr;
-        uint32_t* qa = nullptr;
-        uint32_t qv = 0;
-        int qsel = -1;          // collision queued for the sampling kernel
-        int csel = -1;          // collision sampled in 6
-        double cE = 0.0;        // its kinetic energy
-        bool rb_wait = false;   // an RBEB collision waiting for the cooperative loop
-        double rb_w = -1.0;
-        bool new_r = false;     // the lane's rate bound is recomputed in 8
-        if (have && trem > EPS64 && active) {
+        // E. one push of this lane's particle.  In a further push round a lane whose push would
+        //    end its last step waits, so that it loads its next item ahead.
+        if (have && !pend && trem > EPS64 && active && (first || ks < K - 1 || trem > tnext)) {
             const SpLite& L = sh.sp[sp];
             if (++iters > ITER_LIMIT || g.exhausted()) {
                 atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
                 trem = 0.0;
             } else {
-                const double tnext = tnext0;
                 double dt;
                 bool coll;
                 if (trem > tnext) {
@@ -880,60 +1013,112 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                 }
                 const V3 xo = x, po = p;
                 const double to = t;
-                if (P.nswarm == 1) {
-                    push(sp, sh.field0, x, p, t, dt, foff);
-                } else if (P.field_lds) {
+                V3 dx{0, 0, 0}, dp{0, 0, 0};
+                bool uniform;  // the force does not depend on the position
+                if (P.field_lds) {
                     const PT_LDS double* fv = as_lds(sh.fields_lds) + 6 * swarm;
                     const HomField hf{{fv}, {fv + 3}, {{nullptr, nullptr}}};
-                    push(sp, hf, x, p, t, dt, foff);
+                    push_delta(sp, hf, x, p, dt, foff, dx, dp);
+                    uniform = true;
+                } else if (P.nswarm == 1) {
+                    push_delta(sp, sh.field0, x, p, dt, foff, dx, dp);
+                    uniform = sp == PT_PHOTON;
                 } else {
-                    push(sp, as_global(P.fields)[swarm], x, p, t, dt, foff);
+                    push_delta(sp, as_global(P.fields)[swarm], x, p, dt, foff, dx, dp);
+                    uniform = sp == PT_PHOTON;
                 }
+                if (foff & off_push(sp)) {
+                    dx = V3{0, 0, 0};  // only its time advances
+                } else {
+                    x = V3{x.x + dx.x, x.y + dx.y, x.z + dx.z};
+                    p = V3{p.x + dp.x, p.y + dp.y, p.z + dp.z};
+                }
+                t = t + dt;
                 if constexpr (WALL) wall_check(P, sp, xo, po, to, x, p, w, t, uid, swarm, active);
+                trem -= dt;
                 if (coll && r != 0.0 && (!WALL || active)) {
-                    double E = kinenergy(sp, p);
+                    const double E = kinenergy(sp, p);
                     if (E >= L.cut) {
                         nev++;
-                        double t1, t2;
-                        bool o;
-                        int iv = precheb(E, L.k, L.xmax, L.ixmax, t1, t2, o);
-                        oob |= o;
-                        double xi = g.next() * r;
-                        const int sel = select_process(as_lds(L.rate) + (size_t)iv * L.nprocs * 3, L.nprocs, t1,
-                                                       t2, xi);
-                        if (sel < 0) {
-                            if (!(xi >= 0.0)) atomicAdd(&sh.bc.flags[FLAG_RATEBOUND], 1ull);
-                            atomicAdd(&sh.bc.counts[sp * NCOUNT], 1ull);
-                            new_r = true;  // setr! of the null collision (p unchanged): in 8
-                            s = nextcoll(g);
-                        } else {
-                            atomicAdd(&sh.bc.counts[sp * NCOUNT + 1 + sel], 1ull);
-                            const DevProc& pr = sh.procs[sp][sel];
-                            if (EVENT && ((P.defer_mask >> pr.kind) & 1u)) {
-                                qsel = sel;
-                            } else {
-                                csel = sel;
-                                cE = E;
-                                if (pr.kind == PT_PROC_RBEB) {
-                                    RbebJob& J = ((RbebJob*)wlds)[lane];
-                                    J.s = rbeb_setup(E, pr);
-                                    J.first = g.c1;
-                                    J.uid = uid;
-                                    J.d0 = g.draw;
-                                    J.k = 0;
-                                    rb_wait = true;
-                                }
-                            }
+                        cE = E;
+                        pend = true;
+                    } else if (MULTI && !WALL && uniform && p.x == po.x && p.y == po.y && p.z == po.z) {
+                        // Below the cut a particle moves on in pushes of s / r until the step
+                        // ends (s is not drawn again, src/collisions.jl:151).  This push left
+                        // its momentum as it was and depends on nothing else, so the next
+                        // ones repeat it.
+                        while (trem > tnext && iters < ITER_LIMIT) {
+                            iters++;
+                            x = V3{x.x + dx.x, x.y + dx.y, x.z + dx.z};
+                            t = t + dt;
+                            trem -= dt;
                         }
                     }
                 }
-                trem -= dt;
             }
         }
-        // 5. every lane of the wave runs the pending RBEB rejection loops
-        rbeb_coop(P, wlds, lane, ltmask, step, rb_wait, rb_w, g);
-        // 5b. learned samplers: the wave's bremsstrahlung and Moller collisions whose network
-        //     is in use go through it on the matrix cores, one kind at a time
+        if constexpr (MULTI) {
+            // F. another push round before the collisions: when no lane has one, or when
+            //    enough lanes can still reach theirs
+            const uint64_t pends = __ballot(pend);
+            if (pends == 0) {
+                extra = 0;
+                continue;
+            }
+            const bool ready = have && !pend && active && (trem > EPS64 ? ks < K - 1 || trem > tnext : ks < K - 1);
+            if (extra < MORE_ROUNDS && __popcll(__ballot(ready)) >= MORE_LANES) {
+                extra++;
+                continue;
+            }
+            extra = 0;
+        }
+        // G. the selection; a real collision is finished in I, after the wave's RBEB rejection
+        //    loops (H)
+        ull* qc = nullptr;
+        uint32_t* qa = nullptr;
+        uint32_t qv = 0;
+        int qsel = -1;          // collision queued for the sampling kernel
+        int csel = -1;          // collision sampled in I
+        bool rb_wait = false;   // an RBEB collision waiting for the cooperative loop
+        double rb_w = -1.0;
+        if (pend) {
+            const SpLite& L = sh.sp[sp];
+            pend = false;
+            double t1, t2;
+            bool o;
+            int iv = precheb(cE, L.k, L.xmax, L.ixmax, t1, t2, o);
+            oob |= o;
+            double xi = g.next() * r;
+            const int sel = select_process(as_lds(L.rate) + (size_t)iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
+            if (sel < 0) {
+                if (!(xi >= 0.0)) atomicAdd(&sh.bc.flags[FLAG_RATEBOUND], 1ull);
+                atomicAdd(&sh.bc.counts[sp * NCOUNT], 1ull);
+                new_r = true;  // setr! of the null collision (p unchanged)
+                s = nextcoll(g);
+            } else {
+                atomicAdd(&sh.bc.counts[sp * NCOUNT + 1 + sel], 1ull);
+                const DevProc& pr = sh.procs[sp][sel];
+                if (EVENT && ((P.defer_mask >> pr.kind) & 1u)) {
+                    qsel = sel;
+                } else {
+                    csel = sel;
+                    if (pr.kind == PT_PROC_RBEB) {
+                        RbebJob& J = ((RbebJob*)wlds)[lane];
+                        J.s = rbeb_setup(cE, pr);
+                        J.first = g.c1;
+                        J.uid = uid;
+                        J.d0 = g.draw;
+                        J.step = g.step;
+                        J.k = 0;
+                        rb_wait = true;
+                    }
+                }
+            }
+        }
+        // H. every lane of the wave runs the pending RBEB rejection loops
+        rbeb_coop(P, wlds, lane, ltmask, rb_wait, rb_w, g);
+        // learned samplers: the wave's bremsstrahlung and Moller collisions whose network
+        // is in use go through it on the matrix cores, one kind at a time
         float ly0 = 0.0f, ly1 = 0.0f;
         bool lnet = false;
         if constexpr (MLP) {
@@ -946,62 +1131,60 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
             for (int which = 0; which < NLEARN; which++)
                 if (__ballot(lnet && lw == which)) learned_pass(P, sh, which, lnet && lw == which, sp, csel, cE, g, ly0, ly1);
         }
-        // 6. the sampled collision, then the end of the particle's step
-        if (have) {
-            const SpLite& L = sh.sp[sp];
-            if (csel >= 0) {
-                const double E = cE;
-                double pn = norm3(p);
-                // the two common kinds draw their azimuth first here: one draw site for both
-                const int kind = sh.procs[sp][csel].kind;
-                double phi = -1.0;
-                if (kind == PT_PROC_ELASTIC || (kind == PT_PROC_RBEB && rb_w >= 0.0)) phi = TWO_PI * g.next();
-                // without a dose tally a secondary below the cut leaves nothing behind
-                const double dropcut = P.dose_bins > 0 ? -1.0 : sh.cut[PT_ELECTRON] * (1.0 - 1e-9);
-                Ev e;
-                if (MLP && lnet) learned_event(sh.procs[sp][csel], sp, E, ly0, ly1, g, e);
-                else sample_event(sh.procs[sp][csel], sp, p, pn, E, P.sb, P.pe, g, e, rb_w, phi, dropcut);
-                if (e.err) atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
-                if (e.dep != 0.0) deposit(P, sh.bc, e.dep * w, x.z);
-                V3 m0, m1;
-                double s0, s1;
-                bool drop1;
-                finish_event(p, pn, e, g, m0, m1, s0, s1, sh.cut, sh.stored, dropcut, drop1);
-                uint32_t dend = g.draw;
-                if (e.keep) {
-                    p = m0;
-                    s = s0;
-                    new_r = true;  // setr! of apply!: at the end of the iteration
-                } else {
-                    active = false;
-                    ull sl = append(P, sh, e.sp0, x, m0, w, t, s0, uid, step, dend, 0, swarm, main_pass, tfinal);
-                    if (sl != NO_SLOT && nch < NCHILD) {
-                        if (nch == 0) {
-                            chsp[0] = e.sp0;
-                            chidx[0] = sl;
-                        } else {
-                            chsp[1] = e.sp0;
-                            chidx[1] = sl;
-                        }
-                        nch++;
-                    }
-                }
-                if (e.ne == 2 && !drop1) {
-                    ull sl = append(P, sh, e.sp1, x, m1, w, t, s1, uid, step, dend, e.keep ? 0 : 1, swarm, main_pass,
-                                    tfinal);
-                    if (sl != NO_SLOT && nch < NCHILD) {
-                        if (nch == 0) {
-                            chsp[0] = e.sp1;
-                            chidx[0] = sl;
-                        } else {
-                            chsp[1] = e.sp1;
-                            chidx[1] = sl;
-                        }
-                        nch++;
-                    }
-                }
+        // I. the sampled collision
+        ull sl0 = NO_SLOT, sl1 = NO_SLOT;  // slots of the secondaries it stored
+        int cs0 = 0, cs1 = 0;
+        if (csel >= 0) {
+            const double E = cE;
+            double pn = norm3(p);
+            // the two common kinds draw their azimuth first here: one draw site for both
+            const int kind = sh.procs[sp][csel].kind;
+            double phi = -1.0;
+            if (kind == PT_PROC_ELASTIC || (kind == PT_PROC_RBEB && rb_w >= 0.0)) phi = TWO_PI * g.next();
+            // without a dose tally a secondary below the cut leaves nothing behind
+            const double dropcut = P.dose_bins > 0 ? -1.0 : sh.cut[PT_ELECTRON] * (1.0 - 1e-9);
+            Ev e;
+            if (MLP && lnet) learned_event(sh.procs[sp][csel], sp, E, ly0, ly1, g, e);
+            else sample_event(sh.procs[sp][csel], sp, p, pn, E, P.sb, P.pe, g, e, rb_w, phi, dropcut);
+            if (e.err) atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
+            if (e.dep != 0.0) deposit(P, sh.bc, e.dep * w, x.z);
+            V3 m0, m1;
+            double s0, s1;
+            bool drop1;
+            finish_event(p, pn, e, g, m0, m1, s0, s1, sh.cut, sh.stored, dropcut, drop1);
+            const uint32_t dend = g.draw;
+            if (e.keep) {
+                p = m0;
+                s = s0;
+                new_r = true;  // setr! of apply!
+            } else {
+                active = false;
+                cs0 = e.sp0;
+                sl0 = append(P, sh, e.sp0, x, m0, w, t, s0, uid, g.step, dend, 0, swarm, main_pass, (uint32_t)ks);
             }
-            if (EVENT && qsel >= 0) {
+            if (e.ne == 2 && !drop1) {
+                cs1 = e.sp1;
+                sl1 = append(P, sh, e.sp1, x, m1, w, t, s1, uid, g.step, dend, e.keep ? 0 : 1, swarm, main_pass,
+                             (uint32_t)ks);
+            }
+        }
+        // the secondaries wait on the wave's stack for its free lanes; those that find it full
+        // are left to the passes over the step's secondaries
+        if (__ballot(sl0 != NO_SLOT || sl1 != NO_SLOT)) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const ull sl = q ? sl1 : sl0;
+                const uint64_t m = __ballot(sl != NO_SLOT);
+                const int at = nstk + __popcll(m & ltmask);
+                if (sl != NO_SLOT && at < STACK)
+                    stk[at] = sl | (uint64_t)(q ? cs1 : cs0) << 32 | (uint64_t)(uint32_t)ks << 40;
+                nstk = nstk + __popcll(m) < STACK ? nstk + __popcll(m) : STACK;
+            }
+            wave_lds_order();
+        }
+        if constexpr (EVENT) {
+            if (qsel >= 0) {
+                const SpLite& L = sh.sp[sp];
                 // queued for its sampler: the state after the push, the time left and the
                 // stream position (r and s are replaced when the collision is applied)
                 PF(L.f[PT_X], idx) = x.x;
@@ -1021,75 +1204,9 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                 if (oob) atomicAdd(&sh.bc.flags[FLAG_RANGE], 1ull);
                 n_events += nev;
                 have = false;
-            } else if (!(trem > EPS64) || !active) {
-                // droplow!: the energy is computed only where |p|^2 does not settle the test
-                if (active && !(dot3(p, p) > L.ppcut_hi)) {
-                    double Ek = kinenergy(sp, p);
-                    if (Ek < L.cut) {
-                        active = false;
-                        deposit(P, sh.bc, Ek * w, x.z);
-                    }
-                }
-                // a collision at the very end of the step: the record gets the new rate bound
-                if (new_r) {
-                    r = setr(L, kinenergy(sp, p), swarm, oob);
-                    new_r = false;
-                }
-                // the item loaded in 3b: its loads are waited for here, before the stores
-                // below, so that the wait is not a wait for those stores too
-                double ncr = 0.0;
-                bool ntake = false;
-                if (AHEAD && ahead) {
-                    wait_vmem();
-                    ncr = tfinal - na.t;
-                    ntake = na.act != 0 && ncr > EPS64;
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                // the particle's record: 72 contiguous bytes (w unchanged), written in whole
-                // sectors, four of the five stores 16 bytes wide
-                {
-                    PT_GLOBAL pair2* w2 = rec_pairs(L, idx);
-                    const pair2 v0 = {x.x, x.y}, v1 = {x.z, p.x}, v2 = {p.y, p.z}, v4 = {s, r};
-                    w2[0] = v0;
-                    w2[1] = v1;
-                    w2[2] = v2;
-                    PF(L.f[PT_T], idx) = t;
-                    w2[4] = v4;
-                }
-                if (!active) L.active[idx] = 0;
-                if (oob) atomicAdd(&sh.bc.flags[FLAG_RANGE], 1ull);
-                n_events += nev;
-                if (child)
-                    n_tail++;
-                else
-                    n_psteps++;
-                have = false;
-                if (AHEAD && ntake) {
-                    sp = nsp;
-                    idx = nidx;
-                    x = na.x;
-                    p = na.p;
-                    w = na.w;
-                    t = na.t;
-                    s = na.s;
-                    uid = na.uid;
-                    swarm = swarm_of(P, na.swarm);
-                    trem = ncr;
-                    oob = false;
-                    new_r = true;  // its rate bound: at the end of the iteration
-                    g.init(P.seed, uid, step);
-                    iters = 0;
-                    nev = 0;
-                    active = true;
-                    have = true;
-                    child = !main_pass;
-                }
             }
+            wave_push(qc, qa, qv, lane, ltmask);
         }
-        // 8. setr! for a particle that changed in this iteration: after its collision, or
-        //    the item a retiring lane took (one evaluation for both kinds of lane)
-        if (new_r) r = setr(sh.sp[sp], kinenergy(sp, p), swarm, oob);
-        if constexpr (EVENT) wave_push(qc, qa, qv, lane, ltmask);
     }
     // the lane's work counts, kept in registers (an LDS atomic per retiring lane on one
     // address would serialise the wave's lanes every iteration)
@@ -1099,7 +1216,8 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
 }
 
 // ------------------------------------------------------------------ step kernels
-__global__ void k_snapshot(const Params* __restrict__ Pp, int clocked, double tfinal, uint32_t step) {
+__global__ void k_snapshot(const Params* __restrict__ Pp, int clocked, double tfinal, double dt, uint32_t step,
+                           int nsub) {
     const Params& P = *Pp;
     int s = threadIdx.x;
     Clock& C = *P.clock;
@@ -1112,12 +1230,16 @@ __global__ void k_snapshot(const Params* __restrict__ Pp, int clocked, double tf
     }
     for (int q = threadIdx.x; q < NQCNT; q += blockDim.x) P.q.cnt[q] = 0;
     if (s == 0) {
-        if (clocked) {
-            C.tfinal = C.t + C.dt;
-        } else {
-            C.tfinal = tfinal;
-            C.step = step;
+        // the steps' final times, by the host loop's arithmetic (t += dt)
+        double tf = clocked ? C.t + C.dt : tfinal;
+        const double d = clocked ? C.dt : dt;
+        for (int k = 0; k < MAX_SUB; k++) {
+            C.tf[k] = tf;
+            if (k == nsub - 1) C.tfinal = tf;
+            tf = tf + d;
         }
+        C.nsub = (uint32_t)nsub;
+        if (!clocked) C.step = step;
         C.cursor = 0;
         C.ecur = 0;
         C.qpar = 0;
@@ -1148,7 +1270,7 @@ __global__ void k_tick(const Params* __restrict__ Pp) {
     Clock& C = *Pp->clock;
     if (threadIdx.x == 0) {
         C.t = C.tfinal;
-        C.step += 1;
+        C.step += C.nsub;
     }
 }
 
@@ -1204,8 +1326,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
     if (skip) return;
     stage(P, lds, sh);
     char* wlds = (char*)lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES;
-    select_loop<SRC, EVENT, WALL, MLP>(P, sh, wlds, rb, re, &P.clock->cursor, C.tfinal, C.step,
-                                  SRC == SRC_RANGE && C.pass == 0, par);
+    select_loop<SRC, EVENT, WALL, MLP>(P, sh, wlds, rb, re, &P.clock->cursor, C.step,
+                                       SRC == SRC_RANGE && C.pass == 0, par);
     flush_counters(P, &sh.bc);
 }
 
@@ -1318,17 +1440,18 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
             } else {
                 L.active[idx] = 0;
                 atomicAdd(&sh.bc.work[child ? W_TAIL : W_PSTEPS], 1ull);
-                ull sl = append(P, sh, e.sp0, x, m0, w, t, s0, uid, step, dend, 0, swarm, false, tfinal);
+                ull sl = append(P, sh, e.sp0, x, m0, w, t, s0, uid, step, dend, 0, swarm, false, 0);
                 if (sl != NO_SLOT) {
+                    sh.sp[e.sp0].trem[sl] = tfinal - t;
                     c1 = P.q.cnt + QWK(e.sp0, nxt);
                     a1 = P.q.work[e.sp0][nxt];
                     v1 = (uint32_t)sl | CHILD_BIT;
                 }
             }
             if (e.ne == 2) {
-                ull sl = append(P, sh, e.sp1, x, m1, w, t, s1, uid, step, dend, e.keep ? 0 : 1, swarm, false,
-                                tfinal);
+                ull sl = append(P, sh, e.sp1, x, m1, w, t, s1, uid, step, dend, e.keep ? 0 : 1, swarm, false, 0);
                 if (sl != NO_SLOT) {
+                    sh.sp[e.sp1].trem[sl] = tfinal - t;
                     c2 = P.q.cnt + QWK(e.sp1, nxt);
                     a2 = P.q.work[e.sp1][nxt];
                     v2 = (uint32_t)sl | CHILD_BIT;
@@ -1356,7 +1479,6 @@ __global__ void __launch_bounds__(512) k_tail(const Params* __restrict__ Pp, int
     // global atomics (an LDS address used as a global one is an invalid access)
     ull* const cur = &P.clock->tcur;
     stage(P, lds, sh);
-    const double tfinal = P.clock->tfinal;
     const uint32_t step = P.clock->step;
     if (threadIdx.x == 0)
         for (int s = 0; s < PT_NSPECIES; s++) beg[s] = P.clock->nmark[s];
@@ -1383,7 +1505,7 @@ __global__ void __launch_bounds__(512) k_tail(const Params* __restrict__ Pp, int
             re[s] = end[s];
         }
         select_loop<SRC_RANGE, false, WALL, MLP>(P, sh, (char*)lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES,
-                                            rb, re, cur, tfinal, step, false, 0);
+                                                 rb, re, cur, step, false, 0);
         __threadfence();
         __syncthreads();
         if (threadIdx.x == 0)
@@ -2361,7 +2483,10 @@ static int noalloc_scratch(pt_ctx* c) {
 static int dalloc(pt_ctx* c, void** p, size_t bytes) {
     if (bytes == 0) bytes = 8;
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) return fail(c, PT_E_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here: a later launch's check must not find it
+        return fail(c, PT_E_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    }
     c->allocs.push_back(*p);
     return PT_OK;
 }
@@ -2379,7 +2504,7 @@ static int sync_params(pt_ctx* c) {
     }
     // several swarms with homogeneous fields: their E and B vectors in LDS (one swarm's
     // field is staged in the static block)
-    bool hom = c->cfg.nswarm > 1 && c->cfg.nswarm <= MAX_LDS_FIELDS;
+    bool hom = c->cfg.nswarm <= MAX_LDS_FIELDS;
     for (const Field& F : c->hfields)
         hom = hom && F.e.kind == PT_FIELD_HOMOGENEOUS && F.b.kind == PT_FIELD_HOMOGENEOUS && !F.cl.on;
     c->hp.field_lds = hom ? 1 : 0;
@@ -2426,7 +2551,10 @@ struct Scratch {
 template <class T>
 static int dscratch(pt_ctx* c, Scratch<T>& s, size_t count) {
     hipError_t e = hipMalloc((void**)&s.p, sizeof(T) * (count ? count : 1));
-    if (e != hipSuccess) return fail(c, PT_E_NOMEM, "scratch allocation of %zu bytes failed", sizeof(T) * count);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(c, PT_E_NOMEM, "scratch allocation of %zu bytes failed", sizeof(T) * count);
+    }
     return PT_OK;
 }
 
@@ -3092,7 +3220,7 @@ static int launch_kernel_args(pt_ctx* c, int v, bool full) {
 
 // one step.  clocked: tfinal and the step index come from the device clock (captured
 // runs); otherwise they are given and the host counts steps.
-static int launch_step(pt_ctx* c, bool clocked, double tfinal) {
+static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int nsub) {
     int rc = ensure_residency(c);
     if (rc) return rc;
     const int R = c->launch.rounds;
@@ -3102,7 +3230,8 @@ static int launch_step(pt_ctx* c, bool clocked, double tfinal) {
     if (wall && R > 0) return fail(c, PT_E_STATE, "a wall needs collision rounds = 0");
     if (wall && mlp) return fail(c, PT_E_STATE, "a wall needs the learned samplers off");
     if (R > 0 && (rc = ensure_queues(c))) return rc;
-    hipLaunchKernelGGL(k_snapshot, dim3(1), dim3(64), 0, c->stream, c->dp, clocked ? 1 : 0, tfinal, c->step);
+    hipLaunchKernelGGL(k_snapshot, dim3(1), dim3(64), 0, c->stream, c->dp, clocked ? 1 : 0, tfinal, dt, c->step,
+                       nsub);
     HIPCHK(c, hipGetLastError());
     hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr;
     const bool prof = c->profile && !clocked;
@@ -3143,10 +3272,14 @@ static int launch_step(pt_ctx* c, bool clocked, double tfinal) {
         hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, c->stream, c->dp);
         HIPCHK(c, hipGetLastError());
     } else {
-        c->step++;
+        c->step += (uint32_t)nsub;
     }
     return PT_OK;
 }
+
+// steps that one launch may advance: collision rounds queue particles between kernels and
+// take one step at a time
+static int steps_per_launch(const pt_ctx* c) { return c->launch.rounds > 0 ? 1 : MAX_SUB; }
 
 static int check_flags(pt_ctx* c, int64_t* out) {
     ull f[NFLAGS];
@@ -3175,7 +3308,7 @@ int pt_advance(pt_ctx* c, double tfinal) {
     if (rc) return rc;
     rc = sync_params(c);
     if (rc) return rc;
-    rc = launch_step(c, false, tfinal);
+    rc = launch_step(c, false, tfinal, 0.0, 1);
     if (rc) return rc;
     rc = read_counts(c);
     if (rc) return rc;
@@ -3235,16 +3368,20 @@ int pt_run(pt_ctx* c, double t0, double dt, int nsteps, int compact_every, int c
     if (rc) return rc;
     if (check_every < 1) check_every = 1;
     double t = t0;
-    for (int q = 0; q < nsteps; q++) {
-        rc = launch_step(c, false, t + dt);
+    for (int q = 0; q < nsteps;) {
+        // the steps up to the next compaction, check or the end in one launch
+        int k = std::min(nsteps - q, check_every - q % check_every);
+        if (compact_every > 0) k = std::min(k, compact_every - q % compact_every);
+        k = std::min(k, steps_per_launch(c));
+        rc = launch_step(c, false, t + dt, dt, k);
         if (rc) return rc;
-        t += dt;
-        bool last = q == nsteps - 1;
-        if (compact_every > 0 && (q + 1) % compact_every == 0) {
+        for (int i = 0; i < k; i++) t += dt;
+        q += k;
+        if (compact_every > 0 && q % compact_every == 0) {
             rc = compact_all(c, -1, c->profile);
             if (rc) return rc;
         }
-        if (last || (q + 1) % check_every == 0) {
+        if (q == nsteps || q % check_every == 0) {
             rc = read_counts(c);
             if (rc) return rc;
             rc = check_flags(c, nullptr);
@@ -3296,7 +3433,11 @@ static int capture(pt_ctx* c, int which, int steps, bool compact) {
     if (c->launch.rounds > 0 && (rc = ensure_queues(c))) return rc;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int lrc = PT_OK;
-    for (int q = 0; q < steps && lrc == PT_OK; q++) lrc = launch_step(c, true, 0.0);
+    for (int q = 0; q < steps && lrc == PT_OK;) {
+        const int k = std::min(steps - q, steps_per_launch(c));
+        lrc = launch_step(c, true, 0.0, 0.0, k);
+        q += k;
+    }
     if (lrc == PT_OK && compact) lrc = compact_all(c, -1, false);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &g);
@@ -3411,10 +3552,13 @@ int pt_autotune(pt_ctx* c, double t0, double dt, int trial_steps, pt_tune_trial*
         ull p0, p1;
         if ((r2 = psteps_now(c, &p0))) return r2;
         HIPCHK(c, hipEventRecord(a, c->stream));
-        for (int q = 0; q < steps; q++) {
-            if ((r2 = launch_step(c, false, t + dt))) return r2;
-            t += dt;
-            if (ce > 0 && (q + 1) % ce == 0 && (r2 = compact_all(c, -1, false))) return r2;
+        for (int q = 0; q < steps;) {
+            int k = std::min(steps - q, steps_per_launch(c));
+            if (ce > 0) k = std::min(k, ce - q % ce);
+            if ((r2 = launch_step(c, false, t + dt, dt, k))) return r2;
+            for (int i = 0; i < k; i++) t += dt;
+            q += k;
+            if (ce > 0 && q % ce == 0 && (r2 = compact_all(c, -1, false))) return r2;
         }
         HIPCHK(c, hipEventRecord(b, c->stream));
         HIPCHK(c, hipEventSynchronize(b));
@@ -3683,7 +3827,10 @@ int pt_synchronize(pt_ctx* c) {
     Scratch<T> var;                                                                           \
     do {                                                                                      \
         hipError_t e_ = hipMalloc((void**)&var.p, sizeof(T) * ((count) ? (count) : 1));      \
-        if (e_ != hipSuccess) return fail((c), PT_E_NOMEM, "scratch allocation failed");      \
+        if (e_ != hipSuccess) {                                                               \
+            (void)hipGetLastError();                                                          \
+            return fail((c), PT_E_NOMEM, "scratch allocation failed");                        \
+        }                                                                                     \
     } while (0)
 
 int pt_debug_philox(pt_ctx* c, const uint32_t* ctr, const uint32_t key[2], uint32_t* out, size_t n) {

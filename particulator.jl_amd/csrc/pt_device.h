@@ -770,14 +770,11 @@ __device__ __forceinline__ V3 force(int sp, const FT& f, const V3& x, const V3& 
     return F;
 }
 
-// advance_particle(::RK2Pusher, y, dt), src/pusher.jl:41-63; a species the pusher is
-// restricted away from (RestrictedPusher, NullPusher, :66-76) only has its time advanced
+// advance_particle(::RK2Pusher, y, dt), src/pusher.jl:41-63: what a push by dt adds to the
+// position and the momentum
 template <class FT>
-__device__ __forceinline__ void push(int sp, const FT& f, V3& x, V3& p, double& t, double dt, uint32_t off) {
-    if (off & off_push(sp)) {
-        t = t + dt;
-        return;
-    }
+__device__ __forceinline__ void push_delta(int sp, const FT& f, const V3& x, const V3& p, double dt, uint32_t off,
+                                           V3& dx, V3& dp) {
     V3 v1 = velocity(sp, p);
     V3 f1 = force(sp, f, x, p, v1, off);
     double dt2 = 2.0 * dt;
@@ -788,12 +785,22 @@ __device__ __forceinline__ void push(int sp, const FT& f, V3& x, V3& p, double& 
           p.z + div_const(dt2 * f1.z, 3.0, THIRD)};
     V3 v2 = velocity(sp, p2);
     V3 f2 = force(sp, f, x2, p2, v2, off);
-    x.x = x.x + dt * (v1.x / 4.0 + 3.0 * v2.x / 4.0);
-    x.y = x.y + dt * (v1.y / 4.0 + 3.0 * v2.y / 4.0);
-    x.z = x.z + dt * (v1.z / 4.0 + 3.0 * v2.z / 4.0);
-    p.x = p.x + dt * (f1.x / 4.0 + 3.0 * f2.x / 4.0);
-    p.y = p.y + dt * (f1.y / 4.0 + 3.0 * f2.y / 4.0);
-    p.z = p.z + dt * (f1.z / 4.0 + 3.0 * f2.z / 4.0);
+    dx = V3{dt * (v1.x / 4.0 + 3.0 * v2.x / 4.0), dt * (v1.y / 4.0 + 3.0 * v2.y / 4.0),
+            dt * (v1.z / 4.0 + 3.0 * v2.z / 4.0)};
+    dp = V3{dt * (f1.x / 4.0 + 3.0 * f2.x / 4.0), dt * (f1.y / 4.0 + 3.0 * f2.y / 4.0),
+            dt * (f1.z / 4.0 + 3.0 * f2.z / 4.0)};
+}
+
+// the push itself; a species the pusher is restricted away from (RestrictedPusher,
+// NullPusher, src/pusher.jl:66-76) only has its time advanced
+template <class FT>
+__device__ __forceinline__ void push(int sp, const FT& f, V3& x, V3& p, double& t, double dt, uint32_t off) {
+    if (!(off & off_push(sp))) {
+        V3 dx, dp;
+        push_delta(sp, f, x, p, dt, off, dx, dp);
+        x = V3{x.x + dx.x, x.y + dx.y, x.z + dx.z};
+        p = V3{p.x + dp.x, p.y + dp.y, p.z + dp.z};
+    }
     t = t + dt;
 }
 
