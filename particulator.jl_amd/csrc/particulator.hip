@@ -173,7 +173,7 @@ struct SpLite {
     ull cap;
     const double* rate;  // LDS
     const double* rb;    // LDS (one swarm) or global
-    double cut, xmax, ixmax;  // ixmax = 1 / xmax
+    double cut, xmax, ixmax, two_k1;  // ixmax = 1 / xmax, two_k1 = 2^(k+1)
     // |p|^2 above which the kinetic energy is certainly above the cut: the cut's |p|^2
     // times 1 + 1e-9, far beyond the rounding of the energy computed from |p|^2
     double ppcut_hi;
@@ -206,6 +206,7 @@ struct Shared {
 };
 
 __device__ __forceinline__ void stage(const Params& P, double* lds, Shared& sh) {
+    for (int q = threadIdx.x; q < MATH_DOUBLES; q += blockDim.x) lds[q] = g_math[q];
     for (int q = threadIdx.x; q < (int)(sizeof(BlockCounters) / sizeof(ull)); q += blockDim.x)
         ((ull*)&sh.bc)[q] = 0;
     static_assert(sizeof(Field) % sizeof(ull) == 0, "Field is copied in 8-byte words");
@@ -245,6 +246,7 @@ __device__ __forceinline__ void stage(const Params& P, double* lds, Shared& sh) 
             }
             L.xmax = tb.xmax;
             L.ixmax = 1.0 / tb.xmax;
+            L.two_k1 = ldexp(1.0, tb.k + 1);
             L.rate = lds + P.lds_rate_off[s];
             L.rb = P.rb_in_lds ? lds + P.lds_rb_off[s] : tb.ratebound;
             L.rb_lds = P.rb_in_lds;
@@ -271,7 +273,7 @@ __device__ __forceinline__ double setr(const SpLite& L, double E, int swarm, boo
     if (E < L.cut) return 0.0;
     double t1, t2;
     bool o;
-    int i = precheb(E, L.k, L.xmax, L.ixmax, t1, t2, o);
+    int i = precheb(E, L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o);
     oob |= o;
     const size_t off = (size_t)(L.nswarm > 1 ? swarm : 0) * (L.k + 1) * 3 + i * 3;
     return L.rb_lds ? cheb3(as_lds(L.rb) + off, t1, t2) : cheb3(as_global(L.rb) + off, t1, t2);
@@ -543,7 +545,7 @@ constexpr int COOP_WAVE_BYTES = COOP_JOB_BYTES + 8 * STACK;
 // sequential loop; the wave runs about log(n) rounds instead of the longest particle's
 // trip count.  Called by the whole wave; `pending` lanes have written their job.
 __device__ __forceinline__ void rbeb_coop(const Params& P, char* wlds, int lane, uint64_t ltmask, bool& pending,
-                                          double& wout, PhiloxStream& g) {
+                                          double& wout, StepStream& g) {
     RbebJob* jobs = (RbebJob*)wlds;
     uint8_t* rank_lane = (uint8_t*)(wlds + 64 * sizeof(RbebJob));
     const uint32_t k0 = (uint32_t)P.seed, k1 = (uint32_t)(P.seed >> 32);
@@ -706,7 +708,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
     V3 x{0, 0, 0}, p{0, 0, 0};
     double w = 0, t = 0, s = 0, r = 0, trem = 0;
     uint64_t uid = 0;
-    PhiloxStream g;
+    StepStream g;
     g.init(0, 0, 0);
     uint32_t iters = 0, nev = 0;
     uint32_t n_events = 0, n_psteps = 0, n_tail = 0;  // the lane's work counts
@@ -1086,7 +1088,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
             pend = false;
             double t1, t2;
             bool o;
-            int iv = precheb(cE, L.k, L.xmax, L.ixmax, t1, t2, o);
+            int iv = precheb(cE, L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o);
             oob |= o;
             double xi = g.next() * r;
             const int sel = select_process(as_lds(L.rate) + (size_t)iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
@@ -1104,7 +1106,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                     csel = sel;
                     if (pr.kind == PT_PROC_RBEB) {
                         RbebJob& J = ((RbebJob*)wlds)[lane];
-                        J.s = rbeb_setup(cE, pr);
+                        J.s = rbeb_setup(cE, pr, g.tab());
                         J.first = g.c1;
                         J.uid = uid;
                         J.d0 = g.draw;
@@ -1301,7 +1303,7 @@ __global__ void k_rotate(const Params* __restrict__ Pp) {
 // push/select over the step's particles (first round) or the input work queues
 template <int BS, int SRC, bool EVENT, bool WALL = false, bool MLP = false>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_advance(const Params* __restrict__ Pp) {
-    extern __shared__ double lds[];
+    double* const lds = pt_lds;
     __shared__ Shared sh;
     __shared__ int skip;
     const Params& P = *Pp;
@@ -1337,7 +1339,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
 // particles for the next push/select round.
 template <int BS>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_sample(const Params* __restrict__ Pp) {
-    extern __shared__ double lds[];
+    double* const lds = pt_lds;
     __shared__ Shared sh;
     __shared__ ull seg[PT_NSPECIES * NKQ + 1];
     __shared__ int skip;
@@ -1389,7 +1391,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
         double w = 0, t = 0, E = 0, pn = 1;
         uint64_t uid = 0;
         int swarm = 0, sel = 0;
-        PhiloxStream g;
+        StepStream g;
         g.init(0, 0, 0);
         if (valid) {
             ent = P.q.ev[sp][kq][pos];
@@ -1470,7 +1472,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
 // src/mixed_population.jl:43-46).
 template <bool WALL, bool MLP>
 __global__ void __launch_bounds__(512) k_tail(const Params* __restrict__ Pp, int maxpasses) {
-    extern __shared__ double lds[];
+    double* const lds = pt_lds;
     __shared__ Shared sh;
     __shared__ ull beg[PT_NSPECIES], end[PT_NSPECIES];
     __shared__ int done;
@@ -1807,7 +1809,7 @@ __global__ void k_mlp_features(const Params* __restrict__ Pp, int which, const d
 
 // init! / advance_init!: r of every active particle (src/mixed_population.jl:20-35)
 __global__ void __launch_bounds__(256) k_setr(const Params* __restrict__ Pp, int sp) {
-    extern __shared__ double lds[];
+    double* const lds = pt_lds;
     __shared__ Shared sh;
     const Params& P = *Pp;
     stage(P, lds, sh);
@@ -2249,7 +2251,7 @@ __global__ void __launch_bounds__(256) k_dbg_select(const Params* __restrict__ P
                                                     const double* E, const double* u,
                                                     const int32_t* swarm, int32_t* interval,
                                                     int32_t* proc, double* rbound) {
-    extern __shared__ double lds[];
+    double* const lds = pt_lds;
     __shared__ Shared sh;
     const Params& P = *Pp;
     stage(P, lds, sh);
@@ -2262,7 +2264,7 @@ __global__ void __launch_bounds__(256) k_dbg_select(const Params* __restrict__ P
     double r = setr(L, E[i], sw, oob);
     double t1, t2;
     bool o;
-    int iv = precheb(E[i], L.k, L.xmax, L.ixmax, t1, t2, o);
+    int iv = precheb(E[i], L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o);
     double xi = u[i] * r;
     int sel = select_process(as_lds(L.rate) + (size_t)iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
     interval[i] = o ? -1 : iv;
@@ -2493,8 +2495,8 @@ static int dalloc(pt_ctx* c, void** p, size_t bytes) {
 
 static int sync_params(pt_ctx* c) {
     if (!c->dirty) return PT_OK;
-    // LDS layout of the rate tables
-    int off = 0;
+    // LDS layout: the math table, then the rate tables
+    int off = MATH_DOUBLES;
     c->hp.rb_in_lds = c->cfg.nswarm <= 1 ? 1 : 0;
     for (int s = 0; s < PT_NSPECIES; s++) {
         c->hp.lds_rate_off[s] = off;

@@ -12,6 +12,7 @@
 
 #include "../../include/particulator_hip.h"
 #include "pt_consts.h"
+#include "pt_math.h"
 
 namespace pt {
 
@@ -32,6 +33,11 @@ __device__ __forceinline__ const PT_GLOBAL T* as_global(const T* p) {
 __device__ __forceinline__ unsigned long long global_add(unsigned long long* p, unsigned long long v) {
     return __hip_atomic_fetch_add((unsigned long long PT_GLOBAL*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+// the table of pt_math.h: in global memory, and staged at the start of the step kernels' dynamic
+// LDS
+static __device__ const double g_math[MATH_DOUBLES] = {PT_MATH_TABLE};
+extern __shared__ __attribute__((aligned(16))) double pt_lds[];
 
 constexpr int MAX_PROCS = 24;
 constexpr int MAX_INTERVALS = 64;
@@ -165,6 +171,7 @@ struct PhiloxStream {
     uint32_t draw;
     uint32_t cblk;
     double c0, c1;
+    __device__ const PT_GLOBAL double* tab() const { return as_global(g_math); }
     __device__ bool exhausted() const { return draw >= DRAW_LIMIT; }
     __device__ void init(uint64_t seed, uint64_t uid, uint32_t st) {
         k0 = (uint32_t)seed;
@@ -225,12 +232,18 @@ struct PhiloxStream {
     }
 };
 
+// the stream in the step kernels, where the math table is in LDS
+struct StepStream : PhiloxStream {
+    __device__ const PT_LDS double* tab() const { return as_lds(pt_lds); }
+};
+
 // injected uniforms (test hook): consumed in order, 0.5 once exhausted
 struct InjectedStream {
     const double* u;
     int n, pos;
     uint32_t draw;
     bool ran_out;
+    __device__ const PT_GLOBAL double* tab() const { return as_global(g_math); }
     __device__ bool exhausted() const { return ran_out; }
     __device__ __forceinline__ void skip() { (void)next(); }
     __device__ __forceinline__ double next() {
@@ -263,7 +276,7 @@ __device__ __forceinline__ uint64_t child_uid(uint64_t seed, uint64_t uid, uint3
 
 template <class G>
 __device__ __forceinline__ double nextcoll(G& g) {  // src/util.jl:17
-    return -log(g.next());
+    return -log_tab(g.next(), g.tab());
 }
 
 // ---------------------------------------------------------------- kinematics
@@ -273,7 +286,7 @@ struct V3 {
 __device__ __forceinline__ double dot3(const V3& a, const V3& b) {
     return (a.x * b.x + a.y * b.y) + a.z * b.z;
 }
-__device__ __forceinline__ double norm3(const V3& a) { return sqrt(dot3(a, a)); }
+__device__ __forceinline__ double norm3(const V3& a) { return qsqrt(dot3(a, a)); }
 
 // a / b for a constant b with inv = 1/b correctly rounded: the product a * inv is within an
 // ulp of a/b, the remainder a - q b is exact in one FMA, and one more FMA rounds the quotient
@@ -286,11 +299,18 @@ __device__ __forceinline__ double div_const(double a, double b, double inv) {
     return (r == 0.0 || r != r) ? q : fma(r, inv, q);
 }
 
-// src/electron.jl:53, src/photon.jl:52
+// the same for finite operands, without the test of the remainder
+__device__ __forceinline__ double div_const_fin(double a, double b, double inv) {
+    const double q = a * inv;
+    return fma(fma(-q, b, a), inv, q);
+}
+
+// src/electron.jl:53, src/photon.jl:52.  Photons and electrons of a wave share the root.
 __device__ __forceinline__ double kinenergy(int sp, const V3& p) {
-    double pp = dot3(p, p);
-    if (sp == PT_PHOTON) return sqrt(pp) * C;
-    return sqrt(MC2 * MC2 + C2 * pp) - MC2;
+    const double pp = dot3(p, p);
+    const bool ph = sp == PT_PHOTON;
+    const double q = qsqrt(ph ? pp : MC2 * MC2 + C2 * pp);
+    return ph ? q * C : q - MC2;
 }
 // src/electron.jl:51
 __device__ __forceinline__ double mom_from_kin(int sp, double kin) {
@@ -298,40 +318,30 @@ __device__ __forceinline__ double mom_from_kin(int sp, double kin) {
     double a = kin + MC2;
     return sqrt(a * a - MC2 * MC2) / C;
 }
-// src/electron.jl:54-56, src/photon.jl:47
+// src/electron.jl:54-56, src/photon.jl:47: p c / |p|, or p / (m gamma)
 __device__ __forceinline__ V3 velocity(int sp, const V3& p) {
-    if (sp == PT_PHOTON) {
-        double f = C / norm3(p);
-        return V3{p.x * f, p.y * f, p.z * f};
-    }
     constexpr double MC2SQ = MC2 * MC2;
-    double g = sqrt(1.0 + div_const(C2 * dot3(p, p), MC2SQ, 1.0 / MC2SQ));
-    double inv = 1.0 / (ME * g);
-    return V3{p.x * inv, p.y * inv, p.z * inv};
+    const double pp = dot3(p, p);
+    const bool ph = sp == PT_PHOTON;
+    const double q = qsqrt(ph ? pp : 1.0 + div_const_fin(C2 * pp, MC2SQ, 1.0 / MC2SQ));
+    const double f = qdiv(ph ? C : 1.0, ph ? q : ME * q);
+    return V3{p.x * f, p.y * f, p.z * f};
 }
 
 // ---------------------------------------------------------------- Chebyshev
 // precheb, src/cheby.jl:127-143 (+ chebval :57-81).  The index is clamped to [0, k]
 // (the reference reads out of bounds above xmax); `oob` reports it.
-__device__ __forceinline__ int precheb(double x, int k, double xmax, double ixmax, double& t1,
+// two_k1 = 2^(k+1).
+__device__ __forceinline__ int precheb(double x, int k, double xmax, double ixmax, double two_k1, double& t1,
                                        double& t2, bool& oob) {
-    double x1 = div_const(x, xmax, ixmax);  // x / xmax; ixmax = 1 / xmax
-    int l = 0;
-    double s;
-    if (x1 != x1) {
-        s = x1;
-        l = 0;
-    } else {
-        s = frexp(x1, &l);
-    }
-    int i = (x1 == 0.0) ? 0 : l + k;
-    double xi;
-    if (i > 0) {
-        xi = 4.0 * s - 3.0;
-    } else {
-        xi = ldexp(1.0, k + 1) * x1 - 1.0;
-        i = 0;
-    }
+    // x / xmax (ixmax = 1 / xmax) and its frexp
+    const double x1 = div_fixup(div_const_fin(x, xmax, ixmax), xmax, x);
+    const double s = frexp_mant(x1);
+    int i = (x1 == 0.0) ? 0 : frexp_exp(x1) + k;
+    // 4 s - 3, or 2^(k+1) x1 - 1 in the lowest interval (the products are exact)
+    const bool low = i <= 0;
+    const double xi = fma(low ? two_k1 : 4.0, low ? x1 : s, low ? -1.0 : -3.0);
+    i = low ? 0 : i;
     t1 = xi;
     t2 = 2.0 * xi * xi - 1.0;
     oob = i > k;
@@ -406,7 +416,7 @@ __device__ __forceinline__ double sample_rel_sr(double alpha, double beta, G& g)
     for (;;) {
         double u, z;
         g.next2(u, z);
-        x = alpha * u / (alpha + 1.0 - u);
+        x = qdiv(alpha * u, alpha + 1.0 - u);
         if (z < 1.0 - beta * beta * x || g.exhausted()) break;
     }
     return 1.0 - 2.0 * x;
@@ -421,18 +431,20 @@ struct RbebSetup {
 // The orbital's own terms come with the process (set when the table is uploaded): pr.c[0] =
 // b' = B / mc^2, pr.c[1] = log(2 b'), pr.c[2] = 1 / B.  T / mc^2 and T / B are exact
 // divisions by constants (div_const).
-__device__ __forceinline__ RbebSetup rbeb_setup(double T, const DevProc& pr) {
+template <class T_>
+__device__ __forceinline__ RbebSetup rbeb_setup(double T, const DevProc& pr, T_ tab) {
     RbebSetup s;
-    double t1 = div_const(T, MC2, 1.0 / MC2);
-    double bt2 = 1.0 - 1.0 / ((1.0 + t1) * (1.0 + t1));
+    const double t1 = div_const_fin(T, MC2, 1.0 / MC2);
+    const Recip g2((1.0 + t1) * (1.0 + t1));
+    const double bt2 = 1.0 - g2.inverse();
     const double b1 = pr.c[0];
-    s.t = div_const(T, pr.B, pr.c[2]);
-    s.A = -(1.0 + 2.0 * t1) / (s.t + 1.0) / ((1.0 + t1) * (1.0 + t1));
-    s.Cc = (log(bt2 / (1.0 - bt2)) - bt2) - pr.c[1];
-    s.M = b1 * b1 / ((1.0 + t1) * (1.0 + t1));
+    s.t = div_const_fin(T, pr.B, pr.c[2]);
+    s.A = g2(qdiv(-(1.0 + 2.0 * t1), s.t + 1.0));
+    s.Cc = (log_tab(qdiv(bt2, 1.0 - bt2), tab) - bt2) - pr.c[1];
+    s.M = g2(b1 * b1);
     s.pbn = 2.0 * 1.0 + 2.0 * s.Cc + (s.t + 1.0) * (s.t + 1.0) * 1.0 * s.M / 4.0;
-    s.ratio = (s.t + 1.0) / (s.t - 1.0);
-    s.iratio = 1.0 / s.ratio;
+    s.ratio = qdiv_any(s.t + 1.0, s.t - 1.0);
+    s.iratio = qdiv_any(1.0, s.ratio);
     return s;
 }
 // One trip: w (exact) and whether it is accepted.  The reference's 1/(1+w)^k and
@@ -441,9 +453,9 @@ __device__ __forceinline__ RbebSetup rbeb_setup(double T, const DevProc& pr) {
 // only a z * pb within ~1e-15 of p0 could be decided otherwise.
 __device__ __forceinline__ bool rbeb_trip(const RbebSetup& s, double u, double z, double& w) {
     const double den = s.ratio - u;
-    w = u / den;
+    w = qdiv(u, den);
     double tw = s.t - w;
-    double ra = den * s.iratio, rt = 1.0 / tw;
+    double ra = den * s.iratio, rt = Recip(tw).inverse();
     double ra2 = ra * ra, rt2 = rt * rt;
     double pb = s.pbn * ra2;
     double g1 = ra + rt;
@@ -454,7 +466,7 @@ __device__ __forceinline__ bool rbeb_trip(const RbebSetup& s, double u, double z
 }
 template <class G>
 __device__ __forceinline__ double rbeb_sample(double T, const DevProc& pr, G& g) {
-    const RbebSetup s = rbeb_setup(T, pr);
+    const RbebSetup s = rbeb_setup(T, pr, g.tab());
     double w;
     for (;;) {
         double u, z;
@@ -728,7 +740,7 @@ template <typename Ptr>
 __device__ __forceinline__ double chebeval_n(Ptr c, int k, int order, double xmax, double ixmax, double x) {
     double t1, t2;
     bool oob;
-    int i = precheb(x, k, xmax, ixmax, t1, t2, oob);
+    int i = precheb(x, k, xmax, ixmax, ldexp(1.0, k + 1), t1, t2, oob);
     Ptr a = c + (size_t)i * order;
     double tm2 = 1.0, tm1 = t1;
     double acc = a[0] * 1.0;
@@ -779,16 +791,16 @@ __device__ __forceinline__ void push_delta(int sp, const FT& f, const V3& x, con
     V3 f1 = force(sp, f, x, p, v1, off);
     double dt2 = 2.0 * dt;
     constexpr double THIRD = 1.0 / 3.0;
-    V3 x2{x.x + div_const(dt2 * v1.x, 3.0, THIRD), x.y + div_const(dt2 * v1.y, 3.0, THIRD),
-          x.z + div_const(dt2 * v1.z, 3.0, THIRD)};
-    V3 p2{p.x + div_const(dt2 * f1.x, 3.0, THIRD), p.y + div_const(dt2 * f1.y, 3.0, THIRD),
-          p.z + div_const(dt2 * f1.z, 3.0, THIRD)};
+    V3 x2{x.x + div_const_fin(dt2 * v1.x, 3.0, THIRD), x.y + div_const_fin(dt2 * v1.y, 3.0, THIRD),
+          x.z + div_const_fin(dt2 * v1.z, 3.0, THIRD)};
+    V3 p2{p.x + div_const_fin(dt2 * f1.x, 3.0, THIRD), p.y + div_const_fin(dt2 * f1.y, 3.0, THIRD),
+          p.z + div_const_fin(dt2 * f1.z, 3.0, THIRD)};
     V3 v2 = velocity(sp, p2);
     V3 f2 = force(sp, f, x2, p2, v2, off);
-    dx = V3{dt * (v1.x / 4.0 + 3.0 * v2.x / 4.0), dt * (v1.y / 4.0 + 3.0 * v2.y / 4.0),
-            dt * (v1.z / 4.0 + 3.0 * v2.z / 4.0)};
-    dp = V3{dt * (f1.x / 4.0 + 3.0 * f2.x / 4.0), dt * (f1.y / 4.0 + 3.0 * f2.y / 4.0),
-            dt * (f1.z / 4.0 + 3.0 * f2.z / 4.0)};
+    // dt (v1 / 4 + 3 v2 / 4): the quarters are exact and are taken out of the sum
+    const double q = dt * 0.25;
+    dx = V3{q * (v1.x + 3.0 * v2.x), q * (v1.y + 3.0 * v2.y), q * (v1.z + 3.0 * v2.z)};
+    dp = V3{q * (f1.x + 3.0 * f2.x), q * (f1.y + 3.0 * f2.y), q * (f1.z + 3.0 * f2.z)};
 }
 
 // the push itself; a species the pusher is restricted away from (RestrictedPusher,
@@ -854,15 +866,16 @@ __device__ __forceinline__ void sample_event(const DevProc& pr, int sp, const V3
         constexpr double MC2SQ = MC2 * MC2;
         const double E0 = eng, E2 = pr.B * rbeb_w, E1 = E0 - E2 - pr.B;
         const double pp = dot3(p, p);
-        const double r1 = sqrt(el ? 1.0 + div_const(C2 * pp, MC2SQ, 1.0 / MC2SQ) : E1 * E1 + 2.0 * MC2 * E1);
-        const double q = el ? 1.0 / (ME * r1) : E1 * (E0 + 2.0 * MC2) / (E0 * (E1 + 2.0 * MC2));
+        const double r1 =
+            qsqrt(el ? 1.0 + div_const_fin(C2 * pp, MC2SQ, 1.0 / MC2SQ) : E1 * E1 + 2.0 * MC2 * E1);
+        const double q = qdiv(el ? 1.0 : E1 * (E0 + 2.0 * MC2), el ? ME * r1 : E0 * (E1 + 2.0 * MC2));
         const V3 v{p.x * q, p.y * q, p.z * q};
-        const double r2 = sqrt(el ? dot3(v, v) : q);
-        const double n = div_const(el ? r2 : r1, C, 1.0 / C);
+        const double r2 = qsqrt(el ? dot3(v, v) : q);
+        const double n = div_const_fin(el ? r2 : r1, C, 1.0 / C);
         e.phi = phi >= 0.0 ? phi : TWO_PI * g.next();
         if (el) {  // src/relativistic_coulomb.jl:10-23
             const double a = pr.c[0];
-            const double al = HBAR * HBAR / (4.0 * pp * (a * a));
+            const double al = qdiv(HBAR * HBAR, 4.0 * pp * (a * a));
             e.cA = sample_rel_sr(al, n, g);
             e.nA = pnorm;
             e.keep = 1;
@@ -876,8 +889,8 @@ __device__ __forceinline__ void sample_event(const DevProc& pr, int sp, const V3
             e.eB = E2;
             e.cA = r2;
             if (!(E2 < dropcut)) {
-                e.nB = div_const(sqrt(E2 * E2 + 2.0 * MC2 * E2), C, 1.0 / C);
-                e.cB = sqrt(E2 * (E0 + 2.0 * MC2) / (E0 * (E2 + 2.0 * MC2)));
+                e.nB = div_const_fin(qsqrt(E2 * E2 + 2.0 * MC2 * E2), C, 1.0 / C);
+                e.cB = qsqrt(qdiv(E2 * (E0 + 2.0 * MC2), E0 * (E2 + 2.0 * MC2)));
             }
             e.nturn = 2;
             e.sgnB = -1;
@@ -896,7 +909,7 @@ __device__ __forceinline__ void sample_event(const DevProc& pr, int sp, const V3
         V3 v = velocity(sp, p);
         double beta = div_const(norm3(v), C, 1.0 / C);  // exact: |v| / c
         double a = pr.c[0];
-        double al = HBAR * HBAR / (4.0 * dot3(p, p) * (a * a));
+        double al = qdiv(HBAR * HBAR, 4.0 * dot3(p, p) * (a * a));
         e.cA = sample_rel_sr(al, beta, g);
         e.nA = pnorm;
         e.keep = 1;
@@ -922,12 +935,12 @@ __device__ __forceinline__ void sample_event(const DevProc& pr, int sp, const V3
         e.phi = phi >= 0.0 ? phi : TWO_PI * g.next();
         // Lehtinen 1999 angles; those of a secondary the caller drops unseen (E2 < dropcut,
         // see finish_event) are not needed
-        e.nA = div_const(sqrt(E1 * E1 + 2.0 * MC2 * E1), C, 1.0 / C);
+        e.nA = div_const(qsqrt(E1 * E1 + 2.0 * MC2 * E1), C, 1.0 / C);
         e.eB = E2;
-        e.cA = sqrt(E1 * (E0 + 2.0 * MC2) / (E0 * (E1 + 2.0 * MC2)));
+        e.cA = qsqrt(qdiv(E1 * (E0 + 2.0 * MC2), E0 * (E1 + 2.0 * MC2)));
         if (!(E2 < dropcut)) {
-            e.nB = div_const(sqrt(E2 * E2 + 2.0 * MC2 * E2), C, 1.0 / C);
-            e.cB = sqrt(E2 * (E0 + 2.0 * MC2) / (E0 * (E2 + 2.0 * MC2)));
+            e.nB = div_const(qsqrt(E2 * E2 + 2.0 * MC2 * E2), C, 1.0 / C);
+            e.cB = qsqrt(qdiv(E2 * (E0 + 2.0 * MC2), E0 * (E2 + 2.0 * MC2)));
         }
         e.nturn = 2;
         e.sgnB = -1;
@@ -1100,21 +1113,23 @@ __device__ __forceinline__ void finish_event(const V3& p, double pnorm, const Ev
                                              V3& m1, double& s0, double& s1, const double* cut,
                                              const int* tracked, double dropcut, bool& drop1) {
     drop1 = e.ne == 2 && e.src1 == SRC_B && e.eB >= 0.0 && e.eB < dropcut;
-    double u0 = p.x / pnorm, u1 = p.y / pnorm, u2 = p.z / pnorm;
+    const Recip rp(pnorm);
+    const double u0 = rp(p.x), u1 = rp(p.y), u2 = rp(p.z);
     double sp, cp;
-    sincos(e.phi, &sp, &cp);
+    sincos_turn(e.phi, sp, cp, g.tab());
     double qs = 1.0 - u2 * u2;
-    double s = sqrt(qs > 0.0 ? qs : 0.0);
+    const double s = qsqrt(qs > 0.0 ? qs : 0.0);
+    const Recip rs(s);  // used where s > 0
     V3 pa, pb;
     {
         double q = 1.0 - e.cA * e.cA;
-        double st = sqrt(q > 0.0 ? q : 0.0);
+        const double st = qsqrt(q > 0.0 ? q : 0.0);
         double x, y, z;
         if (s > 0.0) {
             double bx = u0 * u2 * cp + (-u1) * sp;
             double by = u1 * u2 * cp + u0 * sp;
-            x = st * bx / s + u0 * e.cA;
-            y = st * by / s + u1 * e.cA;
+            x = rs(st * bx) + u0 * e.cA;
+            y = rs(st * by) + u1 * e.cA;
             z = -s * st * cp + u2 * e.cA;
         } else {
             x = st * cp;
@@ -1126,13 +1141,13 @@ __device__ __forceinline__ void finish_event(const V3& p, double pnorm, const Ev
     if (e.nturn == 2 && !drop1) {
         double spb = e.sgnB > 0 ? sp : -sp;
         double q = 1.0 - e.cB * e.cB;
-        double st = sqrt(q > 0.0 ? q : 0.0);
+        const double st = qsqrt(q > 0.0 ? q : 0.0);
         double x, y, z;
         if (s > 0.0) {
             double bx = u0 * u2 * cp + (-u1) * spb;
             double by = u1 * u2 * cp + u0 * spb;
-            x = st * bx / s + u0 * e.cB;
-            y = st * by / s + u1 * e.cB;
+            x = rs(st * bx) + u0 * e.cB;
+            y = rs(st * by) + u1 * e.cB;
             z = -s * st * cp + u2 * e.cB;
         } else {
             x = st * cp;
@@ -1156,8 +1171,8 @@ __device__ __forceinline__ void finish_event(const V3& p, double pnorm, const Ev
     const bool need1 = e.ne == 2 && !drop1 && stored(e.sp1, m1);
     double q0, q1;
     g.next12(e.ne == 2 ? 2 : 1, q0, q1);  // both draws at one place
-    s0 = need0 ? -log(q0) : 0.0;          // nextcoll(), src/util.jl:17
-    s1 = need1 ? -log(q1) : 0.0;
+    s0 = need0 ? -log_tab(q0, g.tab()) : 0.0;  // nextcoll(), src/util.jl:17
+    s1 = need1 ? -log_tab(q1, g.tab()) : 0.0;
 }
 
 }  // namespace pt
