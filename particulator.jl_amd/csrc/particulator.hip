@@ -83,6 +83,8 @@ struct Clock {
     uint32_t pass;           // 0: the launch's main pass; > 0: passes over its secondaries
     uint32_t nsub;           // steps of this launch
     ull tcur;                // items claimed in the current pass of the one-workgroup tail
+    ull left;                // secondaries that found their wave's stack full
+    uint32_t done, pad;      // workgroups that have ended the current pass
     double tf[MAX_SUB];      // their final times
 };
 
@@ -146,7 +148,8 @@ struct Params {
     uint32_t forcing_off;  // restrictions of the forcing and the pusher (off_em / off_cl / off_push)
     int lds_rate_off[PT_NSPECIES];
     int lds_rb_off[PT_NSPECIES];
-    int lds_doubles;
+    int lds_doubles;      // even
+    ull* image;           // what a workgroup stages: the Staged block, then lds_doubles doubles
 };
 
 // ------------------------------------------------------------------ LDS state
@@ -171,8 +174,9 @@ struct SpLite {
     gptr<uint8_t> evp;
     ull* n;
     ull cap;
-    const double* rate;  // LDS
-    const double* rb;    // LDS (one swarm) or global
+    const double* rb;  // rate bounds in global memory (several swarms)
+    int rate_off;      // the rate table in the dynamic LDS (doubles)
+    int rb_off;        // the rate bounds there (one swarm)
     double cut, xmax, ixmax, two_k1;  // ixmax = 1 / xmax, two_k1 = 2^(k+1)
     // |p|^2 above which the kinetic energy is certainly above the cut: the cut's |p|^2
     // times 1 + 1e-9, far beyond the rounding of the energy computed from |p|^2
@@ -190,40 +194,46 @@ struct BlockCounters {
     double dose[DOSE_LDS + 2];
 };
 
-struct Shared {
+// What every workgroup needs of the parameters, in the form it needs it: built once in global
+// memory when parameters change (k_build_image) with the doubles of the dynamic LDS behind it,
+// so that staging is one coalesced copy with all its loads in flight.  (Built by each workgroup
+// from the parameters, with its dependent loads and the serial work of one thread, it took
+// about 20 us of a launch.)
+struct __attribute__((aligned(16))) Staged {
     SpLite sp[PT_NSPECIES];
     DevProc procs[PT_NSPECIES][MAX_PROCS];
-    BlockCounters bc;
     double cut[PT_NSPECIES];  // new particles at or below the cut are not stored
     int stored[PT_NSPECIES];  // species whose new particles are stored (tracked, with a table)
     // the field of swarm 0 (the push of a one-swarm population reads it here: from global
     // memory each read would be a vector load whose wait also waits for every memory
     // operation issued before it)
     Field field0;
-    const double* fields_lds;  // homogeneous fields: the swarms' E, B vectors in the dynamic LDS
+};
+
+struct Shared : Staged {
+    BlockCounters bc;
     double tf[MAX_SUB];  // the final times of the launch's steps (nsub of them)
     int nsub, pad;
 };
 
-__device__ __forceinline__ void stage(const Params& P, double* lds, Shared& sh) {
+constexpr size_t IMAGE_BYTES = 160 * 1024;  // a workgroup's LDS is no larger
+
+__global__ void __launch_bounds__(256) k_build_image(const Params* __restrict__ Pp) {
+    const Params& P = *Pp;
+    Staged& st = *(Staged*)P.image;
+    double* const lds = (double*)(&st + 1);
     for (int q = threadIdx.x; q < MATH_DOUBLES; q += blockDim.x) lds[q] = g_math[q];
-    for (int q = threadIdx.x; q < (int)(sizeof(BlockCounters) / sizeof(ull)); q += blockDim.x)
-        ((ull*)&sh.bc)[q] = 0;
-    static_assert(sizeof(Field) % sizeof(ull) == 0, "Field is copied in 8-byte words");
-    for (int q = threadIdx.x; q < (int)(sizeof(Field) / sizeof(ull)); q += blockDim.x)
-        ((ull*)&sh.field0)[q] = ((const ull*)P.fields)[q];
     if (P.field_lds)
         for (int q = threadIdx.x; q < 6 * P.nswarm; q += blockDim.x) {
             const FieldFn& f = (q % 6) < 3 ? P.fields[q / 6].e : P.fields[q / 6].b;
             lds[P.lds_field_off + q] = f.v[q % 3];
         }
-    if (threadIdx.x < MAX_SUB) sh.tf[threadIdx.x] = P.clock->tf[threadIdx.x];
-    if (threadIdx.x == 0) sh.nsub = (int)P.clock->nsub;
+    if (threadIdx.x == 0) st.field0 = P.fields[0];
     for (int s = 0; s < PT_NSPECIES; s++) {
         const DevTable& tb = P.tab[s];
         const SpeciesDev& S = P.sp[s];
         if (threadIdx.x == 0) {
-            SpLite& L = sh.sp[s];
+            SpLite& L = st.sp[s];
             for (int f = 0; f < PT_NFIELDS; f++) L.f[f] = (gptr<double>)S.f[f];
             L.active = (gptr<uint8_t>)S.active;
             L.uid = (gptr<uint64_t>)S.uid;
@@ -247,15 +257,15 @@ __device__ __forceinline__ void stage(const Params& P, double* lds, Shared& sh) 
             L.xmax = tb.xmax;
             L.ixmax = 1.0 / tb.xmax;
             L.two_k1 = ldexp(1.0, tb.k + 1);
-            L.rate = lds + P.lds_rate_off[s];
-            L.rb = P.rb_in_lds ? lds + P.lds_rb_off[s] : tb.ratebound;
+            L.rate_off = P.lds_rate_off[s];
+            L.rb_off = P.lds_rb_off[s];
+            L.rb = tb.ratebound;
             L.rb_lds = P.rb_in_lds;
-            sh.cut[s] = tb.cut;
-            sh.stored[s] = S.tracked && tb.valid;
-            if (s == 0) sh.fields_lds = lds + P.lds_field_off;
+            st.cut[s] = tb.cut;
+            st.stored[s] = S.tracked && tb.valid;
         }
         if (!tb.valid) continue;
-        for (int q = threadIdx.x; q < tb.nprocs; q += blockDim.x) sh.procs[s][q] = tb.procs[q];
+        for (int q = threadIdx.x; q < tb.nprocs; q += blockDim.x) st.procs[s][q] = tb.procs[q];
         int nr = (tb.k + 1) * tb.nprocs * 3;
         double* dst = lds + P.lds_rate_off[s];
         for (int q = threadIdx.x; q < nr + SCAN_PAD; q += blockDim.x) dst[q] = q < nr ? tb.rate[q] : 0.0;
@@ -265,6 +275,34 @@ __device__ __forceinline__ void stage(const Params& P, double* lds, Shared& sh) 
             for (int q = threadIdx.x; q < nb; q += blockDim.x) d2[q] = tb.ratebound[q];
         }
     }
+}
+
+__device__ __forceinline__ void stage(const Params& P, Shared& sh) {
+    typedef uint32_t word4 __attribute__((ext_vector_type(4)));
+    const PT_GLOBAL word4* src = (const PT_GLOBAL word4*)P.image;
+    const int n0 = sizeof(Staged) / 16, n = n0 + P.lds_doubles / 2;
+    PT_LDS word4* const d0 = (PT_LDS word4*)(Staged*)&sh;
+    PT_LDS word4* const d1 = (PT_LDS word4*)pt_lds;
+    constexpr int U = 8;  // loads in flight per thread
+    for (int q0 = threadIdx.x; q0 < n; q0 += U * blockDim.x) {
+        word4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int q = q0 + u * (int)blockDim.x;
+            v[u] = src[q < n ? q : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int q = q0 + u * (int)blockDim.x;
+            if (q < n0) d0[q] = v[u];
+            else if (q < n) d1[q - n0] = v[u];
+        }
+    }
+    if (threadIdx.x < MAX_SUB) sh.tf[threadIdx.x] = P.clock->tf[threadIdx.x];
+    if (threadIdx.x == 0) sh.nsub = (int)P.clock->nsub;
+    ull* const z = (ull*)&sh.bc;  // the dose bins (the last member) only where there is a tally
+    const int nz = (int)((P.dose_bins > 0 ? sizeof(BlockCounters) : offsetof(BlockCounters, dose)) / sizeof(ull));
+    for (int q = threadIdx.x; q < nz; q += blockDim.x) z[q] = 0;
     __syncthreads();
 }
 
@@ -276,7 +314,7 @@ __device__ __forceinline__ double setr(const SpLite& L, double E, int swarm, boo
     int i = precheb(E, L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o);
     oob |= o;
     const size_t off = (size_t)(L.nswarm > 1 ? swarm : 0) * (L.k + 1) * 3 + i * 3;
-    return L.rb_lds ? cheb3(as_lds(L.rb) + off, t1, t2) : cheb3(as_global(L.rb) + off, t1, t2);
+    return L.rb_lds ? cheb3(as_lds(pt_lds) + L.rb_off + off, t1, t2) : cheb3(as_global(L.rb) + off, t1, t2);
 }
 
 // The selection scan of do_one_collision! (src/collisions.jl:160-186): the first process j
@@ -457,10 +495,21 @@ __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, cons
 // stream position and queued for that sampler kind (wave-aggregated appends), and the
 // lane moves on.  The sampling kernel then runs each queued kind with whole waves of the
 // same kind (no divergence between samplers; the learned samplers need it).
-// items a wave claims at a time: 128 in workgroups of up to 256 threads, 256 in larger ones
+// Items a wave claims at a time: 128 in workgroups of up to 256 threads, 256 in larger ones
 // (the faster size for each launch shape the autotuner picks: the avalanche's 256-thread
-// and the sweep's 512-thread workgroups)
-__device__ __forceinline__ ull claim_chunk() { return blockDim.x > 256 ? 256ull : 128ull; }
+// and the sweep's 512-thread workgroups), and a quarter of the wave's share of what is left
+// when that is less, so that the waves end together.
+constexpr ull LEAST_CHUNK = 16;
+__device__ __forceinline__ ull claim_chunk(ull left, ull nwaves, ull least) {
+    const ull most = blockDim.x > 256 ? 256ull : 128ull, share = left / (4 * nwaves);
+    return share > most ? most : share < least ? least : share;
+}
+// Lanes of a wave that take items.  An iteration of a wave whose lanes are in different
+// branches takes up to three times as long as that of a single lane (14 against 5 us), so a
+// population with fewer particles than the launch has lanes is spread over all its waves.
+__device__ __forceinline__ int lanes_used(ull total, ull nwaves) {
+    return total >= 64 * nwaves ? 64 : (int)((total + nwaves - 1) / nwaves);
+}
 enum { SRC_RANGE = 0, SRC_QUEUE = 1 };
 // a further push round before the collisions, when at least MORE_LANES lanes can use it
 constexpr int MORE_ROUNDS = 1, MORE_LANES = 20;
@@ -694,9 +743,27 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
     const int lane = threadIdx.x & 63;
     const uint64_t ltmask = lane ? (~0ull >> (64 - lane)) : 0ull;
     // wave-uniform chunk state
-    const ull chunk = claim_chunk();
+    const ull nwaves = (ull)gridDim.x * (blockDim.x >> 6);
+    const int lanes = lanes_used(total, nwaves);
+    const ull least = lanes < LEAST_CHUNK ? lanes : LEAST_CHUNK;
+    ull chunk = claim_chunk(total, nwaves, least);
     ull cbeg = 0, cend = 0;
     bool drained = false;
+    // the wave's next chunk of items; false when they are all claimed
+    auto claim = [&]() {
+        int fl = __ffsll((unsigned long long)__ballot(1)) - 1;
+        ull b = 0;
+        if (lane == fl) b = global_add(cursor, chunk);
+        b = __shfl(b, fl);
+        if (b >= total) {
+            drained = true;
+            return false;
+        }
+        cbeg = b;
+        cend = b + chunk < total ? b + chunk : total;
+        chunk = claim_chunk(total - cend, nwaves, least);
+        return true;
+    };
     // the wave's secondaries waiting to be advanced (LDS, last in first out)
     uint64_t* const stk = (uint64_t*)(wlds + COOP_JOB_BYTES);
     int nstk = 0;  // wave-uniform
@@ -848,22 +915,11 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                     mine = true;
                 }
                 nstk -= pop;
-                const int want = nfree - pop;
-                if (want > 0 && !drained) {
-                    if (cbeg >= cend) {
-                        int fl = __ffsll((unsigned long long)__ballot(1)) - 1;
-                        ull b = 0;
-                        if (lane == fl) b = global_add(cursor, chunk);
-                        b = __shfl(b, fl);
-                        if (b >= total) {
-                            drained = true;
-                        } else {
-                            cbeg = b;
-                            cend = b + chunk < total ? b + chunk : total;
-                        }
-                    }
-                    const ull q = cbeg + (ull)(rank - pop);
-                    if (!have && rank >= pop && q < cend) {
+                const uint64_t open = __ballot(!have && rank >= pop && lane < lanes);
+                if (open && !drained && (cbeg < cend || claim())) {
+                    const ull want = (ull)__popcll(open);
+                    const ull q = cbeg + (ull)__popcll(open & ltmask);
+                    if (((open >> lane) & 1) && q < cend) {
                         if (q < n0) {
                             qs = 0;
                             qi = rb[0] + q;
@@ -876,7 +932,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                         }
                         mine = true;
                     }
-                    cbeg = cbeg + (ull)want < cend ? cbeg + (ull)want : cend;
+                    cbeg = cbeg + want < cend ? cbeg + want : cend;
                 }
                 if (__ballot(mine) == 0) break;
                 if (mine) {
@@ -951,23 +1007,12 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         if constexpr (AHEAD) {
             // (waiting secondaries are taken first; a pass over secondaries of several steps
             // reads their birth steps in B)
-            const bool ends = first && nstk == 0 && (main_pass || K == 1) && have && !pend && ks == K - 1 && trem > EPS64 && active &&
+            const bool ends = first && nstk == 0 && lane < lanes && (main_pass || K == 1) && have && !pend && ks == K - 1 && trem > EPS64 && active &&
                               !(trem > tnext);
             bool got = false;
             uint64_t want = __ballot(ends);
             while (want && !drained) {
-                if (cbeg >= cend) {
-                    int fl = __ffsll((unsigned long long)__ballot(1)) - 1;
-                    ull b = 0;
-                    if (lane == fl) b = global_add(cursor, chunk);
-                    b = __shfl(b, fl);
-                    if (b >= total) {
-                        drained = true;
-                        break;
-                    }
-                    cbeg = b;
-                    cend = b + chunk < total ? b + chunk : total;
-                }
+                if (cbeg >= cend && !claim()) break;
                 const ull q = cbeg + (ull)__popcll(want & ltmask);
                 const ull cnt = (ull)__popcll(want);
                 const bool mine = ends && !got && q < cend;
@@ -1018,7 +1063,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                 V3 dx{0, 0, 0}, dp{0, 0, 0};
                 bool uniform;  // the force does not depend on the position
                 if (P.field_lds) {
-                    const PT_LDS double* fv = as_lds(sh.fields_lds) + 6 * swarm;
+                    const PT_LDS double* fv = as_lds(pt_lds) + P.lds_field_off + 6 * swarm;
                     const HomField hf{{fv}, {fv + 3}, {{nullptr, nullptr}}};
                     push_delta(sp, hf, x, p, dt, foff, dx, dp);
                     uniform = true;
@@ -1091,7 +1136,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
             int iv = precheb(cE, L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o);
             oob |= o;
             double xi = g.next() * r;
-            const int sel = select_process(as_lds(L.rate) + (size_t)iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
+            const int sel = select_process(as_lds(pt_lds) + L.rate_off + iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
             if (sel < 0) {
                 if (!(xi >= 0.0)) atomicAdd(&sh.bc.flags[FLAG_RATEBOUND], 1ull);
                 atomicAdd(&sh.bc.counts[sp * NCOUNT], 1ull);
@@ -1180,7 +1225,9 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                 const int at = nstk + __popcll(m & ltmask);
                 if (sl != NO_SLOT && at < STACK)
                     stk[at] = sl | (uint64_t)(q ? cs1 : cs0) << 32 | (uint64_t)(uint32_t)ks << 40;
-                nstk = nstk + __popcll(m) < STACK ? nstk + __popcll(m) : STACK;
+                const int all = nstk + __popcll(m);
+                nstk = all < STACK ? all : STACK;
+                if (all > STACK && lane == 0) global_add(&P.clock->left, (ull)(all - STACK));
             }
             wave_lds_order();
         }
@@ -1246,26 +1293,36 @@ __global__ void k_snapshot(const Params* __restrict__ Pp, int clocked, double tf
         C.ecur = 0;
         C.qpar = 0;
         C.pass = 0;
+        C.left = 0;
+        C.done = 0;
     }
 }
 
-// the next advance1! pass (src/mixed_population.jl:43-46): the particles appended since the
-// last mark, processed by the whole grid
-__global__ void k_next_pass(const Params* __restrict__ Pp) {
-    const Params& P = *Pp;
+// The end of a pass, called by every workgroup of its launch: the last one to end sets up the
+// next advance1! pass (src/mixed_population.jl:43-46) over the particles appended since the
+// last mark, for the whole grid.  When every secondary found room on its wave's stack there is
+// nothing left to do, and the next pass is empty.  What the last workgroup reads was written
+// by atomics, which have all been performed once every wave has waited for its own: no cache
+// is written back (a __threadfence() in each of the 512 workgroups takes 13 us).
+__device__ __forceinline__ void end_pass(const Params& P) {
+    wait_vmem();
+    __syncthreads();
+    if (threadIdx.x != 0) return;
     Clock& C = *P.clock;
-    int s = threadIdx.x;
-    if (s < PT_NSPECIES) {
+    const uint32_t k = __hip_atomic_fetch_add(&C.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (k != gridDim.x - 1) return;
+    const ull left = __hip_atomic_load(&C.left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int s = 0; s < PT_NSPECIES; s++) {
         ull n = __hip_atomic_load(P.sp[s].n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (n > P.sp[s].cap) n = P.sp[s].cap;
-        P.range[2 * s] = C.nmark[s];
+        P.range[2 * s] = left ? C.nmark[s] : n;
         P.range[2 * s + 1] = n;
-        C.nmark[s] = n;
+        if (left) C.nmark[s] = n;
     }
-    if (s == 0) {
-        C.cursor = 0;
-        C.pass += 1;
-    }
+    C.cursor = 0;
+    C.pass += 1;
+    C.left = 0;
+    C.done = 0;
 }
 
 __global__ void k_tick(const Params* __restrict__ Pp) {
@@ -1303,7 +1360,6 @@ __global__ void k_rotate(const Params* __restrict__ Pp) {
 // push/select over the step's particles (first round) or the input work queues
 template <int BS, int SRC, bool EVENT, bool WALL = false, bool MLP = false>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_advance(const Params* __restrict__ Pp) {
-    double* const lds = pt_lds;
     __shared__ Shared sh;
     __shared__ int skip;
     const Params& P = *Pp;
@@ -1325,12 +1381,18 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
     if (threadIdx.x == 0)
         skip = __hip_atomic_load(&P.clock->cursor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= total;
     __syncthreads();
-    if (skip) return;
-    stage(P, lds, sh);
-    char* wlds = (char*)lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES;
+    if (skip) {
+        if constexpr (!EVENT) {
+            if (total > 0) end_pass(P);  // (a pass over nothing leaves the next one empty, too)
+        }
+        return;
+    }
+    stage(P, sh);
+    char* wlds = (char*)pt_lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES;
     select_loop<SRC, EVENT, WALL, MLP>(P, sh, wlds, rb, re, &P.clock->cursor, C.step,
                                        SRC == SRC_RANGE && C.pass == 0, par);
     flush_counters(P, &sh.bc);
+    if constexpr (!EVENT) end_pass(P);
 }
 
 // Sampling round: each wave takes 64 queued collisions of one sampler kind (the queues are
@@ -1339,7 +1401,6 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
 // particles for the next push/select round.
 template <int BS>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_sample(const Params* __restrict__ Pp) {
-    double* const lds = pt_lds;
     __shared__ Shared sh;
     __shared__ ull seg[PT_NSPECIES * NKQ + 1];
     __shared__ int skip;
@@ -1359,7 +1420,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
     }
     __syncthreads();
     if (skip) return;
-    stage(P, lds, sh);
+    stage(P, sh);
     const int lane = threadIdx.x & 63;
     const uint64_t ltmask = lane ? (~0ull >> (64 - lane)) : 0ull;
     const ull total = seg[PT_NSPECIES * NKQ];
@@ -1467,23 +1528,23 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
     flush_counters(P, &sh.bc);
 }
 
-// Secondaries born in this step and not yet advanced: one workgroup repeats passes over
-// [begin, n) until a pass appends nothing (the `while n > 0` loop of advance!,
-// src/mixed_population.jl:43-46).
+// Secondaries not yet advanced after those passes: one workgroup repeats passes over the range
+// the last one left and then over what it appends itself, until a pass appends nothing (the
+// `while n > 0` loop of advance!, src/mixed_population.jl:43-46).
 template <bool WALL, bool MLP>
 __global__ void __launch_bounds__(512) k_tail(const Params* __restrict__ Pp, int maxpasses) {
-    double* const lds = pt_lds;
     __shared__ Shared sh;
     __shared__ ull beg[PT_NSPECIES], end[PT_NSPECIES];
     __shared__ int done;
     const Params& P = *Pp;
+    bool none = true;
+    for (int s = 0; s < PT_NSPECIES; s++) none = none && P.range[2 * s + 1] <= P.range[2 * s];
+    if (none) return;
     // the passes' claim counter: in global memory, since the loop claims its chunks with
     // global atomics (an LDS address used as a global one is an invalid access)
     ull* const cur = &P.clock->tcur;
-    stage(P, lds, sh);
+    stage(P, sh);
     const uint32_t step = P.clock->step;
-    if (threadIdx.x == 0)
-        for (int s = 0; s < PT_NSPECIES; s++) beg[s] = P.clock->nmark[s];
     if (threadIdx.x == 0) done = 0;
     for (int pass = 0; pass < maxpasses; pass++) {
         __threadfence();
@@ -1495,8 +1556,9 @@ __global__ void __launch_bounds__(512) k_tail(const Params* __restrict__ Pp, int
             for (int s = 0; s < PT_NSPECIES; s++) {
                 ull n = __hip_atomic_load(P.sp[s].n, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
                 if (n > P.sp[s].cap) n = P.sp[s].cap;
-                end[s] = n;
-                if (n > beg[s]) done = 0;
+                beg[s] = pass == 0 ? P.range[2 * s] : end[s];
+                end[s] = pass == 0 ? P.range[2 * s + 1] : n;
+                if (end[s] > beg[s]) done = 0;
             }
         }
         __syncthreads();
@@ -1506,12 +1568,8 @@ __global__ void __launch_bounds__(512) k_tail(const Params* __restrict__ Pp, int
             rb[s] = beg[s];
             re[s] = end[s];
         }
-        select_loop<SRC_RANGE, false, WALL, MLP>(P, sh, (char*)lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES,
+        select_loop<SRC_RANGE, false, WALL, MLP>(P, sh, (char*)pt_lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES,
                                                  rb, re, cur, step, false, 0);
-        __threadfence();
-        __syncthreads();
-        if (threadIdx.x == 0)
-            for (int s = 0; s < PT_NSPECIES; s++) beg[s] = end[s];
     }
     // the pass limit was reached with work left: report it
     if (threadIdx.x == 0 && !done) sh.bc.flags[FLAG_TAIL] += 1;
@@ -1809,10 +1867,9 @@ __global__ void k_mlp_features(const Params* __restrict__ Pp, int which, const d
 
 // init! / advance_init!: r of every active particle (src/mixed_population.jl:20-35)
 __global__ void __launch_bounds__(256) k_setr(const Params* __restrict__ Pp, int sp) {
-    double* const lds = pt_lds;
     __shared__ Shared sh;
     const Params& P = *Pp;
-    stage(P, lds, sh);
+    stage(P, sh);
     const SpLite& L = sh.sp[sp];
     ull n = *L.n;
     if (n > L.cap) n = L.cap;
@@ -2251,10 +2308,9 @@ __global__ void __launch_bounds__(256) k_dbg_select(const Params* __restrict__ P
                                                     const double* E, const double* u,
                                                     const int32_t* swarm, int32_t* interval,
                                                     int32_t* proc, double* rbound) {
-    double* const lds = pt_lds;
     __shared__ Shared sh;
     const Params& P = *Pp;
-    stage(P, lds, sh);
+    stage(P, sh);
     ull i = (ull)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const SpLite& L = sh.sp[sp];
@@ -2266,7 +2322,7 @@ __global__ void __launch_bounds__(256) k_dbg_select(const Params* __restrict__ P
     bool o;
     int iv = precheb(E[i], L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o);
     double xi = u[i] * r;
-    int sel = select_process(as_lds(L.rate) + (size_t)iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
+    int sel = select_process(as_lds(pt_lds) + L.rate_off + iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
     interval[i] = o ? -1 : iv;
     proc[i] = sel;
     rbound[i] = r;
@@ -2523,10 +2579,15 @@ static int sync_params(pt_ctx* c) {
     c->hp.forcing_off = (c->hp.forcing_off & ~OFF_NO_B) | (nob ? OFF_NO_B : 0u);
     c->hp.lds_field_off = off;
     if (hom) off += 6 * c->cfg.nswarm;
+    off = (off + 1) & ~1;
     c->hp.lds_doubles = off;
+    if (sizeof(Staged) + sizeof(double) * (size_t)off > IMAGE_BYTES)
+        return fail(c, PT_E_ARG, "the tables (%zu bytes) do not fit a workgroup's LDS", sizeof(double) * (size_t)off);
     c->lds_bytes = off * (int)sizeof(double);
     c->hp.lds_coop_off = (c->lds_bytes + 15) & ~15;
     HIPCHK(c, hipMemcpyAsync(c->dp, &c->hp, sizeof(Params), hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(k_build_image, dim3(1), dim3(256), 0, c->stream, c->dp);
+    HIPCHK(c, hipGetLastError());
     c->dirty = false;
     // a captured step bakes in host-side choices made from these parameters (the kernel
     // variant for a wall, the LDS sizes, the queues): graphs captured before are stale
@@ -2726,6 +2787,7 @@ int pt_create(const pt_config* cfg, pt_ctx** out) {
     TRY(dalloc(c, (void**)&c->cinfo, sizeof(ull) * 4));
     TRY(dalloc(c, (void**)&c->stat_part, sizeof(double) * NSTAT * 4096));
     TRY(dalloc(c, (void**)&c->dp, sizeof(Params)));
+    TRY(dalloc(c, (void**)&P.image, IMAGE_BYTES));
     hipDeviceProp_t prop;
     HIPCHK(c, hipGetDeviceProperties(&prop, c->device));
     c->ncu = prop.multiProcessorCount;
@@ -3213,7 +3275,7 @@ static int launch_kernel_args(pt_ctx* c, int v, bool full) {
     ull blocks = (ull)c->resident[v][block_index(bs)] * c->ncu * std::max(1, c->launch.grid_mult);
     if (!full) {
         ull est = c->hn[0] + c->hn[1] + c->hn[2];
-        blocks = std::min<ull>(blocks, std::max<ull>((ull)c->ncu, (2 * est + bs - 1) / bs));
+        blocks = std::min<ull>(blocks, std::max<ull>((ull)c->ncu, est / (ull)(bs / 64)));
     }
     HIPCHK(c, hipLaunchKernel(kernel_of(v, bs), dim3((unsigned)std::max<ull>(blocks, 1)), dim3(bs), args,
                               kernel_lds(c, v, bs), c->stream));
@@ -3255,8 +3317,6 @@ static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int ns
     // secondaries the lanes' stacks could not take: whole-grid passes, then one workgroup
     // for whatever the last pass created
     for (int q = 0; q < c->launch.tail_passes; q++) {
-        hipLaunchKernelGGL(k_next_pass, dim3(1), dim3(64), 0, c->stream, c->dp);
-        HIPCHK(c, hipGetLastError());
         if ((rc = launch_kernel_args(c, in_place, true))) return rc;
     }
     if (prof && (rc = mark(c, &e1))) return rc;
