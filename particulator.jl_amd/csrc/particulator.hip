@@ -320,15 +320,21 @@ __device__ __forceinline__ double setr(const SpLite& L, double E, int swarm, boo
 // The selection scan of do_one_collision! (src/collisions.jl:160-186): the first process j
 // whose rate exceeds what is left of xi after subtracting the rates of processes 0..j-1; -1
 // for a null collision, xi then holding the remainder.  Rates are evaluated four at a time,
-// branch-free within a group, so that their LDS reads overlap; a group may run past the
-// row's last process into the next row or the table's padding (SCAN_PAD), whose values are
-// never used.
+// branch-free within a group, and the next group's coefficients are read before a group is
+// tested, so that their LDS reads overlap; a group may run past the row's last process into
+// the next row or the table's padding (SCAN_PAD), whose values are never used.
 __device__ __forceinline__ int select_process(const PT_LDS double* rt, int np, double t1, double t2, double& xi) {
     int sel = -1;
+    double c[12];
+#pragma unroll
+    for (int u = 0; u < 12; u++) c[u] = rt[u];
     for (int j = 0; j < np; j += 4) {
         double nu[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) nu[u] = cheb3(rt + 3 * (j + u), t1, t2);
+        for (int u = 0; u < 4; u++) nu[u] = (c[3 * u] * 1.0 + c[3 * u + 1] * t1) + c[3 * u + 2] * t2;
+        const PT_LDS double* nx = rt + 3 * (j + 4 < np ? j + 4 : 0);
+#pragma unroll
+        for (int u = 0; u < 12; u++) c[u] = nx[u];
         bool found = false;
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -574,17 +580,24 @@ __device__ __forceinline__ void wave_push(ull* cnt, uint32_t* arr, uint32_t val,
 
 // A lane's RBEB collision waiting for the wave's cooperative rejection loop (LDS, one slot
 // per lane of the wave, then a 64-entry rank table)
-struct RbebJob {
+struct __attribute__((aligned(16))) RbebJob {
     RbebSetup s;
     double first;  // uniform number d0 of the stream when d0 is odd (a cached block's half)
     uint64_t uid;
-    uint32_t d0, k;  // stream position before the loop, trips evaluated so far
-    uint32_t step, pad;
+    uint32_t d0, step;  // stream position before the loop, step of the stream
 };
 // a wave's LDS area: the RBEB jobs and their rank table, then its stack of secondaries
 constexpr int STACK = 64;
 constexpr int COOP_JOB_BYTES = 64 * (int)sizeof(RbebJob) + 64;
 constexpr int COOP_WAVE_BYTES = COOP_JOB_BYTES + 8 * STACK;
+
+// v of the lane before (lane 0: anything): a wave-wide shift by one on the vector unit, without
+// the round trip through LDS of a shuffle
+__device__ __forceinline__ double lane_before(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x138, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x138, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
 
 // The rejection loops of the wave's pending RBEB collisions (_rbeb_sample,
 // src/rbeb.jl:170-196), run by every lane of the wave together.  Trip k of a particle uses
@@ -592,76 +605,80 @@ constexpr int COOP_WAVE_BYTES = COOP_JOB_BYTES + 8 * STACK;
 // lanes are shared out over the particles still waiting (64 / n trips each, in order), and
 // a particle takes its first accepting trip.  Result and stream position are those of the
 // sequential loop; the wave runs about log(n) rounds instead of the longest particle's
-// trip count.  Called by the whole wave; `pending` lanes have written their job.
-__device__ __forceinline__ void rbeb_coop(const Params& P, char* wlds, int lane, uint64_t ltmask, bool& pending,
-                                          double& wout, StepStream& g) {
-    RbebJob* jobs = (RbebJob*)wlds;
-    uint8_t* rank_lane = (uint8_t*)(wlds + 64 * sizeof(RbebJob));
+// trip count.  Called by the whole wave; `pending` lanes have written their job.  Every
+// particle still waiting has evaluated the same number of trips, so a round's stream
+// positions need no memory, and its only shuffles are the accepted w and the second half of
+// the last block looked at (LDS round trips take about 130 cycles each).
+__device__ __forceinline__ void rbeb_coop(const Params& P, PT_LDS char* wlds, int lane, uint64_t ltmask,
+                                          bool& pending, double& wout, StepStream& g) {
+    PT_LDS RbebJob* jobs = (PT_LDS RbebJob*)wlds;
+    PT_LDS uint8_t* rank_lane = (PT_LDS uint8_t*)(wlds + 64 * sizeof(RbebJob));
     const uint32_t k0 = (uint32_t)P.seed, k1 = (uint32_t)(P.seed >> 32);
     uint64_t U = __ballot(pending);
+    uint32_t done = 0;  // trips of each waiting particle so far
     while (U) {
         const int nU = __popcll(U);
-        const int m = 64 / nU;
+        // m = 64 / nU and gi = lane / m: the quotients are at least 1/128 away from the next
+        // integers, far more than the error of the reciprocals
+        const int m = (int)(64.5f * __builtin_amdgcn_rcpf((float)nU));
         const int myrank = __popcll(U & ltmask);
         if (pending) rank_lane[myrank] = (uint8_t)lane;
         wave_lds_order();
-        const int gi = lane / m, j = lane - gi * m;
+        const int gi = (int)(((float)lane + 0.5f) * __builtin_amdgcn_rcpf((float)m)), j = lane - gi * m;
         const bool act = gi < nU;
         double c0b = 0.0, c1b = 0.0, wv = 0.0;
-        uint32_t blk = 0, D = 0;
-        int ow = 0;
+        uint32_t D = 0;
+        RbebSetup js;
+        double jfirst = 0.0;
         if (act) {
-            ow = rank_lane[gi];
-            const RbebJob& J = jobs[ow];
-            D = J.d0 + 2u * (J.k + (uint32_t)j);
-            blk = (D + 1) >> 1;  // the block of the trip's second draw
-            uint32_t a = (uint32_t)J.uid, b = (uint32_t)(J.uid >> 32), c = J.step, e = blk;
+            const PT_LDS RbebJob& J = jobs[rank_lane[gi]];
+            js.t = J.s.t;
+            js.A = J.s.A;
+            js.Cc = J.s.Cc;
+            js.M = J.s.M;
+            js.pbn = J.s.pbn;
+            js.ratio = J.s.ratio;
+            js.iratio = J.s.iratio;
+            jfirst = J.first;
+            D = J.d0 + 2u * (done + (uint32_t)j);
+            // the block of the trip's second draw
+            uint32_t a = (uint32_t)J.uid, b = (uint32_t)(J.uid >> 32), c = J.step, e = (D + 1) >> 1;
             philox10(a, b, c, e, k0, k1);
             c0b = u01(a, b);
             c1b = u01(c, e);
         }
-        const double prev = __shfl_up(c1b, 1);  // the previous trip's block (same particle when j > 0)
+        const double prev = lane_before(c1b);  // the previous trip's block (same particle when j > 0)
         bool acc = false;
         if (act) {
-            const RbebJob& J = jobs[ow];
-            double u, z;
-            if (D & 1) {
-                u = j == 0 ? J.first : prev;
-                z = c0b;
-            } else {
-                u = c0b;
-                z = c1b;
-            }
-            acc = rbeb_trip(J.s, u, z, wv) || D + 2u >= DRAW_LIMIT;
+            const bool odd = (D & 1) != 0;
+            const double u = odd ? (j == 0 ? jfirst : prev) : c0b;
+            acc = rbeb_trip(js, u, odd ? c0b : c1b, wv) || D + 2u >= DRAW_LIMIT;
         }
         const uint64_t Acc = __ballot(act && acc);
-        int src = lane, last = lane;
+        // the first accepting trip, or the last one
+        int hit = m - 1;
         bool got = false;
         if (pending) {
             const uint64_t gm = m >= 64 ? ~0ull : ((1ull << m) - 1ull);
             const uint64_t bits = (Acc >> (myrank * m)) & gm;
             got = bits != 0;
-            if (got) src = myrank * m + __ffsll((unsigned long long)bits) - 1;
-            last = myrank * m + m - 1;
+            if (got) hit = __ffsll((unsigned long long)bits) - 1;
         }
-        const double w_s = __shfl(wv, src), c0_s = __shfl(c0b, src), c1_s = __shfl(c1b, src);
-        const uint32_t blk_s = __shfl(blk, src), D_s = __shfl(D, src);
-        const double c1_last = __shfl(c1b, last);
-        wave_lds_order();
+        const int src = pending ? myrank * m + hit : lane;
+        const double w_s = __shfl(wv, src), c1_s = __shfl(c1b, src);
         if (pending) {
-            RbebJob& J = jobs[lane];
             if (got) {
                 wout = w_s;
-                g.draw = D_s + 2u;
-                g.c0 = c0_s;
+                // (at an odd position the second half of the last block is the next draw)
+                g.draw += 2u * (done + (uint32_t)hit) + 2u;
                 g.c1 = c1_s;
-                g.cblk = blk_s + 1;
+                g.cblk = (g.draw >> 1) + (g.draw & 1);
                 pending = false;
             } else {
-                J.k += (uint32_t)m;
-                J.first = c1_last;
+                jobs[lane].first = c1_s;
             }
         }
+        done += (uint32_t)m;
         wave_lds_order();
         U = __ballot(pending);
     }
@@ -728,7 +745,7 @@ __device__ __forceinline__ void learned_pass(const Params& P, const Shared& sh, 
 __device__ __forceinline__ int swarm_of(const Params& P, int32_t sw) { return (sw < 0 || sw >= P.nswarm) ? 0 : sw; }
 
 template <int SRC, bool EVENT, bool WALL = false, bool MLP = false>
-__device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* wlds, const ull* rb, const ull* re,
+__device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS char* wlds, const ull* rb, const ull* re,
                                             ull* cursor, uint32_t step0, bool main_pass, int par) {
     // range passes load a retiring lane's next item ahead (D); a lane that retires ends its
     // last step without a collision, so it neither queues one (EVENT) nor runs a network (MLP)
@@ -765,7 +782,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         return true;
     };
     // the wave's secondaries waiting to be advanced (LDS, last in first out)
-    uint64_t* const stk = (uint64_t*)(wlds + COOP_JOB_BYTES);
+    PT_LDS uint64_t* const stk = (PT_LDS uint64_t*)(wlds + COOP_JOB_BYTES);
     int nstk = 0;  // wave-uniform
     int extra = 0;  // push rounds since the wave's last collision phase (wave-uniform)
     // lane state
@@ -786,6 +803,64 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
     bool new_r = false;  // its rate bound is to be recomputed
     double cE = 0.0;     // kinetic energy at the pending collision
     int ks = 0;          // the step it is in (0..K-1)
+    // what the lane's particle needs of its species and swarm, in registers while it has the
+    // lane (each read from LDS is a round trip in the chain of dependent operations that an
+    // iteration is): table grid, cut, offsets of its tables, and with a uniform electric field
+    // and no magnetic one its force
+    double cut = 0, pphi = 0, xmax = 1, ixmax = 1, two_k1 = 1;
+    int kint = 0, nprocs = 0, rate_off = 0, rb_off = 0;
+    V3 F{0, 0, 0};
+    const bool ffree = P.field_lds && (foff & OFF_NO_B);
+    const bool falong = (foff & OFF_E_Z) != 0;
+    // the rate bound's coefficients in the interval ci of its energy
+    int ci = -1;
+    double rc0 = 0, rc1 = 0, rc2 = 0;
+    // setr! of the lane's particle (src/collisions.jl:63-74)
+    auto rate_bound = [&](double E) {
+        if (E < cut) return 0.0;
+        double t1, t2;
+        bool o;
+        const int i = precheb(E, kint, xmax, ixmax, two_k1, t1, t2, o);
+        oob |= o;
+        if (i != ci) {
+            ci = i;
+            if (P.rb_in_lds) {
+                const PT_LDS double* c = as_lds(pt_lds) + rb_off + 3 * i;
+                rc0 = c[0];
+                rc1 = c[1];
+                rc2 = c[2];
+            } else {
+                const PT_GLOBAL double* c =
+                    as_global(sh.sp[sp].rb) + ((size_t)(P.nswarm > 1 ? swarm : 0) * (kint + 1) + i) * 3;
+                rc0 = c[0];
+                rc1 = c[1];
+                rc2 = c[2];
+            }
+        }
+        return (rc0 * 1.0 + rc1 * t1) + rc2 * t2;
+    };
+    // with no dose tally nothing is left of a secondary below the cut; with one, its energy
+    const double dropcut = sh.cut[PT_ELECTRON] * (1.0 - 1e-9);
+    // the particle that has just been given to the lane: its species' and swarm's constants
+    auto settle = [&]() {
+        const SpLite& L = sh.sp[sp];
+        cut = L.cut;
+        pphi = L.ppcut_hi;
+        xmax = L.xmax;
+        ixmax = L.ixmax;
+        two_k1 = L.two_k1;
+        kint = L.k;
+        nprocs = L.nprocs;
+        rate_off = L.rate_off;
+        rb_off = L.rb_off;
+        ci = -1;
+        if (ffree) {
+            const PT_LDS double* e = as_lds(pt_lds) + P.lds_field_off + 6 * swarm;
+            const double q = (sp == PT_ELECTRON ? -1.0 : 1.0) * QE;
+            const bool none = sp == PT_PHOTON || (foff & off_em(sp));
+            F = V3{none ? 0.0 : q * e[0], none ? 0.0 : q * e[1], none ? 0.0 : q * e[2]};
+        }
+    };
     // the item loaded ahead for this lane
     bool ahead = false;
     int nsp = 0;
@@ -824,6 +899,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         have = true;
         child = ch;
         born = bo;
+        settle();
     };
     for (;;) {
         const bool first = !MULTI || extra == 0;
@@ -831,18 +907,17 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         //    memory.  A lane whose next item is loaded waits for the first push round after
         //    a collision phase, when its loads have had that phase's time.
         if (have && !pend && (!(trem > EPS64) || !active) && (first || !ahead)) {
-            const SpLite& L = sh.sp[sp];
             // droplow!: the energy is computed only where |p|^2 does not settle the test
-            if (active && !(dot3(p, p) > L.ppcut_hi)) {
+            if (active && !(dot3(p, p) > pphi)) {
                 double Ek = kinenergy(sp, p);
-                if (Ek < L.cut) {
+                if (Ek < cut) {
                     active = false;
                     deposit(P, sh.bc, Ek * w, x.z);
                 }
             }
             // a collision at the very end of the step: the record gets the new rate bound
             if (new_r) {
-                r = setr(L, kinenergy(sp, p), swarm, oob);
+                r = rate_bound(kinenergy(sp, p));
                 new_r = false;
             }
             if (oob) atomicAdd(&sh.bc.flags[FLAG_RANGE], 1ull);
@@ -865,7 +940,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
             }
             if (cont) {
                 // the next step's advance_init!: a new rate bound and random stream
-                g.init(P.seed, uid, step0 + (uint32_t)ks);
+                g.restart(step0 + (uint32_t)ks);
                 iters = 0;
                 nev = 0;
                 oob = false;
@@ -878,6 +953,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                 __builtin_amdgcn_sched_barrier(0);
                 // the particle's record: 72 contiguous bytes (w unchanged), written in whole
                 // sectors, four of the five stores 16 bytes wide
+                const SpLite& L = sh.sp[sp];
                 {
                     PT_GLOBAL pair2* w2 = rec_pairs(L, idx);
                     const pair2 v0 = {x.x, x.y}, v1 = {x.z, p.x}, v2 = {p.y, p.z}, v4 = {s, r};
@@ -971,6 +1047,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                             have = true;
                             child = ch;
                             born = false;
+                            settle();
                         } else {
                             take(qs, qi, a, 0, ch, false);
                         }
@@ -994,10 +1071,10 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         // setr! for a particle that changed: after its collision, at the start of a step, or
         // newly taken (one evaluation for all these lanes)
         if (new_r) {
-            r = setr(sh.sp[sp], kinenergy(sp, p), swarm, oob);
+            r = rate_bound(kinenergy(sp, p));
             new_r = false;
         }
-        const double tnext = s / r;
+        const double tnext = qdiv_any(s, r);
         // D. a lane whose push reaches the end of its last step without a collision retires at
         //    the next A: it claims its next item now and loads it while the push, the wave's
         //    collisions and the other lanes' work run, and takes it when it writes its particle
@@ -1043,7 +1120,6 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         // E. one push of this lane's particle.  In a further push round a lane whose push would
         //    end its last step waits, so that it loads its next item ahead.
         if (have && !pend && trem > EPS64 && active && (first || ks < K - 1 || trem > tnext)) {
-            const SpLite& L = sh.sp[sp];
             if (++iters > ITER_LIMIT || g.exhausted()) {
                 atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
                 trem = 0.0;
@@ -1062,7 +1138,10 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                 const double to = t;
                 V3 dx{0, 0, 0}, dp{0, 0, 0};
                 bool uniform;  // the force does not depend on the position
-                if (P.field_lds) {
+                if (ffree) {
+                    push_uniform(sp, F, falong, p, dt, dx, dp);
+                    uniform = true;
+                } else if (P.field_lds) {
                     const PT_LDS double* fv = as_lds(pt_lds) + P.lds_field_off + 6 * swarm;
                     const HomField hf{{fv}, {fv + 3}, {{nullptr, nullptr}}};
                     push_delta(sp, hf, x, p, dt, foff, dx, dp);
@@ -1085,7 +1164,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
                 trem -= dt;
                 if (coll && r != 0.0 && (!WALL || active)) {
                     const double E = kinenergy(sp, p);
-                    if (E >= L.cut) {
+                    if (E >= cut) {
                         nev++;
                         cE = E;
                         pend = true;
@@ -1128,35 +1207,45 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         int csel = -1;          // collision sampled in I
         bool rb_wait = false;   // an RBEB collision waiting for the cooperative loop
         double rb_w = -1.0;
+        ProcVals cp{0, 0.0, 0.0};  // what the common samplers need of its process
         if (pend) {
-            const SpLite& L = sh.sp[sp];
             pend = false;
             double t1, t2;
             bool o;
-            int iv = precheb(cE, L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o);
+            int iv = precheb(cE, kint, xmax, ixmax, two_k1, t1, t2, o);
             oob |= o;
             double xi = g.next() * r;
-            const int sel = select_process(as_lds(pt_lds) + L.rate_off + iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
+            const int sel = select_process(as_lds(pt_lds) + rate_off + iv * nprocs * 3, nprocs, t1, t2, xi);
             if (sel < 0) {
                 if (!(xi >= 0.0)) atomicAdd(&sh.bc.flags[FLAG_RATEBOUND], 1ull);
                 atomicAdd(&sh.bc.counts[sp * NCOUNT], 1ull);
                 new_r = true;  // setr! of the null collision (p unchanged)
                 s = nextcoll(g);
             } else {
-                atomicAdd(&sh.bc.counts[sp * NCOUNT + 1 + sel], 1ull);
                 const DevProc& pr = sh.procs[sp][sel];
-                if (EVENT && ((P.defer_mask >> pr.kind) & 1u)) {
+                cp.kind = pr.kind;
+                cp.B = pr.B;
+                cp.c0 = pr.c[0];
+                const double c1 = pr.c[1], c2 = pr.c[2];
+                atomicAdd(&sh.bc.counts[sp * NCOUNT + 1 + sel], 1ull);
+                if (EVENT && ((P.defer_mask >> cp.kind) & 1u)) {
                     qsel = sel;
                 } else {
                     csel = sel;
-                    if (pr.kind == PT_PROC_RBEB) {
-                        RbebJob& J = ((RbebJob*)wlds)[lane];
-                        J.s = rbeb_setup(cE, pr, g.tab());
+                    if (cp.kind == PT_PROC_RBEB) {
+                        PT_LDS RbebJob& J = ((PT_LDS RbebJob*)wlds)[lane];
+                        const RbebSetup js = rbeb_setup(cE, cp.B, cp.c0, c1, c2, g.tab());
+                        J.s.t = js.t;
+                        J.s.A = js.A;
+                        J.s.Cc = js.Cc;
+                        J.s.M = js.M;
+                        J.s.pbn = js.pbn;
+                        J.s.ratio = js.ratio;
+                        J.s.iratio = js.iratio;
                         J.first = g.c1;
                         J.uid = uid;
                         J.d0 = g.draw;
                         J.step = g.step;
-                        J.k = 0;
                         rb_wait = true;
                     }
                 }
@@ -1171,7 +1260,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         if constexpr (MLP) {
             int lw = -1;
             if (csel >= 0) {
-                const int kd = sh.procs[sp][csel].kind;
+                const int kd = cp.kind;
                 lw = kd == PT_PROC_SB ? LEARN_SB : (kd == PT_PROC_MOLLER ? LEARN_MOLLER : -1);
             }
             lnet = lw >= 0 && P.mlp[lw].on && cE >= P.mlp[lw].emin && cE <= P.mlp[lw].emax;
@@ -1181,24 +1270,43 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, char* w
         // I. the sampled collision
         ull sl0 = NO_SLOT, sl1 = NO_SLOT;  // slots of the secondaries it stored
         int cs0 = 0, cs1 = 0;
-        if (csel >= 0) {
+        // elastic scattering and ionisation are nearly all collisions of electrons: the lanes
+        // of both kinds go through one straight path together
+        const bool common = csel >= 0 && ((cp.kind == PT_PROC_ELASTIC && sp != PT_PHOTON) ||
+                                          (cp.kind == PT_PROC_RBEB && rb_w >= 0.0));
+        if (common) {
+            const bool el = cp.kind == PT_PROC_ELASTIC;
+            const double E2 = cp.B * rb_w;
+            const bool drop = el || E2 < dropcut;
+            V3 m0, m1;
+            double s0, s1;
+            const bool ok = common_event(el, cp, p, cE, E2, drop, g, m0, m1, s0, s1);
+            if (!el) {
+                if (!ok) atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
+                // left here: the binding energy, and that of a secondary below the cut
+                deposit(P, sh.bc, (drop ? cp.B + E2 : cp.B) * w, x.z);
+                if (!drop) {
+                    cs1 = PT_ELECTRON;
+                    sl1 = append(P, sh, PT_ELECTRON, x, m1, w, t, s1, uid, g.step, g.draw, 0, swarm, main_pass,
+                                 (uint32_t)ks);
+                }
+            }
+            p = m0;
+            s = s0;
+            new_r = true;  // setr! of apply!
+        } else if (csel >= 0) {
             const double E = cE;
-            double pn = norm3(p);
-            // the two common kinds draw their azimuth first here: one draw site for both
-            const int kind = sh.procs[sp][csel].kind;
-            double phi = -1.0;
-            if (kind == PT_PROC_ELASTIC || (kind == PT_PROC_RBEB && rb_w >= 0.0)) phi = TWO_PI * g.next();
-            // without a dose tally a secondary below the cut leaves nothing behind
-            const double dropcut = P.dose_bins > 0 ? -1.0 : sh.cut[PT_ELECTRON] * (1.0 - 1e-9);
+            const double pn = norm3(p);
             Ev e;
             if (MLP && lnet) learned_event(sh.procs[sp][csel], sp, E, ly0, ly1, g, e);
-            else sample_event(sh.procs[sp][csel], sp, p, pn, E, P.sb, P.pe, g, e, rb_w, phi, dropcut);
+            else sample_event(sh.procs[sp][csel], sp, p, pn, E, P.sb, P.pe, g, e, dropcut);
             if (e.err) atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
             if (e.dep != 0.0) deposit(P, sh.bc, e.dep * w, x.z);
             V3 m0, m1;
             double s0, s1;
             bool drop1;
             finish_event(p, pn, e, g, m0, m1, s0, s1, sh.cut, sh.stored, dropcut, drop1);
+            if (drop1) deposit(P, sh.bc, e.eB * w, x.z);
             const uint32_t dend = g.draw;
             if (e.keep) {
                 p = m0;
@@ -1388,7 +1496,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
         return;
     }
     stage(P, sh);
-    char* wlds = (char*)pt_lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES;
+    PT_LDS char* wlds = (PT_LDS char*)pt_lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES;
     select_loop<SRC, EVENT, WALL, MLP>(P, sh, wlds, rb, re, &P.clock->cursor, C.step,
                                        SRC == SRC_RANGE && C.pass == 0, par);
     flush_counters(P, &sh.bc);
@@ -1568,7 +1676,7 @@ __global__ void __launch_bounds__(512) k_tail(const Params* __restrict__ Pp, int
             rb[s] = beg[s];
             re[s] = end[s];
         }
-        select_loop<SRC_RANGE, false, WALL, MLP>(P, sh, (char*)pt_lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES,
+        select_loop<SRC_RANGE, false, WALL, MLP>(P, sh, (PT_LDS char*)pt_lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES,
                                                  rb, re, cur, step, false, 0);
     }
     // the pass limit was reached with work left: report it
@@ -2576,7 +2684,10 @@ static int sync_params(pt_ctx* c) {
             for (int d = 0; d < 3; d++) eok = eok && !(F.e.v[d] == 0.0 && std::signbit(F.e.v[d]));
         nob = nob && bzero && eok;
     }
-    c->hp.forcing_off = (c->hp.forcing_off & ~OFF_NO_B) | (nob ? OFF_NO_B : 0u);
+    // homogeneous electric fields along z only
+    bool along = hom;
+    for (const Field& F : c->hfields) along = along && F.e.v[0] == 0.0 && F.e.v[1] == 0.0;
+    c->hp.forcing_off = (c->hp.forcing_off & ~(OFF_NO_B | OFF_E_Z)) | (nob ? OFF_NO_B : 0u) | (along ? OFF_E_Z : 0u);
     c->hp.lds_field_off = off;
     if (hom) off += 6 * c->cfg.nswarm;
     off = (off + 1) & ~1;

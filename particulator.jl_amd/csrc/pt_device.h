@@ -123,6 +123,8 @@ __host__ __device__ constexpr uint32_t off_push(int sp) { return 64u << sp; }
 // absent) with no component -0.0.  Then each component of v x B is +0 or -0, and E + v x B
 // equals E bit for bit, so the electromagnetic force is qE.
 constexpr uint32_t OFF_NO_B = 1u << 9;
+// Set by the library: every swarm's E is homogeneous and along z.
+constexpr uint32_t OFF_E_Z = 1u << 10;
 
 // ---------------------------------------------------------------- Philox4x32-10
 // Salmon et al., SC'11: multipliers 0xD2511F53, 0xCD9E8D57; key increments 0x9E3779B9,
@@ -178,6 +180,12 @@ struct PhiloxStream {
         k1 = (uint32_t)(seed >> 32);
         u0 = (uint32_t)uid;
         u1 = (uint32_t)(uid >> 32);
+        step = st;
+        draw = 0;
+        cblk = 0;
+    }
+    // the same particle's stream of another step
+    __device__ __forceinline__ void restart(uint32_t st) {
         step = st;
         draw = 0;
         cblk = 0;
@@ -432,15 +440,15 @@ struct RbebSetup {
 // b' = B / mc^2, pr.c[1] = log(2 b'), pr.c[2] = 1 / B.  T / mc^2 and T / B are exact
 // divisions by constants (div_const).
 template <class T_>
-__device__ __forceinline__ RbebSetup rbeb_setup(double T, const DevProc& pr, T_ tab) {
+__device__ __forceinline__ RbebSetup rbeb_setup(double T, double B, double c0, double c1, double c2, T_ tab) {
     RbebSetup s;
     const double t1 = div_const_fin(T, MC2, 1.0 / MC2);
     const Recip g2((1.0 + t1) * (1.0 + t1));
     const double bt2 = 1.0 - g2.inverse();
-    const double b1 = pr.c[0];
-    s.t = div_const_fin(T, pr.B, pr.c[2]);
+    const double b1 = c0;
+    s.t = div_const_fin(T, B, c2);
     s.A = g2(qdiv(-(1.0 + 2.0 * t1), s.t + 1.0));
-    s.Cc = (log_tab(qdiv(bt2, 1.0 - bt2), tab) - bt2) - pr.c[1];
+    s.Cc = (log_tab(qdiv(bt2, 1.0 - bt2), tab) - bt2) - c1;
     s.M = g2(b1 * b1);
     s.pbn = 2.0 * 1.0 + 2.0 * s.Cc + (s.t + 1.0) * (s.t + 1.0) * 1.0 * s.M / 4.0;
     s.ratio = qdiv_any(s.t + 1.0, s.t - 1.0);
@@ -466,7 +474,7 @@ __device__ __forceinline__ bool rbeb_trip(const RbebSetup& s, double u, double z
 }
 template <class G>
 __device__ __forceinline__ double rbeb_sample(double T, const DevProc& pr, G& g) {
-    const RbebSetup s = rbeb_setup(T, pr, g.tab());
+    const RbebSetup s = rbeb_setup(T, pr.B, pr.c[0], pr.c[1], pr.c[2], g.tab());
     double w;
     for (;;) {
         double u, z;
@@ -803,6 +811,25 @@ __device__ __forceinline__ void push_delta(int sp, const FT& f, const V3& x, con
     dp = V3{q * (f1.x + 3.0 * f2.x), q * (f1.y + 3.0 * f2.y), q * (f1.z + 3.0 * f2.z)};
 }
 
+// the same for a force F that does not depend on position, momentum or time; `along`: F is
+// along z (the other components are zero, and adding a zero changes nothing)
+__device__ __forceinline__ void push_uniform(int sp, const V3& F, bool along, const V3& p, double dt, V3& dx, V3& dp) {
+    const V3 v1 = velocity(sp, p);
+    const double dt2 = 2.0 * dt, q = dt * 0.25;
+    constexpr double THIRD = 1.0 / 3.0;
+    V3 p2 = p;
+    dp = V3{0.0, 0.0, q * (F.z + 3.0 * F.z)};
+    p2.z = p.z + div_const_fin(dt2 * F.z, 3.0, THIRD);
+    if (!along) {
+        p2.x = p.x + div_const_fin(dt2 * F.x, 3.0, THIRD);
+        p2.y = p.y + div_const_fin(dt2 * F.y, 3.0, THIRD);
+        dp.x = q * (F.x + 3.0 * F.x);
+        dp.y = q * (F.y + 3.0 * F.y);
+    }
+    const V3 v2 = velocity(sp, p2);
+    dx = V3{q * (v1.x + 3.0 * v2.x), q * (v1.y + 3.0 * v2.y), q * (v1.z + 3.0 * v2.z)};
+}
+
 // the push itself; a species the pusher is restricted away from (RestrictedPusher,
 // NullPusher, src/pusher.jl:66-76) only has its time advanced
 template <class FT>
@@ -841,10 +868,7 @@ struct Ev {
 template <class G>
 __device__ __forceinline__ void sample_event(const DevProc& pr, int sp, const V3& p, double pnorm,
                                              double eng, const DevSB* sbs, const DevPE* pes, G& g,
-                                             Ev& e, double rbeb_w = -1.0, double phi = -1.0,
-                                             double dropcut = -1.0) {
-    // phi >= 0: the azimuth was drawn by the caller at the point where this event draws
-    // it (elastic: first; RBEB after a finished rejection loop: first)
+                                             Ev& e, double dropcut = -1.0) {
     e.err = 0;
     e.nturn = 1;
     e.sgnB = 1;
@@ -854,58 +878,9 @@ __device__ __forceinline__ void sample_event(const DevProc& pr, int sp, const V3
     e.eB = -1.0;
     e.src1 = SRC_A;
     e.sp1 = sp;
-    // The two common kinds side by side (an RBEB collision whose rejection loop has run):
-    // each lane takes its own operands to the same two square roots, division and division
-    // by c, so that a wave holding both kinds runs each of them once.  Operands and order of
-    // operations are those of the cases below.
-    //   elastic: g = sqrt(1 + c^2 p.p / (mc^2)^2), v = p / (m g), beta = |v| / c
-    //   RBEB: n = sqrt(E1^2 + 2 mc^2 E1) / c, cos = sqrt(E1 (E0 + 2 mc^2) / (E0 (E1 + 2 mc^2)))
-    const bool el = pr.kind == PT_PROC_ELASTIC && sp != PT_PHOTON;
-    const bool rb = pr.kind == PT_PROC_RBEB && rbeb_w >= 0.0;
-    if (el || rb) {
-        constexpr double MC2SQ = MC2 * MC2;
-        const double E0 = eng, E2 = pr.B * rbeb_w, E1 = E0 - E2 - pr.B;
-        const double pp = dot3(p, p);
-        const double r1 =
-            qsqrt(el ? 1.0 + div_const_fin(C2 * pp, MC2SQ, 1.0 / MC2SQ) : E1 * E1 + 2.0 * MC2 * E1);
-        const double q = qdiv(el ? 1.0 : E1 * (E0 + 2.0 * MC2), el ? ME * r1 : E0 * (E1 + 2.0 * MC2));
-        const V3 v{p.x * q, p.y * q, p.z * q};
-        const double r2 = qsqrt(el ? dot3(v, v) : q);
-        const double n = div_const_fin(el ? r2 : r1, C, 1.0 / C);
-        e.phi = phi >= 0.0 ? phi : TWO_PI * g.next();
-        if (el) {  // src/relativistic_coulomb.jl:10-23
-            const double a = pr.c[0];
-            const double al = qdiv(HBAR * HBAR, 4.0 * pp * (a * a));
-            e.cA = sample_rel_sr(al, n, g);
-            e.nA = pnorm;
-            e.keep = 1;
-            e.ne = 1;
-            e.src0 = SRC_A;
-            e.sp0 = sp;
-        } else {  // src/rbeb.jl:54-80
-            e.dep = pr.B;
-            if (!(E2 < E1)) e.err = 1;
-            e.nA = n;
-            e.eB = E2;
-            e.cA = r2;
-            if (!(E2 < dropcut)) {
-                e.nB = div_const_fin(qsqrt(E2 * E2 + 2.0 * MC2 * E2), C, 1.0 / C);
-                e.cB = qsqrt(qdiv(E2 * (E0 + 2.0 * MC2), E0 * (E2 + 2.0 * MC2)));
-            }
-            e.nturn = 2;
-            e.sgnB = -1;
-            e.keep = 1;
-            e.ne = 2;
-            e.src0 = SRC_A;
-            e.sp0 = sp;
-            e.src1 = SRC_B;
-            e.sp1 = PT_ELECTRON;
-        }
-        return;
-    }
     switch (pr.kind) {
     case PT_PROC_ELASTIC: {  // src/relativistic_coulomb.jl:10-23
-        e.phi = phi >= 0.0 ? phi : TWO_PI * g.next();
+        e.phi = TWO_PI * g.next();
         V3 v = velocity(sp, p);
         double beta = div_const(norm3(v), C, 1.0 / C);  // exact: |v| / c
         double a = pr.c[0];
@@ -923,8 +898,7 @@ __device__ __forceinline__ void sample_event(const DevProc& pr, int sp, const V3
     case PT_PROC_BHABHA: {  // src/bhaba.jl:9-33
         double E0 = eng, E1, E2;
         if (pr.kind == PT_PROC_RBEB) {
-            // rbeb_w >= 0: the rejection loop already ran (its stream position included)
-            E2 = rbeb_w >= 0.0 ? pr.B * rbeb_w : rbeb_sample(E0, pr, g);
+            E2 = rbeb_sample(E0, pr, g);
             E1 = E0 - E2 - pr.B;
             e.dep = pr.B;
             if (!(E2 < E1)) e.err = 1;
@@ -932,7 +906,7 @@ __device__ __forceinline__ void sample_event(const DevProc& pr, int sp, const V3
             E2 = pr.kind == PT_PROC_MOLLER ? moller_sample(pr.tcut, eng, g) : bhabha_sample(pr.tcut, eng, g);
             E1 = E0 - E2;
         }
-        e.phi = phi >= 0.0 ? phi : TWO_PI * g.next();
+        e.phi = TWO_PI * g.next();
         // Lehtinen 1999 angles; those of a secondary the caller drops unseen (E2 < dropcut,
         // see finish_event) are not needed
         e.nA = div_const(qsqrt(E1 * E1 + 2.0 * MC2 * E1), C, 1.0 / C);
@@ -1173,6 +1147,106 @@ __device__ __forceinline__ void finish_event(const V3& p, double pnorm, const Ev
     g.next12(e.ne == 2 ? 2 : 1, q0, q1);  // both draws at one place
     s0 = need0 ? -log_tab(q0, g.tab()) : 0.0;  // nextcoll(), src/util.jl:17
     s1 = need1 ? -log_tab(q1, g.tab()) : 0.0;
+}
+
+// What the common event needs of its process record, in registers.
+struct ProcVals {
+    int kind;
+    double B, c0;
+};
+
+// The two common collisions of electrons (and elastic ones of positrons) from selection to
+// momentum, for lanes of both kinds at once: `el`, elastic scattering (src/
+// relativistic_coulomb.jl:10-23), or an ionisation whose rejection loop has run and left a
+// secondary of energy E2 (src/rbeb.jl:54-80).  Operations and their order are those of
+// sample_event and finish_event (bit for bit: collision rounds sample these kinds there), but
+// each lane selects its operands and a wave runs every root, division, sine and logarithm
+// once for both kinds; the azimuth, the first trial of the elastic rejection loop and the
+// constructors' draws come from the two blocks that follow in the stream, computed at two
+// places instead of up to four.  `drop`: there is no secondary to return.  False: the
+// secondary's energy is not below the primary's.
+//   elastic: g = sqrt(1 + c^2 p.p / (mc^2)^2), v = p / (m g), beta = |v| / c
+//   ionisation: n = sqrt(E1^2 + 2 mc^2 E1) / c, cos = sqrt(E1 (E0 + 2 mc^2) / (E0 (E1 + 2 mc^2)))
+__device__ __forceinline__ bool common_event(bool el, const ProcVals& pv, const V3& p, double E0, double E2, bool drop,
+                                             StepStream& g, V3& m0, V3& m1, double& s0, double& s1) {
+    constexpr double MC2SQ = MC2 * MC2;
+    // the stream: q0, q1, q2, q3 are its next four draws
+    const uint32_t d = g.draw, blk = (d + 1) >> 1;
+    const bool odd = (d & 1) != 0;
+    const double half = g.c1;
+    g.fill(blk);
+    const double a0 = g.c0, a1 = g.c1;
+    double b0 = 0.0, b1 = 0.0;
+    if (el || !drop) {
+        g.fill(blk + 1);
+        b0 = g.c0;
+        b1 = g.c1;
+    }
+    const double q0 = odd ? half : a0, q1 = odd ? a0 : a1, q2 = odd ? a1 : b0, q3 = odd ? b0 : b1;
+    const double phi = TWO_PI * q0;
+    // energies and angles
+    const double pp = dot3(p, p), pn = qsqrt(pp);
+    const double E1 = E0 - E2 - pv.B;
+    const double r1 = qsqrt(el ? 1.0 + div_const_fin(C2 * pp, MC2SQ, 1.0 / MC2SQ) : E1 * E1 + 2.0 * MC2 * E1);
+    const double q = qdiv(el ? 1.0 : E1 * (E0 + 2.0 * MC2), el ? ME * r1 : E0 * (E1 + 2.0 * MC2));
+    const V3 v{p.x * q, p.y * q, p.z * q};
+    const double r2 = qsqrt(el ? dot3(v, v) : q);
+    const double n = div_const_fin(el ? r2 : r1, C, 1.0 / C);
+    double cA = r2, u0 = q1;  // u0: the draw of s
+    uint32_t used = 3;
+    if (el) {
+        // sample_rel_sr (src/relativistic_coulomb.jl:35-51), the first trial here
+        const double al = qdiv(HBAR * HBAR, 4.0 * pp * (pv.c0 * pv.c0));
+        const double xs = qdiv(al * q1, al + 1.0 - q1);
+        cA = 1.0 - 2.0 * xs;
+        used = 4;
+        u0 = q3;
+        if (!(q2 < 1.0 - n * n * xs)) {
+            // rejected: the loop goes on from the draw after this trial
+            g.draw = d + 3;
+            cA = sample_rel_sr(al, n, g);
+            u0 = g.next();
+            used = g.draw - d;
+        }
+    }
+    g.draw = d + used;
+    const double nA = el ? pn : n;
+    // turn (src/util.jl:40-57)
+    const Recip rp(pn);
+    const double w0 = rp(p.x), w1 = rp(p.y), w2 = rp(p.z);
+    double sp, cp;
+    sincos_turn(phi, sp, cp, g.tab());
+    const double qs = 1.0 - w2 * w2;
+    const double s = qsqrt(qs > 0.0 ? qs : 0.0);
+    const Recip rs(s);  // used where s > 0
+    {
+        const double qa = 1.0 - cA * cA;
+        const double st = qsqrt(qa > 0.0 ? qa : 0.0);
+        const double bx = w0 * w2 * cp + (-w1) * sp;
+        const double by = w1 * w2 * cp + w0 * sp;
+        const bool tilted = s > 0.0;
+        const double x = tilted ? rs(st * bx) + w0 * cA : st * cp;
+        const double y = tilted ? rs(st * by) + w1 * cA : st * sp;
+        const double z = tilted ? -s * st * cp + w2 * cA : w2 * cA;
+        m0 = V3{nA * x, nA * y, nA * z};
+    }
+    s0 = -log_tab(u0, g.tab());  // nextcoll(), src/util.jl:17
+    if (!drop) {
+        const double nB = div_const_fin(qsqrt(E2 * E2 + 2.0 * MC2 * E2), C, 1.0 / C);
+        const double cB = qsqrt(qdiv(E2 * (E0 + 2.0 * MC2), E0 * (E2 + 2.0 * MC2)));
+        const double spb = -sp;
+        const double qb = 1.0 - cB * cB;
+        const double st = qsqrt(qb > 0.0 ? qb : 0.0);
+        const double bx = w0 * w2 * cp + (-w1) * spb;
+        const double by = w1 * w2 * cp + w0 * spb;
+        const bool tilted = s > 0.0;
+        const double x = tilted ? rs(st * bx) + w0 * cB : st * cp;
+        const double y = tilted ? rs(st * by) + w1 * cB : st * spb;
+        const double z = tilted ? -s * st * cp + w2 * cB : w2 * cB;
+        m1 = V3{nB * x, nB * y, nB * z};
+        s1 = -log_tab(q2, g.tab());
+    }
+    return el || E2 < E1;
 }
 
 }  // namespace pt
