@@ -117,6 +117,16 @@ struct WallDev {
     int pad;
 };
 
+// What the host reads after nearly every call, written by the kernels into pinned host memory,
+// so that a call ends with one synchronisation and no copies.
+constexpr int NSTAT = 8;
+struct Report {
+    ull n[PT_NSPECIES];  // slots in use
+    ull flags[NFLAGS];
+    ull left;            // secondaries the last pass left to a further one
+    double stat[NSTAT];  // population statistics (k_stats)
+};
+
 struct Params {
     SpeciesDev sp[PT_NSPECIES];
     DevTable tab[PT_NSPECIES];
@@ -149,6 +159,7 @@ struct Params {
     int lds_rate_off[PT_NSPECIES];
     int lds_rb_off[PT_NSPECIES];
     int lds_doubles;      // even
+    Report* report;       // pinned host memory
     ull* image;           // what a workgroup stages: the Staged block, then lds_doubles doubles
 };
 
@@ -763,7 +774,8 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
     const ull nwaves = (ull)gridDim.x * (blockDim.x >> 6);
     const int lanes = lanes_used(total, nwaves);
     const ull least = lanes < LEAST_CHUNK ? lanes : LEAST_CHUNK;
-    ull chunk = claim_chunk(total, nwaves, least);
+    // (the first one fills the wave's lanes at once: each further claim is a round trip)
+    ull chunk = total / nwaves > 64 ? claim_chunk(4 * total, nwaves, least) : (ull)lanes;
     ull cbeg = 0, cend = 0;
     bool drained = false;
     // the wave's next chunk of items; false when they are all claimed
@@ -1406,6 +1418,22 @@ __global__ void k_snapshot(const Params* __restrict__ Pp, int clocked, double tf
     }
 }
 
+template <class T>
+__device__ __forceinline__ void to_host(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void report_state(const Params& P, ull left) {
+    Report& R = *P.report;
+    for (int s = 0; s < PT_NSPECIES; s++)
+        to_host(&R.n[s], __hip_atomic_load(P.sp[s].n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    for (int q = 0; q < NFLAGS; q++)
+        to_host(&R.flags[q], __hip_atomic_load(&P.flags[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    to_host(&R.left, left);
+}
+__global__ void k_report(const Params* __restrict__ Pp) {
+    if (threadIdx.x == 0) report_state(*Pp, 0);
+}
+
 // The end of a pass, called by every workgroup of its launch: the last one to end sets up the
 // next advance1! pass (src/mixed_population.jl:43-46) over the particles appended since the
 // last mark, for the whole grid.  When every secondary found room on its wave's stack there is
@@ -1431,6 +1459,7 @@ __device__ __forceinline__ void end_pass(const Params& P) {
     C.pass += 1;
     C.left = 0;
     C.done = 0;
+    report_state(P, left);
 }
 
 __global__ void k_tick(const Params* __restrict__ Pp) {
@@ -1491,7 +1520,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
     __syncthreads();
     if (skip) {
         if constexpr (!EVENT) {
-            if (total > 0) end_pass(P);  // (a pass over nothing leaves the next one empty, too)
+            // (a further pass over nothing leaves the next one empty, too)
+            if (total > 0 || C.pass == 0) end_pass(P);
         }
         return;
     }
@@ -2120,6 +2150,9 @@ __global__ void __launch_bounds__(256) k_split(const Params* __restrict__ Pp, in
 // (One launch per kernel and species, with a grid over the whole capacity: 52 us for three
 // nearly empty species of 2^27 slots, now 11.)
 constexpr int CH = 4096;  // slots per chunk: one 16-byte read of flags per thread of a workgroup
+// chunks that one workgroup compacts alone, in one launch (16384 slots: 14 us, with three
+// launches 17; with twice as many the one workgroup takes longer)
+constexpr int CMP_SMALL = 4;
 struct Compaction {
     SpeciesDev sp[PT_NSPECIES];
     unsigned* cnt[PT_NSPECIES];   // actives of each chunk
@@ -2129,6 +2162,7 @@ struct Compaction {
     unsigned* tpos[PT_NSPECIES];
     ull* info;  // per species: active count, moves, slots in use before, workgroups done
     ull* work;
+    Report* report;
 };
 
 // bit i: flag i of the 16 from slot i0 is set (slots from n on: not)
@@ -2170,6 +2204,43 @@ __device__ __forceinline__ unsigned block_prefix(unsigned v, unsigned* wsum, uns
     return base + inc - v;
 }
 
+// positions of the k-th hole and the k-th active above, in chunk order
+__device__ __forceinline__ void fill_chunk(const Compaction& cp, int s, int c, int nchunks, ull A, ull n, ull moves,
+                                           unsigned* wsum) {
+    const unsigned h0 = cp.hole[s][c], t0 = cp.tail[s][c];
+    const unsigned h1 = c + 1 < nchunks ? cp.hole[s][c + 1] : (unsigned)moves;
+    const unsigned t1 = c + 1 < nchunks ? cp.tail[s][c + 1] : (unsigned)moves;
+    if (h1 == h0 && t1 == t0) return;
+    const ull i0 = (ull)c * CH + 16 * threadIdx.x;
+    const unsigned act = flags16(cp.sp[s].active, i0, n);
+    const unsigned below = i0 >= A ? 0u : i0 + 16 <= A ? 0xFFFFu : (1u << (A - i0)) - 1u;
+    unsigned holes = below & ~act, tails = act & ~below, tot;
+    unsigned hk = h0 + block_prefix(__popc(holes), wsum, tot), tk = t0 + block_prefix(__popc(tails), wsum, tot);
+    for (; holes; holes &= holes - 1) cp.hpos[s][hk++] = (unsigned)(i0 + __ffs(holes) - 1);
+    for (; tails; tails &= tails - 1) cp.tpos[s][tk++] = (unsigned)(i0 + __ffs(tails) - 1);
+}
+
+// the k-th active above the active count into the k-th hole below it, k = k0, k0 + step, ...
+__device__ __forceinline__ void move_slots(const Compaction& cp, int s, ull m, ull k0, ull step) {
+    const SpeciesDev& S = cp.sp[s];
+    for (ull k = k0; k < m; k += step) {
+        const unsigned d = cp.hpos[s][k], q = cp.tpos[s][k];
+        const PT_GLOBAL pair2* from = (const PT_GLOBAL pair2*)&PF(S.f[0], q);
+        PT_GLOBAL pair2* to = (PT_GLOBAL pair2*)&PF(S.f[0], d);
+        pair2 v[PT_NFIELDS / 2];
+#pragma unroll
+        for (int f = 0; f < PT_NFIELDS / 2; f++) v[f] = from[f];
+        const uint64_t u = S.uid[q];
+        const int32_t w = S.swarm[q];
+#pragma unroll
+        for (int f = 0; f < PT_NFIELDS / 2; f++) to[f] = v[f];
+        S.uid[d] = u;
+        S.swarm[d] = w;
+        S.active[d] = 1;
+    }
+    if (m && k0 == 0) atomicAdd(&cp.work[W_MOVED], m);
+}
+
 __global__ void __launch_bounds__(256) k_cmp_count(const Compaction cp, unsigned mask) {
     const int s = blockIdx.y;
     if (!((mask >> s) & 1)) return;
@@ -2179,12 +2250,13 @@ __global__ void __launch_bounds__(256) k_cmp_count(const Compaction cp, unsigned
     ull n = *S.n;
     if (n > S.cap) n = S.cap;
     const int nchunks = (int)((n + CH - 1) / CH);
-    // the workgroups that have a chunk (the first one always takes part)
-    const int parts = nchunks < 1 ? 1 : nchunks < (int)gridDim.x ? nchunks : (int)gridDim.x;
+    // the workgroups that have a chunk (the first one always takes part); a few chunks are left
+    // to one workgroup, which then does the moves as well
+    const int parts = nchunks <= CMP_SMALL ? 1 : nchunks < (int)gridDim.x ? nchunks : (int)gridDim.x;
     if ((int)blockIdx.x >= parts) return;
     __shared__ unsigned wsum[4];
     __shared__ bool last;
-    for (int c = blockIdx.x; c < nchunks; c += gridDim.x) {
+    for (int c = blockIdx.x; c < nchunks; c += parts) {
         unsigned tot;
         (void)block_prefix(__popc(flags16(S.active, (ull)c * CH + 16 * threadIdx.x, n)), wsum, tot);
         // (read by the last workgroup, which may be on another die)
@@ -2232,14 +2304,20 @@ __global__ void __launch_bounds__(256) k_cmp_count(const Compaction cp, unsigned
     }
     if (threadIdx.x == 0) {
         info[0] = A;
-        info[1] = htot;  // holes below A == actives from A on
+        info[1] = parts == 1 ? 0 : htot;  // holes below A == actives from A on, still to be moved
         info[2] = n;
         info[3] = 0;
         *S.n = A;
+        __hip_atomic_store(&cp.report->n[s], A, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (parts == 1 && htot) {
+        __syncthreads();
+        for (int c = 0; c < nchunks; c++) fill_chunk(cp, s, c, nchunks, A, n, htot, wsum);
+        __syncthreads();
+        move_slots(cp, s, htot, threadIdx.x, blockDim.x);
     }
 }
 
-// positions of the k-th hole and the k-th active above, in chunk order
 __global__ void __launch_bounds__(256) k_cmp_fill(const Compaction cp, unsigned mask) {
     const int s = blockIdx.y;
     const ull* const info = cp.info + 4 * s;
@@ -2247,42 +2325,13 @@ __global__ void __launch_bounds__(256) k_cmp_fill(const Compaction cp, unsigned 
     if (!((mask >> s) & 1) || moves == 0) return;
     __shared__ unsigned wsum[4];
     const int nchunks = (int)((n + CH - 1) / CH);
-    for (int c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        const unsigned h0 = cp.hole[s][c], t0 = cp.tail[s][c];
-        const unsigned h1 = c + 1 < nchunks ? cp.hole[s][c + 1] : (unsigned)moves;
-        const unsigned t1 = c + 1 < nchunks ? cp.tail[s][c + 1] : (unsigned)moves;
-        if (h1 == h0 && t1 == t0) continue;
-        const ull i0 = (ull)c * CH + 16 * threadIdx.x;
-        const unsigned act = flags16(cp.sp[s].active, i0, n);
-        const unsigned below = i0 >= A ? 0u : i0 + 16 <= A ? 0xFFFFu : (1u << (A - i0)) - 1u;
-        unsigned holes = below & ~act, tails = act & ~below, tot;
-        unsigned hk = h0 + block_prefix(__popc(holes), wsum, tot), tk = t0 + block_prefix(__popc(tails), wsum, tot);
-        for (; holes; holes &= holes - 1) cp.hpos[s][hk++] = (unsigned)(i0 + __ffs(holes) - 1);
-        for (; tails; tails &= tails - 1) cp.tpos[s][tk++] = (unsigned)(i0 + __ffs(tails) - 1);
-    }
+    for (int c = blockIdx.x; c < nchunks; c += gridDim.x) fill_chunk(cp, s, c, nchunks, A, n, moves, wsum);
 }
 
 __global__ void __launch_bounds__(256) k_cmp_move(const Compaction cp, unsigned mask) {
     const int s = blockIdx.y;
     if (!((mask >> s) & 1)) return;
-    const SpeciesDev& S = cp.sp[s];
-    const ull m = cp.info[4 * s + 1];
-    for (ull k = (ull)blockIdx.x * blockDim.x + threadIdx.x; k < m; k += (ull)gridDim.x * blockDim.x) {
-        const unsigned d = cp.hpos[s][k], q = cp.tpos[s][k];
-        const PT_GLOBAL pair2* from = (const PT_GLOBAL pair2*)&PF(S.f[0], q);
-        PT_GLOBAL pair2* to = (PT_GLOBAL pair2*)&PF(S.f[0], d);
-        pair2 v[PT_NFIELDS / 2];
-#pragma unroll
-        for (int f = 0; f < PT_NFIELDS / 2; f++) v[f] = from[f];
-        const uint64_t u = S.uid[q];
-        const int32_t w = S.swarm[q];
-#pragma unroll
-        for (int f = 0; f < PT_NFIELDS / 2; f++) to[f] = v[f];
-        S.uid[d] = u;
-        S.swarm[d] = w;
-        S.active[d] = 1;
-    }
-    if (m && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&cp.work[W_MOVED], m);
+    move_slots(cp, s, cp.info[4 * s + 1], (ull)blockIdx.x * blockDim.x + threadIdx.x, (ull)gridDim.x * blockDim.x);
 }
 
 // ------------------------------------------------------------------ copies of the state
@@ -2305,52 +2354,106 @@ __global__ void __launch_bounds__(256) k_copy_ranges(const Copies c) {
 }
 
 // ------------------------------------------------------------------ statistics
-// per-block partial sums over active particles: count, w, w*E, w*x, w*y, w*z, w*|x|^2, maxE
-constexpr int NSTAT = 8;
-__global__ void __launch_bounds__(256) k_stats_partial(const Params* __restrict__ Pp, int sp,
-                                                       double* __restrict__ part) {
+// sums over active particles: count, w, w*E, w*x, w*y, w*z, w*|x|^2, and max E; each workgroup
+// leaves its part and the last one adds them up and reports them.  Bound by memory (a record's
+// first 64 bytes: the whole line): every lane reads its particle with 16-byte loads, two
+// particles at a time.  2 x 10^6 particles: 49 -> 33 us (with the host's sum of the parts, which
+// this saves, 85 -> 40).
+__device__ __forceinline__ double agent_load(const double* p) {
+    return __longlong_as_double(
+        (long long)__hip_atomic_load((const ull*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+__device__ __forceinline__ void agent_store(double* p, double v) {
+    __hip_atomic_store((ull*)p, (ull)__double_as_longlong(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// sums of a[] over the workgroup (the last one: maximum), in threads 0..NSTAT-1
+__device__ __forceinline__ double stat_reduce(double a[NSTAT]) {
+    __shared__ double red[4][NSTAT];
+#pragma unroll
+    for (int q = 0; q < NSTAT; q++)
+        for (int off = 32; off > 0; off >>= 1) {
+            const double o = __shfl_down(a[q], off, 64);
+            a[q] = q == NSTAT - 1 ? fmax(a[q], o) : a[q] + o;
+        }
+    if ((threadIdx.x & 63) == 0)
+        for (int q = 0; q < NSTAT; q++) red[threadIdx.x >> 6][q] = a[q];
+    __syncthreads();
+    double v = 0.0;
+    if (threadIdx.x < NSTAT)
+        for (int k = 0; k < 4; k++)
+            v = threadIdx.x == NSTAT - 1 ? fmax(v, red[k][threadIdx.x]) : v + red[k][threadIdx.x];
+    __syncthreads();
+    return v;
+}
+constexpr int STAT_BLOCKS = 1024;
+__global__ void __launch_bounds__(256) k_stats(const Params* __restrict__ Pp, int sp, double* __restrict__ part,
+                                               ull* __restrict__ ticket) {
     const Params& P = *Pp;
     const SpeciesDev& S = P.sp[sp];
+    __shared__ bool last;
     ull n = *S.n;
     if (n > S.cap) n = S.cap;
     double a[NSTAT] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (ull i = (ull)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (ull)gridDim.x * blockDim.x) {
-        if (!S.active[i]) continue;
-        V3 p{PF(S.f[PT_PX], i), PF(S.f[PT_PY], i), PF(S.f[PT_PZ], i)};
-        V3 x{PF(S.f[PT_X], i), PF(S.f[PT_Y], i), PF(S.f[PT_Z], i)};
-        double w = PF(S.f[PT_W], i);
-        double E = kinenergy(sp, p);
-        a[0] += 1.0;
-        a[1] += w;
-        a[2] += w * E;
-        a[3] += w * x.x;
-        a[4] += w * x.y;
-        a[5] += w * x.z;
-        a[6] += w * dot3(x, x);
-        a[7] = fmax(a[7], E);
+    const ull stride = (ull)gridDim.x * blockDim.x;
+    for (ull i0 = (ull)blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += 2 * stride) {
+        pair2 v[2][4];
+        bool act[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const ull i = i0 + u * stride < n ? i0 + u * stride : i0;
+            const PT_GLOBAL pair2* r = (const PT_GLOBAL pair2*)&PF(S.f[0], i);
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[u][q] = r[q];
+            act[u] = S.active[i] && (u == 0 || i != i0);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            if (!act[u]) continue;
+            const V3 x{v[u][0].x, v[u][0].y, v[u][1].x}, p{v[u][1].y, v[u][2].x, v[u][2].y};
+            const double w = v[u][3].x, E = kinenergy(sp, p);
+            a[0] += 1.0;
+            a[1] += w;
+            a[2] += w * E;
+            a[3] += w * x.x;
+            a[4] += w * x.y;
+            a[5] += w * x.z;
+            a[6] += w * dot3(x, x);
+            a[7] = fmax(a[7], E);
+        }
     }
-    __shared__ double red[NSTAT][256];
-    for (int q = 0; q < NSTAT; q++) red[q][threadIdx.x] = a[q];
+    const double mine = stat_reduce(a);
+    if (threadIdx.x < NSTAT) agent_store(&part[blockIdx.x * NSTAT + threadIdx.x], mine);
+    wait_vmem();
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off)
-            for (int q = 0; q < NSTAT; q++) {
-                if (q == 7) red[q][threadIdx.x] = fmax(red[q][threadIdx.x], red[q][threadIdx.x + off]);
-                else red[q][threadIdx.x] += red[q][threadIdx.x + off];
-            }
-        __syncthreads();
-    }
-    if (threadIdx.x < NSTAT) part[blockIdx.x * NSTAT + threadIdx.x] = red[threadIdx.x][0];
+    if (threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    double t[NSTAT] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x)
+        for (int q = 0; q < NSTAT; q++) {
+            const double v = agent_load(&part[b * NSTAT + q]);
+            t[q] = q == NSTAT - 1 ? fmax(t[q], v) : t[q] + v;
+        }
+    const double sum = stat_reduce(t);
+    if (threadIdx.x < NSTAT) to_host(&P.report->stat[threadIdx.x], sum);
+    if (threadIdx.x == 0) *ticket = 0;
 }
 
-
-// per-swarm sums over active particles: count, w, w*E and max E of each swarm.  With up
-// to SWARM_LDS swarms a workgroup accumulates in LDS and adds its partial sums once;
-// beyond that it adds into global memory directly.  out[4*i + 3] holds max E as the bit
-// pattern of a non-negative double (ordered like the value).
+// per-swarm sums over active particles: count, w, w*E and max E of each swarm.  Each workgroup
+// has a run of consecutive slots, and each lane adds up its particles in registers as long as
+// they belong to one swarm (they mostly do: swarms are laid out one after the other), then
+// once into LDS (up to SWARM_LDS swarms; beyond that into global memory directly), and the
+// workgroup adds what it found to the output.  (With an LDS atomic per particle the 64 lanes of
+// a wave met on one address four times over: 2 x 10^6 particles 89 us, now 31.)
+// out[4*i + 3] holds max E as the bit pattern of a non-negative double (ordered like the value).
 constexpr int SWARM_LDS = 1024;
+// With `host` (pinned memory) the last workgroup copies the sums there and clears `out` for the
+// next call.
 __global__ void __launch_bounds__(256) k_swarm_stats(const Params* __restrict__ Pp, int sp, int nswarm,
-                                                     double* __restrict__ out) {
+                                                     double* __restrict__ out, double* __restrict__ host,
+                                                     ull* __restrict__ ticket) {
+    __shared__ bool last;
     __shared__ double acc[3 * SWARM_LDS];
     __shared__ ull emax[SWARM_LDS];
     const Params& P = *Pp;
@@ -2363,26 +2466,53 @@ __global__ void __launch_bounds__(256) k_swarm_stats(const Params* __restrict__ 
     }
     ull n = *S.n;
     if (n > S.cap) n = S.cap;
-    for (ull i = (ull)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (ull)gridDim.x * blockDim.x) {
-        if (!S.active[i]) continue;
-        int sw = S.swarm[i];
-        if (sw < 0 || sw >= nswarm) continue;
-        V3 p{PF(S.f[PT_PX], i), PF(S.f[PT_PY], i), PF(S.f[PT_PZ], i)};
-        double w = PF(S.f[PT_W], i);
-        double E = kinenergy(sp, p);
-        ull eb = (ull)__double_as_longlong(E > 0.0 ? E : 0.0);
+    const ull per = (n + gridDim.x - 1) / gridDim.x;
+    const ull beg = (ull)blockIdx.x * per, end = beg + per < n ? beg + per : n;
+    int cur = -1;
+    double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
+    auto leave = [&]() {
+        if (cur < 0) return;
+        const ull eb = (ull)__double_as_longlong(c3);
         if (local) {
-            atomicAdd(&acc[3 * sw], 1.0);
-            atomicAdd(&acc[3 * sw + 1], w);
-            atomicAdd(&acc[3 * sw + 2], w * E);
-            atomicMax(&emax[sw], eb);
+            atomicAdd(&acc[3 * cur], c0);
+            atomicAdd(&acc[3 * cur + 1], c1);
+            atomicAdd(&acc[3 * cur + 2], c2);
+            atomicMax(&emax[cur], eb);
         } else {
-            atomicAdd(&out[4 * sw], 1.0);
-            atomicAdd(&out[4 * sw + 1], w);
-            atomicAdd(&out[4 * sw + 2], w * E);
-            atomicMax((ull*)&out[4 * sw + 3], eb);
+            atomicAdd(&out[4 * cur], c0);
+            atomicAdd(&out[4 * cur + 1], c1);
+            atomicAdd(&out[4 * cur + 2], c2);
+            atomicMax((ull*)&out[4 * cur + 3], eb);
         }
+        c0 = c1 = c2 = c3 = 0.0;
+    };
+    for (ull i = beg + threadIdx.x; i < end; i += blockDim.x) {
+        const PT_GLOBAL pair2* r = (const PT_GLOBAL pair2*)&PF(S.f[0], i);
+        const pair2 v1 = r[1], v2 = r[2], v3 = r[3];
+        const int sw = S.swarm[i];
+        if (!S.active[i] || sw < 0 || sw >= nswarm) continue;
+        if (sw != cur) {
+            leave();
+            cur = sw;
+        }
+        const double E = kinenergy(sp, V3{v1.y, v2.x, v2.y});
+        c0 += 1.0;
+        c1 += v3.x;
+        c2 += v3.x * E;
+        c3 = fmax(c3, E > 0.0 ? E : 0.0);
     }
+    // the lanes of a wave that ends in one swarm are added up first
+    const int lead = __builtin_amdgcn_readfirstlane(cur);
+    if (__ballot(cur != lead) == 0) {
+        for (int off = 32; off > 0; off >>= 1) {
+            c0 += __shfl_down(c0, off, 64);
+            c1 += __shfl_down(c1, off, 64);
+            c2 += __shfl_down(c2, off, 64);
+            c3 = fmax(c3, __shfl_down(c3, off, 64));
+        }
+        if ((threadIdx.x & 63) != 0) cur = -1;
+    }
+    leave();
     if (local) {
         __syncthreads();
         for (int q = threadIdx.x; q < nswarm; q += blockDim.x) {
@@ -2393,6 +2523,18 @@ __global__ void __launch_bounds__(256) k_swarm_stats(const Params* __restrict__ 
             atomicMax((ull*)&out[4 * q + 3], emax[q]);
         }
     }
+    if (!host) return;
+    wait_vmem();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    for (int q = threadIdx.x; q < 4 * nswarm; q += blockDim.x) {
+        to_host(&host[q], agent_load(&out[q]));
+        agent_store(&out[q], 0.0);
+    }
+    if (threadIdx.x == 0) *ticket = 0;
 }
 
 // p[0..n) = 0 (a kernel, not a memset, so that it can also be captured in a graph)
@@ -2531,8 +2673,11 @@ struct pt_ctx {
     hipStream_t stream = nullptr;
     Params hp{};          // host copy of the parameters
     Params* dp = nullptr;  // device copy
+    Report* report = nullptr;  // pinned: what kernels report
     bool dirty = true;
     std::vector<void*> allocs;
+    char* slab = nullptr;  // block that small allocations are cut from
+    size_t slab_used = 0;
     // per species
     ull* dn = nullptr;  // [3] counters
     ull hn[PT_NSPECIES] = {0, 0, 0};  // host view of the counts: exact while counts_known
@@ -2577,9 +2722,9 @@ struct pt_ctx {
     int resident[MAX_KV][3] = {};  // resident workgroups per CU: kernel variant x block 128/256/512
     bool queues = false;      // work and collision queues allocated
     int resident_lds = -1;        // LDS size the residency was computed for
-    int stat_cap = 0;             // swarms the per-swarm statistics buffer holds
     double* noalloc = nullptr;    // this device's copy of the allocation-free scratch array
-    double* swarm_part = nullptr;
+    double* swarm_part = nullptr;  // per-swarm sums (zero between calls), and their copy in
+    double* swarm_host = nullptr;  // pinned memory (behind the report)
     // learned samplers
     struct Learned {
         float* params = nullptr;  // FP32 parameters (device)
@@ -2660,14 +2805,32 @@ static int noalloc_scratch(pt_ctx* c) {
     return PT_OK;
 }
 
-static int dalloc(pt_ctx* c, void** p, size_t bytes) {
-    if (bytes == 0) bytes = 8;
-    hipError_t e = hipMalloc(p, bytes);
+// device memory of its own, freed with the context
+static int dalloc_own(pt_ctx* c, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes ? bytes : 8);
     if (e != hipSuccess) {
         (void)hipGetLastError();  // reported here: a later launch's check must not find it
+        *p = nullptr;
         return fail(c, PT_E_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     }
     c->allocs.push_back(*p);
+    return PT_OK;
+}
+
+// device memory, the small pieces from a zeroed block (a context has some forty of them, and
+// each hipMalloc or clearing takes several us)
+static int dalloc(pt_ctx* c, void** p, size_t bytes) {
+    constexpr size_t BLOCK = 1 << 20, SMALL = 1 << 16;
+    if (bytes > SMALL) return dalloc_own(c, p, bytes);
+    const size_t need = std::max<size_t>(256, (bytes + 255) & ~(size_t)255);
+    if (!c->slab || c->slab_used + need > BLOCK) {
+        int rc = dalloc_own(c, (void**)&c->slab, BLOCK);
+        if (rc) return rc;
+        c->slab_used = 0;
+        HIPCHK(c, hipMemsetAsync(c->slab, 0, BLOCK, c->stream));
+    }
+    *p = c->slab + c->slab_used;
+    c->slab_used += need;
     return PT_OK;
 }
 
@@ -2720,14 +2883,22 @@ static int sync_params(pt_ctx* c) {
     return PT_OK;
 }
 
-static int read_counts(pt_ctx* c) {
-    HIPCHK(c, hipMemcpyAsync(c->hn, c->dn, sizeof(ull) * PT_NSPECIES, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int s = 0; s < PT_NSPECIES; s++)
-        if (c->hn[s] > c->cfg.capacity[s]) c->hn[s] = c->cfg.capacity[s];
+// the counts that a finished kernel has reported
+static void take_counts(pt_ctx* c) {
+    for (int s = 0; s < PT_NSPECIES; s++) c->hn[s] = std::min<ull>(c->report->n[s], c->cfg.capacity[s]);
     c->counts_known = true;
+}
+
+// counts and flags as they are now
+static int read_state(pt_ctx* c) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, c->stream, c->dp);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    take_counts(c);
     return PT_OK;
 }
+
+static int read_counts(pt_ctx* c) { return c->counts_known ? PT_OK : read_state(c); }
 
 template <class T>
 struct Scratch {
@@ -2791,6 +2962,7 @@ void pt_destroy(pt_ctx* c) {
     for (auto& g : c->gexec)
         if (g) (void)hipGraphExecDestroy(g);
     for (void* p : c->allocs) (void)hipFree(p);
+    if (c->report) (void)hipHostFree(c->report);
     for (auto& e : c->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : c->evq)
@@ -2837,8 +3009,17 @@ int pt_create(const pt_config* cfg, pt_ctx** out) {
         TRY(fail(c, PT_E_HIP, "hipStreamCreate failed"));
     for (auto& e : c->ev)
         if (hipEventCreate(&e) != hipSuccess) TRY(fail(c, PT_E_HIP, "hipEventCreate failed"));
+    const size_t pinned = sizeof(Report) + sizeof(double) * 4 * (size_t)c->cfg.nswarm;
+    if (hipHostMalloc((void**)&c->report, pinned, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->report = nullptr;
+        TRY(fail(c, PT_E_NOMEM, "pinned host memory allocation of %zu bytes failed", pinned));
+    }
+    c->swarm_host = (double*)(c->report + 1);
     Params& P = c->hp;
     memset(&P, 0, sizeof(P));
+    memset(c->report, 0, sizeof(Report));
+    P.report = c->report;
     TRY(dalloc(c, (void**)&c->dn, sizeof(ull) * PT_NSPECIES));
     for (int s = 0; s < PT_NSPECIES; s++) {
         SpeciesDev& S = P.sp[s];
@@ -2846,15 +3027,22 @@ int pt_create(const pt_config* cfg, pt_ctx** out) {
         S.cap = cap;
         S.tracked = c->cfg.tracked[s];
         S.n = c->dn + s;
-        // one record array: slot i's field k at f[0][i * PT_NFIELDS + k]
-        TRY(dalloc(c, (void**)&S.f[0], sizeof(double) * PT_NFIELDS * cap));
+        // one allocation: the records (slot i's field k at f[0][i * PT_NFIELDS + k]), then the
+        // columns
+        const size_t size[7] = {sizeof(double) * PT_NFIELDS, sizeof(uint64_t), sizeof(int32_t), sizeof(double),
+                                sizeof(uint32_t), 1, 1};
+        size_t off[8] = {0};
+        for (int q = 0; q < 7; q++) off[q + 1] = off[q] + ((size[q] * std::max<ull>(cap, 1) + 255) & ~(size_t)255);
+        char* base = nullptr;
+        TRY(dalloc(c, (void**)&base, off[7]));
+        S.f[0] = (double*)base;
         for (int f = 1; f < PT_NFIELDS; f++) S.f[f] = S.f[0] + f;
-        TRY(dalloc(c, (void**)&S.active, cap));
-        TRY(dalloc(c, (void**)&S.uid, sizeof(uint64_t) * cap));
-        TRY(dalloc(c, (void**)&S.swarm, sizeof(int32_t) * cap));
-        TRY(dalloc(c, (void**)&S.trem, sizeof(double) * cap));
-        TRY(dalloc(c, (void**)&S.draw, sizeof(uint32_t) * cap));
-        TRY(dalloc(c, (void**)&S.evp, cap));
+        S.uid = (uint64_t*)(base + off[1]);
+        S.swarm = (int32_t*)(base + off[2]);
+        S.trem = (double*)(base + off[3]);
+        S.draw = (uint32_t*)(base + off[4]);
+        S.active = (uint8_t*)(base + off[5]);
+        S.evp = (uint8_t*)(base + off[6]);
         HIPCHK(c, hipMemsetAsync(S.active, 0, cap ? cap : 1, c->stream));
     }
     HIPCHK(c, hipMemsetAsync(c->dn, 0, sizeof(ull) * PT_NSPECIES, c->stream));
@@ -2905,18 +3093,25 @@ int pt_create(const pt_config* cfg, pt_ctx** out) {
     for (int s = 0; s < PT_NSPECIES; s++) {
         const size_t cap = c->cfg.capacity[s], chunks = (cap + CH - 1) / CH + 1;
         c->cmp.sp[s] = P.sp[s];
-        TRY(dalloc(c, (void**)&c->cmp.cnt[s], sizeof(unsigned) * chunks));
-        TRY(dalloc(c, (void**)&c->cmp.hole[s], sizeof(unsigned) * chunks));
-        TRY(dalloc(c, (void**)&c->cmp.tail[s], sizeof(unsigned) * chunks));
-        TRY(dalloc(c, (void**)&c->cmp.hpos[s], sizeof(unsigned) * (cap / 2 + 1)));
-        TRY(dalloc(c, (void**)&c->cmp.tpos[s], sizeof(unsigned) * (cap / 2 + 1)));
+        const size_t size[5] = {chunks, chunks, chunks, cap / 2 + 1, cap / 2 + 1};
+        unsigned** part[5] = {&c->cmp.cnt[s], &c->cmp.hole[s], &c->cmp.tail[s], &c->cmp.hpos[s], &c->cmp.tpos[s]};
+        size_t words = 0;
+        for (size_t v : size) words += (v + 63) & ~(size_t)63;
+        unsigned* base = nullptr;
+        TRY(dalloc(c, (void**)&base, sizeof(unsigned) * words));
+        for (int q = 0; q < 5; q++) {
+            *part[q] = base;
+            base += (size[q] + 63) & ~(size_t)63;
+        }
         most = std::max(most, chunks);
     }
     TRY(dalloc(c, (void**)&c->cmp.info, sizeof(ull) * 4 * PT_NSPECIES));
     HIPCHK(c, hipMemsetAsync(c->cmp.info, 0, sizeof(ull) * 4 * PT_NSPECIES, c->stream));
     c->cmp.work = c->dwork;
+    c->cmp.report = c->report;
     c->cmp_blocks = (int)std::min<size_t>(most, 512);
-    TRY(dalloc(c, (void**)&c->stat_part, sizeof(double) * NSTAT * 4096));
+    TRY(dalloc(c, (void**)&c->stat_part, sizeof(double) * NSTAT * STAT_BLOCKS + sizeof(ull)));
+    HIPCHK(c, hipMemsetAsync(c->stat_part + NSTAT * STAT_BLOCKS, 0, sizeof(ull), c->stream));
     TRY(dalloc(c, (void**)&c->dp, sizeof(Params)));
     TRY(dalloc(c, (void**)&P.image, IMAGE_BYTES));
     hipDeviceProp_t prop;
@@ -3108,6 +3303,7 @@ int pt_count(pt_ctx* c, int sp, uint64_t* n) {
 static int put_particles(pt_ctx* c, int sp, ull base, const double* const soa[PT_NFIELDS],
                          const uint8_t* active, const uint64_t* uid, const int32_t* swarm, size_t n) {
     SpeciesDev& S = c->hp.sp[sp];
+    if (n == 0) return PT_OK;
     // the host's columns into records (absent fields are zero), one copy
     std::vector<double> rec((size_t)PT_NFIELDS * n, 0.0);
     for (int f = 0; f < PT_NFIELDS; f++)
@@ -3286,8 +3482,9 @@ int pt_init(pt_ctx* c) {
     if (rc) return rc;
     rc = sync_params(c);
     if (rc) return rc;
+    if ((rc = read_counts(c))) return rc;
     for (int s = 0; s < PT_NSPECIES; s++) {
-        if (!c->hp.tab[s].valid) continue;
+        if (!c->hp.tab[s].valid || c->hn[s] == 0) continue;
         hipLaunchKernelGGL(k_setr, dim3(c->grid), dim3(256), c->lds_bytes, c->stream, c->dp, s);
         HIPCHK(c, hipGetLastError());
     }
@@ -3413,9 +3610,25 @@ static int launch_kernel_args(pt_ctx* c, int v, bool full) {
     return PT_OK;
 }
 
+// secondaries the waves' stacks could not take: whole-grid passes, then one workgroup for
+// whatever the last pass created
+static int launch_tail(pt_ctx* c) {
+    int rc;
+    const bool wall = c->hp.wall.on != 0, mlp = mlp_any(c);
+    const int in_place = wall ? KV_RANGE_WALL : with_mlp(KV_RANGE_FULL, mlp);
+    for (int q = 0; q < c->launch.tail_passes; q++)
+        if ((rc = launch_kernel_args(c, in_place, true))) return rc;
+    const size_t tail_lds = (size_t)c->hp.lds_coop_off + (size_t)(512 / 64) * COOP_WAVE_BYTES;
+    if (wall) hipLaunchKernelGGL((k_tail<true, false>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
+    else if (mlp) hipLaunchKernelGGL((k_tail<false, true>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
+    else hipLaunchKernelGGL((k_tail<false, false>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
+    HIPCHK(c, hipGetLastError());
+    return PT_OK;
+}
+
 // one step.  clocked: tfinal and the step index come from the device clock (captured
 // runs); otherwise they are given and the host counts steps.
-static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int nsub) {
+static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int nsub, bool tail = true) {
     c->counts_known = false;
     int rc = ensure_residency(c);
     if (rc) return rc;
@@ -3446,17 +3659,8 @@ static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int ns
         }
         if ((rc = launch_kernel_args(c, with_mlp(KV_QUEUE_FULL, mlp), true))) return rc;
     }
-    // secondaries the lanes' stacks could not take: whole-grid passes, then one workgroup
-    // for whatever the last pass created
-    for (int q = 0; q < c->launch.tail_passes; q++) {
-        if ((rc = launch_kernel_args(c, in_place, true))) return rc;
-    }
     if (prof && (rc = mark(c, &e1))) return rc;
-    const size_t tail_lds = (size_t)c->hp.lds_coop_off + (size_t)(512 / 64) * COOP_WAVE_BYTES;
-    if (wall) hipLaunchKernelGGL((k_tail<true, false>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
-    else if (mlp) hipLaunchKernelGGL((k_tail<false, true>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
-    else hipLaunchKernelGGL((k_tail<false, false>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
-    HIPCHK(c, hipGetLastError());
+    if (tail && (rc = launch_tail(c))) return rc;
     if (prof) {
         if ((rc = mark(c, &e2))) return rc;
         c->spans.push_back(Span{e0, e1, SPAN_ADV});
@@ -3475,10 +3679,9 @@ static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int ns
 // take one step at a time
 static int steps_per_launch(const pt_ctx* c) { return c->launch.rounds > 0 ? 1 : MAX_SUB; }
 
+// the flags that have been reported (read_state, or the end of a pass)
 static int check_flags(pt_ctx* c, int64_t* out) {
-    ull f[NFLAGS];
-    HIPCHK(c, hipMemcpyAsync(f, c->dflags, sizeof(f), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const ull* f = c->report->flags;
     if (out)
         for (int q = 0; q < NFLAGS; q++) out[q] = (int64_t)f[q];
     if (f[FLAG_CAPACITY]) return fail(c, PT_E_CAPACITY, "%llu particles did not fit in their population", f[FLAG_CAPACITY]);
@@ -3492,6 +3695,8 @@ static int check_flags(pt_ctx* c, int64_t* out) {
 int pt_check(pt_ctx* c, int64_t* flags) {
     if (!c) return PT_E_ARG;
     HIPCHK(c, hipSetDevice(c->device));
+    int rc = read_state(c);
+    if (rc) return rc;
     return check_flags(c, flags);
 }
 
@@ -3502,15 +3707,22 @@ int pt_advance(pt_ctx* c, double tfinal) {
     if (rc) return rc;
     rc = sync_params(c);
     if (rc) return rc;
-    rc = launch_step(c, false, tfinal, 0.0, 1);
+    // the main pass reports counts, flags and whether it left secondaries to further passes:
+    // only then are those launched
+    rc = launch_step(c, false, tfinal, 0.0, 1, false);
     if (rc) return rc;
-    rc = read_counts(c);
-    if (rc) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (c->report->left) {
+        if ((rc = launch_tail(c))) return rc;
+        if ((rc = read_state(c))) return rc;
+    } else {
+        take_counts(c);
+    }
     return check_flags(c, nullptr);
 }
 
 // compaction of a species (-1: of all), entirely on the device, so that it can be captured
-static int compact_all(pt_ctx* c, int sp, bool timed) {
+static int compact_all(pt_ctx* c, int sp, bool timed, bool one = false) {
     hipEvent_t a = nullptr, b = nullptr;
     int rc;
     unsigned mask = 0;
@@ -3519,9 +3731,12 @@ static int compact_all(pt_ctx* c, int sp, bool timed) {
     c->counts_known = false;
     if (timed && (rc = mark(c, &a))) return rc;
     if (mask) {
-        const dim3 grid(c->cmp_blocks, PT_NSPECIES);
+        const dim3 grid(one ? 1 : c->cmp_blocks, PT_NSPECIES);
         hipLaunchKernelGGL(k_cmp_count, grid, dim3(256), 0, c->stream, c->cmp, mask);
         HIPCHK(c, hipGetLastError());
+    }
+    if (mask && !one) {
+        const dim3 grid(c->cmp_blocks, PT_NSPECIES);
         hipLaunchKernelGGL(k_cmp_fill, grid, dim3(256), 0, c->stream, c->cmp, mask);
         HIPCHK(c, hipGetLastError());
         hipLaunchKernelGGL(k_cmp_move, grid, dim3(256), 0, c->stream, c->cmp, mask);
@@ -3538,9 +3753,18 @@ int pt_compact(pt_ctx* c, int sp) {
     if (!c) return PT_E_ARG;
     if (sp < -1 || sp >= PT_NSPECIES) return fail(c, PT_E_ARG, "bad species");
     HIPCHK(c, hipSetDevice(c->device));
-    int rc = compact_all(c, sp, c->profile);
-    if (rc) return rc;
-    return read_counts(c);
+    // counts known and small: one launch does it all (k_cmp_count)
+    bool one = c->counts_known;
+    for (int s = 0; s < PT_NSPECIES; s++) one = one && c->hn[s] <= (ull)CMP_SMALL * CH;
+    int rc;
+    if ((rc = read_counts(c))) return rc;
+    if ((rc = compact_all(c, sp, c->profile, one))) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    // (of a species left out the count is as before)
+    for (int s = 0; s < PT_NSPECIES; s++)
+        if (sp >= 0 && s != sp) c->report->n[s] = c->hn[s];
+    take_counts(c);
+    return PT_OK;
 }
 
 // Steps [q, end) of a run from time t, in launches of up to steps_per_launch steps, with a
@@ -3587,7 +3811,7 @@ static int save_state(pt_ctx* c, const ull n[PT_NSPECIES], bool back) {
                     HIPCHK(c, hipFree(*old[q]));
                     *old[q] = nullptr;
                 }
-                if ((rc = dalloc(c, old[q], size[q] * room))) return rc;
+                if ((rc = dalloc_own(c, old[q], size[q] * room))) return rc;
             }
             v.cap[s] = room;
         }
@@ -3629,7 +3853,7 @@ static int run_window(pt_ctx* c, double& t, double dt, int q, int end, int every
     const double t1 = t;
     const uint32_t step1 = c->step;
     if ((rc = run_steps(c, t, dt, q, end, every, late))) return rc;
-    if ((rc = read_counts(c))) return rc;
+    if ((rc = read_state(c))) return rc;
     if (!late) return check_flags(c, nullptr);
     rc = check_flags(c, nullptr);
     if (rc != PT_E_CAPACITY) return rc;
@@ -3637,7 +3861,7 @@ static int run_window(pt_ctx* c, double& t, double dt, int q, int end, int every
     t = t1;
     c->step = step1;
     if ((rc = run_steps(c, t, dt, q, end, every, false))) return rc;
-    if ((rc = read_counts(c))) return rc;
+    if ((rc = read_state(c))) return rc;
     return check_flags(c, nullptr);
 }
 
@@ -3779,6 +4003,7 @@ int pt_run_graph(pt_ctx* c, double t0, double dt, int nsteps, int check_every) {
         since += ce;
         if (since >= check_every && done < nsteps) {
             since = 0;
+            if ((rc = read_state(c))) return rc;
             if ((rc = check_flags(c, nullptr))) {
                 c->step += (uint32_t)done;
                 return rc;
@@ -3787,7 +4012,7 @@ int pt_run_graph(pt_ctx* c, double t0, double dt, int nsteps, int check_every) {
     }
     if (rem > 0 && (rc = replay(c, 1))) return rc;
     c->step += (uint32_t)nsteps;
-    if ((rc = read_counts(c))) return rc;
+    if ((rc = read_state(c))) return rc;
     return check_flags(c, nullptr);
 }
 
@@ -3834,6 +4059,7 @@ int pt_autotune(pt_ctx* c, double t0, double dt, int trial_steps, pt_tune_trial*
         float ms = 0;
         HIPCHK(c, hipEventElapsedTime(&ms, a, b));
         if ((r2 = psteps_now(c, &p1))) return r2;
+        if ((r2 = read_state(c))) return r2;
         if ((r2 = check_flags(c, nullptr))) return r2;
         *rate = ms > 0 ? (double)(p1 - p0) / (ms * 1e-3) : 0.0;
         return PT_OK;
@@ -3913,19 +4139,12 @@ int pt_stats(pt_ctx* c, int sp, pt_pop_stats* out) {
     if (rc) return rc;
     rc = read_counts(c);
     if (rc) return rc;
-    int blocks = (int)std::min<ull>(4096, std::max<ull>(1, (c->hn[sp] + 255) / 256));
-    hipLaunchKernelGGL(k_stats_partial, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, c->stat_part);
+    const int blocks = (int)std::min<ull>(STAT_BLOCKS, std::max<ull>(1, (c->hn[sp] + 511) / 512));
+    hipLaunchKernelGGL(k_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, c->stat_part,
+                       (ull*)(c->stat_part + NSTAT * STAT_BLOCKS));
     HIPCHK(c, hipGetLastError());
-    std::vector<double> part((size_t)blocks * NSTAT);
-    HIPCHK(c, hipMemcpyAsync(part.data(), c->stat_part, sizeof(double) * part.size(), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    double a[NSTAT] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int b = 0; b < blocks; b++)
-        for (int q = 0; q < NSTAT; q++) {
-            double v = part[(size_t)b * NSTAT + q];
-            if (q == 7) a[q] = std::max(a[q], v);
-            else a[q] += v;
-        }
+    const double* a = c->report->stat;
     out->n = c->hn[sp];
     out->nactive = (uint64_t)a[0];
     out->weight = a[1];
@@ -3945,18 +4164,19 @@ int pt_swarm_stats(pt_ctx* c, int sp, int nswarm, double* out) {
     HIPCHK(c, hipSetDevice(c->device));
     int rc = sync_params(c);
     if (rc) return rc;
-    if (c->stat_cap < nswarm) {
-        if ((rc = dalloc(c, (void**)&c->swarm_part, sizeof(double) * 4 * (size_t)c->cfg.nswarm))) return rc;
-        c->stat_cap = c->cfg.nswarm;
+    const size_t bytes = sizeof(double) * 4 * (size_t)c->cfg.nswarm;
+    if (!c->swarm_part) {
+        if ((rc = dalloc(c, (void**)&c->swarm_part, bytes))) return rc;
+        HIPCHK(c, hipMemsetAsync(c->swarm_part, 0, bytes, c->stream));
     }
     rc = read_counts(c);
     if (rc) return rc;
-    HIPCHK(c, hipMemsetAsync(c->swarm_part, 0, sizeof(double) * 4 * (size_t)nswarm, c->stream));
     int blocks = (int)std::min<ull>((ull)c->grid, std::max<ull>(1, (c->hn[sp] + 255) / 256));
-    hipLaunchKernelGGL(k_swarm_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, nswarm, c->swarm_part);
+    hipLaunchKernelGGL(k_swarm_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, nswarm, c->swarm_part,
+                       c->swarm_host, (ull*)(c->stat_part + NSTAT * STAT_BLOCKS));
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(out, c->swarm_part, sizeof(double) * 4 * (size_t)nswarm, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    memcpy(out, c->swarm_host, sizeof(double) * 4 * (size_t)nswarm);
     return PT_OK;
 }
 
@@ -3976,7 +4196,7 @@ int pt_swarm_stats_noalloc(pt_ctx* c, int sp, int nswarm, double* out) {
     hipLaunchKernelGGL(k_zero_doubles, dim3((n4 + 255) / 256), dim3(256), 0, c->stream, c->noalloc, n4);
     HIPCHK(c, hipGetLastError());
     int blocks = (int)std::min<ull>((ull)c->grid, std::max<ull>(1, (c->hn[sp] + 255) / 256));
-    hipLaunchKernelGGL(k_swarm_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, nswarm, c->noalloc);
+    hipLaunchKernelGGL(k_swarm_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, nswarm, c->noalloc, (double*)nullptr, (ull*)nullptr);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(out, c->noalloc, sizeof(double) * (size_t)n4, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -3989,10 +4209,9 @@ int pt_collision_counts(pt_ctx* c, int sp, int64_t* out, int nmax, int reset) {
     HIPCHK(c, hipSetDevice(c->device));
     ull h[NCOUNT];
     HIPCHK(c, hipMemcpyAsync(h, c->dcounts + sp * NCOUNT, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int q = 0; q < std::min(nmax, NCOUNT); q++) out[q] = (int64_t)h[q];
     if (reset) HIPCHK(c, hipMemsetAsync(c->dcounts + sp * NCOUNT, 0, sizeof(h), c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    for (int q = 0; q < std::min(nmax, NCOUNT); q++) out[q] = (int64_t)h[q];
     return PT_OK;
 }
 
@@ -4938,8 +5157,7 @@ static int roulette_split(pt_ctx* c, bool split, int sp, double f, const double*
                                c->step, (ull)c->hn[sp]);
         HIPCHK(c, hipGetLastError());
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if ((rc = read_counts(c))) return rc;
+    if ((rc = read_state(c))) return rc;
     return check_flags(c, nullptr);
 }
 
