@@ -321,7 +321,8 @@ int pt_split_each(pt_ctx* ctx, int species, const double* f, size_t n);
  * (seed, particle uid, step), so launch shape and compaction cadence change only where a
  * particle sits in its population, not its history. */
 typedef struct {
-    int32_t block;          /* threads per workgroup of the advance kernel: 128, 256 or 512 */
+    int32_t block;          /* threads per workgroup of the advance kernel: 128, 256 or 512 (with 256
+                               and 512, large populations run in workgroups of 768) */
     int32_t grid_mult;      /* workgroups launched = resident workgroups x grid_mult (1..16) */
     int32_t compact_every;  /* steps between compactions in pt_run_graph (>= 1) */
     int32_t rounds;         /* collision rounds per step (0..8): the push/select kernels queue

@@ -158,12 +158,17 @@ struct Params {
     uint32_t forcing_off;  // restrictions of the forcing and the pusher (off_em / off_cl / off_push)
     int lds_rate_off[PT_NSPECIES];
     int lds_rb_off[PT_NSPECIES];
+    int lds_proc_off[PT_NSPECIES];
+    int lds_dose_off;     // the depth-dose bins in LDS (when there are any, at most DOSE_LDS)
     int lds_doubles;      // even
     Report* report;       // pinned host memory
     ull* image;           // what a workgroup stages: the Staged block, then lds_doubles doubles
 };
 
 // ------------------------------------------------------------------ LDS state
+// doubles of a swarm's homogeneous fields in LDS: E, and B unless there is none
+__host__ __device__ __forceinline__ int field_doubles(uint32_t off) { return (off & OFF_NO_B) ? 3 : 6; }
+
 // zeros after each species' rate table in LDS: the selection scan reads up to three
 // processes past the last one
 constexpr int SCAN_PAD = 9;
@@ -188,6 +193,7 @@ struct SpLite {
     const double* rb;  // rate bounds in global memory (several swarms)
     int rate_off;      // the rate table in the dynamic LDS (doubles)
     int rb_off;        // the rate bounds there (one swarm)
+    int proc_off;      // the process records there
     double cut, xmax, ixmax, two_k1;  // ixmax = 1 / xmax, two_k1 = 2^(k+1)
     // |p|^2 above which the kinetic energy is certainly above the cut: the cut's |p|^2
     // times 1 + 1e-9, far beyond the rounding of the energy computed from |p|^2
@@ -195,14 +201,14 @@ struct SpLite {
     int tracked, valid, nprocs, k, nswarm, rb_lds;
 };
 
-// block-local counters, flushed once per block (the depth-dose histogram too, when it has
-// at most DOSE_LDS bins: deposits are frequent and would otherwise contend in global memory)
+// block-local counters, flushed once per block (the depth-dose histogram too, in the dynamic
+// LDS, when it has at most DOSE_LDS bins: deposits are frequent and would otherwise contend in
+// global memory)
 constexpr int DOSE_LDS = 512;
 struct BlockCounters {
     ull counts[PT_NSPECIES * NCOUNT];
     ull flags[NFLAGS];
     ull work[NWORK];
-    double dose[DOSE_LDS + 2];
 };
 
 // What every workgroup needs of the parameters, in the form it needs it: built once in global
@@ -212,7 +218,6 @@ struct BlockCounters {
 // about 20 us of a launch.)
 struct __attribute__((aligned(16))) Staged {
     SpLite sp[PT_NSPECIES];
-    DevProc procs[PT_NSPECIES][MAX_PROCS];
     double cut[PT_NSPECIES];  // new particles at or below the cut are not stored
     int stored[PT_NSPECIES];  // species whose new particles are stored (tracked, with a table)
     // the field of swarm 0 (the push of a one-swarm population reads it here: from global
@@ -235,10 +240,12 @@ __global__ void __launch_bounds__(256) k_build_image(const Params* __restrict__ 
     double* const lds = (double*)(&st + 1);
     for (int q = threadIdx.x; q < MATH_DOUBLES; q += blockDim.x) lds[q] = g_math[q];
     if (P.field_lds)
-        for (int q = threadIdx.x; q < 6 * P.nswarm; q += blockDim.x) {
-            const FieldFn& f = (q % 6) < 3 ? P.fields[q / 6].e : P.fields[q / 6].b;
+        for (int q = threadIdx.x, m = field_doubles(P.forcing_off); q < m * P.nswarm; q += blockDim.x) {
+            const FieldFn& f = (q % m) < 3 ? P.fields[q / m].e : P.fields[q / m].b;
             lds[P.lds_field_off + q] = f.v[q % 3];
         }
+    if (P.dose_bins > 0 && P.dose_bins <= DOSE_LDS)
+        for (int q = threadIdx.x; q < P.dose_bins + 2; q += blockDim.x) lds[P.lds_dose_off + q] = 0.0;
     if (threadIdx.x == 0) st.field0 = P.fields[0];
     for (int s = 0; s < PT_NSPECIES; s++) {
         const DevTable& tb = P.tab[s];
@@ -270,13 +277,15 @@ __global__ void __launch_bounds__(256) k_build_image(const Params* __restrict__ 
             L.two_k1 = ldexp(1.0, tb.k + 1);
             L.rate_off = P.lds_rate_off[s];
             L.rb_off = P.lds_rb_off[s];
+            L.proc_off = P.lds_proc_off[s];
             L.rb = tb.ratebound;
             L.rb_lds = P.rb_in_lds;
             st.cut[s] = tb.cut;
             st.stored[s] = S.tracked && tb.valid;
         }
         if (!tb.valid) continue;
-        for (int q = threadIdx.x; q < tb.nprocs; q += blockDim.x) st.procs[s][q] = tb.procs[q];
+        for (int q = threadIdx.x; q < tb.nprocs; q += blockDim.x)
+            ((DevProc*)(lds + P.lds_proc_off[s]))[q] = tb.procs[q];
         int nr = (tb.k + 1) * tb.nprocs * 3;
         double* dst = lds + P.lds_rate_off[s];
         for (int q = threadIdx.x; q < nr + SCAN_PAD; q += blockDim.x) dst[q] = q < nr ? tb.rate[q] : 0.0;
@@ -286,6 +295,11 @@ __global__ void __launch_bounds__(256) k_build_image(const Params* __restrict__ 
             for (int q = threadIdx.x; q < nb; q += blockDim.x) d2[q] = tb.ratebound[q];
         }
     }
+}
+
+// process j of species s
+__device__ __forceinline__ const DevProc& process(const Shared& sh, int s, int j) {
+    return ((const DevProc*)(pt_lds + sh.sp[s].proc_off))[j];
 }
 
 __device__ __forceinline__ void stage(const Params& P, Shared& sh) {
@@ -311,9 +325,8 @@ __device__ __forceinline__ void stage(const Params& P, Shared& sh) {
     }
     if (threadIdx.x < MAX_SUB) sh.tf[threadIdx.x] = P.clock->tf[threadIdx.x];
     if (threadIdx.x == 0) sh.nsub = (int)P.clock->nsub;
-    ull* const z = (ull*)&sh.bc;  // the dose bins (the last member) only where there is a tally
-    const int nz = (int)((P.dose_bins > 0 ? sizeof(BlockCounters) : offsetof(BlockCounters, dose)) / sizeof(ull));
-    for (int q = threadIdx.x; q < nz; q += blockDim.x) z[q] = 0;
+    ull* const z = (ull*)&sh.bc;
+    for (int q = threadIdx.x; q < (int)(sizeof(BlockCounters) / sizeof(ull)); q += blockDim.x) z[q] = 0;
     __syncthreads();
 }
 
@@ -333,38 +346,42 @@ __device__ __forceinline__ double setr(const SpLite& L, double E, int swarm, boo
 // for a null collision, xi then holding the remainder.  Rates are evaluated four at a time,
 // branch-free within a group, and the next group's coefficients are read before a group is
 // tested, so that their LDS reads overlap; a group may run past the row's last process into
-// the next row or the table's padding (SCAN_PAD), whose values are never used.
+// the next row or the table's padding (SCAN_PAD).  A scan that arrives at the row's end there
+// stops as if process `np` had been found.
 __device__ __forceinline__ int select_process(const PT_LDS double* rt, int np, double t1, double t2, double& xi) {
     int sel = -1;
     double c[12];
 #pragma unroll
     for (int u = 0; u < 12; u++) c[u] = rt[u];
     for (int j = 0; j < np; j += 4) {
-        double nu[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) nu[u] = (c[3 * u] * 1.0 + c[3 * u + 1] * t1) + c[3 * u + 2] * t2;
-        const PT_LDS double* nx = rt + 3 * (j + 4 < np ? j + 4 : 0);
-#pragma unroll
-        for (int u = 0; u < 12; u++) c[u] = nx[u];
-        bool found = false;
+        double nu[4], x[5];
+        x[0] = xi;
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            const bool valid = j + u < np;
-            const bool hit = valid && !found && nu[u] > xi;
-            sel = hit ? j + u : sel;
-            found = found || hit;
-            xi = (valid && !found) ? xi - nu[u] : xi;
+            nu[u] = (c[3 * u] * 1.0 + c[3 * u + 1] * t1) + c[3 * u + 2] * t2;
+            x[u + 1] = x[u] - nu[u];
         }
-        if (found) break;
+        const PT_LDS double* nx = rt + (j + 4 < np ? 3 * (j + 4) : 0);
+#pragma unroll
+        for (int u = 0; u < 12; u++) c[u] = nx[u];
+#pragma unroll
+        for (int u = 3; u >= 0; u--) {
+            const bool hit = nu[u] > x[u] || (u > 0 && j + u == np);
+            sel = hit ? j + u : sel;
+            xi = hit ? x[u] : u == 3 ? x[4] : xi;
+        }
+        if (sel >= 0) break;
     }
-    return sel;
+    return sel < np ? sel : -1;
 }
 
 __device__ void flush_counters(const Params& P, BlockCounters* bc) {
     __syncthreads();
     if (P.dose_bins > 0 && P.dose_bins <= DOSE_LDS)
-        for (int q = threadIdx.x; q < P.dose_bins + 2; q += blockDim.x)
-            if (bc->dose[q] != 0.0) atomicAdd(&P.dose[q], bc->dose[q]);
+        for (int q = threadIdx.x; q < P.dose_bins + 2; q += blockDim.x) {
+            const double v = pt_lds[P.lds_dose_off + q];
+            if (v != 0.0) atomicAdd(&P.dose[q], v);
+        }
     for (int q = threadIdx.x; q < PT_NSPECIES * NCOUNT; q += blockDim.x)
         if (bc->counts[q]) atomicAdd(&P.counts[q], bc->counts[q]);
     for (int q = threadIdx.x; q < NFLAGS; q += blockDim.x)
@@ -380,8 +397,9 @@ __device__ __forceinline__ void deposit(const Params& P, BlockCounters& bc, doub
     double f = (z - P.dose_zlo) / (P.dose_zhi - P.dose_zlo);
     int b = f < 0.0 ? P.dose_bins : (f >= 1.0 ? P.dose_bins + 1 : (int)floor(f * P.dose_bins));
     if (b < 0 || b > P.dose_bins + 1) b = P.dose_bins + 1;
-    if (P.dose_bins <= DOSE_LDS) atomicAdd(&bc.dose[b], e);
-    else atomicAdd(&P.dose[b], e);
+    if (P.dose_bins <= DOSE_LDS) __hip_atomic_fetch_add((PT_LDS double*)pt_lds + P.lds_dose_off + b, e, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
+    else __hip_atomic_fetch_add((PT_GLOBAL double*)P.dose + b, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ------------------------------------------------------------------ append
@@ -496,7 +514,7 @@ __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, cons
 // way to memory and back, the launches between steps and the wait for the step's slowest
 // wave.  10^7 electrons, 8 steps a launch: 2.50 -> 2.36 ms a step; 41,000 electrons: 253 ->
 // 168 us; a pencil beam of 2 x 10^6 photons, where the wait is for the electron with the most
-// collisions: 75 -> 26 ms (with the repeated pushes of E).
+// collisions: 75 -> 26 ms (with the repeated pushes of D).
 //
 // Collisions are sampled in the lane.  The secondaries it stores go on a stack in LDS that
 // the wave's free lanes take from before new items; those that find it full are left to the
@@ -548,10 +566,7 @@ __device__ __forceinline__ PT_GLOBAL pair2* rec_pairs(const SpLite& L, ull idx) 
 }
 
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima): every vector memory
-// operation of the wave issued so far has completed.  A refill waits for its loads here,
-// also on the path where the item is skipped and its fields are never read, so that no load
-// into registers the loop reuses is still pending when 3b's loads are in flight (the wait
-// for such a load would be a wait for those too).
+// operation of the wave issued so far has completed
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // one round trip: every column of slot idx is read before any is tested
@@ -737,7 +752,7 @@ __device__ __forceinline__ void learned_pass(const Params& P, const Shared& sh, 
     for (int q = 0; q < MLP_IN; q++) xin[q] = 0.0f;
     if (use) {
         const double u1 = g.next(), u2 = g.next();
-        const DevProc& pr = sh.procs[sp][sel];
+        const DevProc& pr = process(sh, sp, sel);
         const double ph =
             which == LEARN_SB ? sb_phase(P.sb[pr.slot].log_energy, P.sb[pr.slot].thr, P.sb[pr.slot].ne, E) : 0.0;
         mlp_features(E / EV, pr.Z, u1, u2, ph, xin);
@@ -755,12 +770,9 @@ __device__ __forceinline__ void learned_pass(const Params& P, const Shared& sh, 
 // the swarm a particle's statistics go to (out-of-range values count as swarm 0)
 __device__ __forceinline__ int swarm_of(const Params& P, int32_t sw) { return (sw < 0 || sw >= P.nswarm) ? 0 : sw; }
 
-template <int SRC, bool EVENT, bool WALL = false, bool MLP = false>
+template <int SRC, bool EVENT, bool WALL = false, bool MLP = false, bool LEAN = false>
 __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS char* wlds, const ull* rb, const ull* re,
                                             ull* cursor, uint32_t step0, bool main_pass, int par) {
-    // range passes load a retiring lane's next item ahead (D); a lane that retires ends its
-    // last step without a collision, so it neither queues one (EVENT) nor runs a network (MLP)
-    constexpr bool AHEAD = SRC == SRC_RANGE;
     // range passes with every collision in place advance their particles through several
     // steps; the others through one
     constexpr bool MULTI = SRC == SRC_RANGE && !EVENT;
@@ -800,17 +812,17 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
     // lane state
     bool have = false;
     int sp = 0, swarm = 0;
-    ull idx = 0;
+    uint32_t idx = 0;
     V3 x{0, 0, 0}, p{0, 0, 0};
     double w = 0, t = 0, s = 0, r = 0, trem = 0;
-    uint64_t uid = 0;
     StepStream g;
-    g.init(0, 0, 0);
-    uint32_t iters = 0, nev = 0;
+    g.init(P.seed, 0, 0);
+    uint32_t iters = 0;
     uint32_t n_events = 0, n_psteps = 0, n_tail = 0;  // the lane's work counts
     bool active = false, oob = false;
     bool child = false;  // born in the step it is in (counted apart)
     bool born = false;   // born in this launch: marked when it is done
+    bool half = false;   // its next draw is the second half of the block cached in g.c1
     bool pend = false;   // its push ended in a collision, which is still to be selected
     bool new_r = false;  // its rate bound is to be recomputed
     double cE = 0.0;     // kinetic energy at the pending collision
@@ -827,13 +839,24 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
     // the rate bound's coefficients in the interval ci of its energy
     int ci = -1;
     double rc0 = 0, rc1 = 0, rc2 = 0;
+    auto cut_of = [&]() { return LEAN ? sh.sp[sp].cut : cut; };
+    auto grid = [&](double E, double& t1, double& t2, bool& o) {
+        const SpLite& L = sh.sp[sp];
+        return LEAN ? precheb(E, L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o)
+                    : precheb(E, kint, xmax, ixmax, two_k1, t1, t2, o);
+    };
     // setr! of the lane's particle (src/collisions.jl:63-74)
     auto rate_bound = [&](double E) {
-        if (E < cut) return 0.0;
+        if (E < cut_of()) return 0.0;
         double t1, t2;
         bool o;
-        const int i = precheb(E, kint, xmax, ixmax, two_k1, t1, t2, o);
+        const int i = grid(E, t1, t2, o);
         oob |= o;
+        if constexpr (LEAN) {
+            const SpLite& L = sh.sp[sp];
+            if (P.rb_in_lds) return cheb3(as_lds(pt_lds) + L.rb_off + 3 * i, t1, t2);
+            return cheb3(as_global(L.rb) + ((size_t)(P.nswarm > 1 ? swarm : 0) * (L.k + 1) + i) * 3, t1, t2);
+        }
         if (i != ci) {
             ci = i;
             if (P.rb_in_lds) {
@@ -855,6 +878,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
     const double dropcut = sh.cut[PT_ELECTRON] * (1.0 - 1e-9);
     // the particle that has just been given to the lane: its species' and swarm's constants
     auto settle = [&]() {
+        if constexpr (LEAN) return;
         const SpLite& L = sh.sp[sp];
         cut = L.cut;
         pphi = L.ppcut_hi;
@@ -867,18 +891,12 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
         rb_off = L.rb_off;
         ci = -1;
         if (ffree) {
-            const PT_LDS double* e = as_lds(pt_lds) + P.lds_field_off + 6 * swarm;
+            const PT_LDS double* e = as_lds(pt_lds) + P.lds_field_off + field_doubles(P.forcing_off) * swarm;
             const double q = (sp == PT_ELECTRON ? -1.0 : 1.0) * QE;
             const bool none = sp == PT_PHOTON || (foff & off_em(sp));
             F = V3{none ? 0.0 : q * e[0], none ? 0.0 : q * e[1], none ? 0.0 : q * e[2]};
         }
     };
-    // the item loaded ahead for this lane
-    bool ahead = false;
-    int nsp = 0;
-    ull nidx = 0;
-    Loaded na;
-    na.act = 0;
     // an item that was just read becomes the lane's particle if it has a step to do from
     // step k0 on; `ch`: it was born in step k0
     auto take = [&](int qs, ull qi, const Loaded& a, int k0, bool ch, bool bo) {
@@ -892,21 +910,20 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
         }
         if (a.act == 0 || !(cr > EPS64)) return;
         sp = qs;
-        idx = qi;
+        idx = (uint32_t)qi;
         x = a.x;
         p = a.p;
         w = a.w;
         t = a.t;
         s = a.s;
-        uid = a.uid;
         swarm = swarm_of(P, a.swarm);
         trem = cr;
         oob = false;
         new_r = true;
         ks = k;
-        g.init(P.seed, uid, step0 + (uint32_t)k);
+        g.init(P.seed, a.uid, step0 + (uint32_t)k);
+        half = false;
         iters = 0;
-        nev = 0;
         active = true;
         have = true;
         child = ch;
@@ -915,14 +932,12 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
     };
     for (;;) {
         const bool first = !MULTI || extra == 0;
-        // A. the end of a particle's step: droplow!'s cut, then its next step, or back to
-        //    memory.  A lane whose next item is loaded waits for the first push round after
-        //    a collision phase, when its loads have had that phase's time.
-        if (have && !pend && (!(trem > EPS64) || !active) && (first || !ahead)) {
+        // A. the end of a particle's step: droplow!'s cut, then its next step, or back to memory
+        if (have && !pend && (!(trem > EPS64) || !active)) {
             // droplow!: the energy is computed only where |p|^2 does not settle the test
-            if (active && !(dot3(p, p) > pphi)) {
+            if (active && !(dot3(p, p) > (LEAN ? sh.sp[sp].ppcut_hi : pphi))) {
                 double Ek = kinenergy(sp, p);
-                if (Ek < cut) {
+                if (Ek < cut_of()) {
                     active = false;
                     deposit(P, sh.bc, Ek * w, x.z);
                 }
@@ -933,7 +948,6 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                 new_r = false;
             }
             if (oob) atomicAdd(&sh.bc.flags[FLAG_RANGE], 1ull);
-            n_events += nev;
             if (child)
                 n_tail++;
             else
@@ -953,16 +967,12 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
             if (cont) {
                 // the next step's advance_init!: a new rate bound and random stream
                 g.restart(step0 + (uint32_t)ks);
+                half = false;
                 iters = 0;
-                nev = 0;
                 oob = false;
                 child = false;
                 new_r = true;
             } else {
-                // the item loaded ahead: its loads are waited for here, before the stores
-                // below, so that the wait is not a wait for those stores too
-                if (AHEAD && ahead) wait_vmem();
-                __builtin_amdgcn_sched_barrier(0);
                 // the particle's record: 72 contiguous bytes (w unchanged), written in whole
                 // sectors, four of the five stores 16 bytes wide
                 const SpLite& L = sh.sp[sp];
@@ -978,10 +988,6 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                 if (!active) L.active[idx] = 0;
                 if (MULTI && born && K > 1) L.draw[idx] = (uint32_t)K;
                 have = false;
-                if (AHEAD && ahead) {
-                    ahead = false;
-                    take(nsp, nidx, na, 0, !main_pass, false);
-                }
             }
         }
         // B. free lanes take the wave's waiting secondaries, then the next items of its chunk,
@@ -1039,22 +1045,21 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                             const double cr = Lq.trem[qi];
                             const uint32_t d0 = Lq.draw[qi];
                             sp = qs;
-                            idx = qi;
+                            idx = (uint32_t)qi;
                             x = a.x;
                             p = a.p;
                             w = a.w;
                             t = a.t;
                             s = a.s;
-                            uid = a.uid;
                             swarm = swarm_of(P, a.swarm);
                             trem = cr;
                             oob = false;
                             r = PF(Lq.f[PT_R], qi);  // set by the sampler (setr! of apply!) or at birth
                             new_r = false;
-                            g.init(P.seed, uid, step0);
+                            g.init(P.seed, a.uid, step0);
                             g.resume(d0);
+                            half = (d0 & 1) != 0;
                             iters = 0;
-                            nev = 0;
                             active = true;
                             have = true;
                             child = ch;
@@ -1071,7 +1076,6 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                             k0 = (int)sh.sp[qs].draw[qi];
                             bo = true;
                         }
-                        wait_vmem();
                         if (k0 < K) take(qs, qi, a, k0, ch, bo);
                     }
                 }
@@ -1087,51 +1091,8 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
             new_r = false;
         }
         const double tnext = qdiv_any(s, r);
-        // D. a lane whose push reaches the end of its last step without a collision retires at
-        //    the next A: it claims its next item now and loads it while the push, the wave's
-        //    collisions and the other lanes' work run, and takes it when it writes its particle
-        //    back.  Without this the load is issued when the lane is free and used at once, so
-        //    the lane waits for it, and, since memory operations complete in order for that
-        //    wait, also for the stores of the write-back just before.
-        if constexpr (AHEAD) {
-            // (waiting secondaries are taken first; a pass over secondaries of several steps
-            // reads their birth steps in B)
-            const bool ends = first && nstk == 0 && lane < lanes && (main_pass || K == 1) && have && !pend && ks == K - 1 && trem > EPS64 && active &&
-                              !(trem > tnext);
-            bool got = false;
-            uint64_t want = __ballot(ends);
-            while (want && !drained) {
-                if (cbeg >= cend && !claim()) break;
-                const ull q = cbeg + (ull)__popcll(want & ltmask);
-                const ull cnt = (ull)__popcll(want);
-                const bool mine = ends && !got && q < cend;
-                cbeg = cbeg + cnt < cend ? cbeg + cnt : cend;
-                if (mine) {
-                    if (q < n0) {
-                        nsp = 0;
-                        nidx = rb[0] + q;
-                    } else if (q < n0 + n1) {
-                        nsp = 1;
-                        nidx = rb[1] + (q - n0);
-                    } else {
-                        nsp = 2;
-                        nidx = rb[2] + (q - n0 - n1);
-                    }
-                    got = true;
-                }
-                want = __ballot(ends && !got);
-            }
-            // issued after the claim loop and read nowhere before the write-back: values
-            // that a loop carried, or a flag tested here, would make the wave wait for the
-            // loads at once
-            if (got) {
-                na = load_slot(sh.sp[nsp], nidx);
-                ahead = true;
-            }
-        }
-        // E. one push of this lane's particle.  In a further push round a lane whose push would
-        //    end its last step waits, so that it loads its next item ahead.
-        if (have && !pend && trem > EPS64 && active && (first || ks < K - 1 || trem > tnext)) {
+        // D. one push of this lane's particle
+        if (have && !pend && trem > EPS64 && active) {
             if (++iters > ITER_LIMIT || g.exhausted()) {
                 atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
                 trem = 0.0;
@@ -1151,10 +1112,16 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                 V3 dx{0, 0, 0}, dp{0, 0, 0};
                 bool uniform;  // the force does not depend on the position
                 if (ffree) {
+                    if constexpr (LEAN) {
+                        const PT_LDS double* e = as_lds(pt_lds) + P.lds_field_off + field_doubles(P.forcing_off) * swarm;
+                        const double q = (sp == PT_ELECTRON ? -1.0 : 1.0) * QE;
+                        const bool none = sp == PT_PHOTON || (foff & off_em(sp));
+                        F = V3{none || falong ? 0.0 : q * e[0], none || falong ? 0.0 : q * e[1], none ? 0.0 : q * e[2]};
+                    }
                     push_uniform(sp, F, falong, p, dt, dx, dp);
                     uniform = true;
                 } else if (P.field_lds) {
-                    const PT_LDS double* fv = as_lds(pt_lds) + P.lds_field_off + 6 * swarm;
+                    const PT_LDS double* fv = as_lds(pt_lds) + P.lds_field_off + field_doubles(P.forcing_off) * swarm;
                     const HomField hf{{fv}, {fv + 3}, {{nullptr, nullptr}}};
                     push_delta(sp, hf, x, p, dt, foff, dx, dp);
                     uniform = true;
@@ -1172,12 +1139,12 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                     p = V3{p.x + dp.x, p.y + dp.y, p.z + dp.z};
                 }
                 t = t + dt;
-                if constexpr (WALL) wall_check(P, sp, xo, po, to, x, p, w, t, uid, swarm, active);
+                if constexpr (WALL) wall_check(P, sp, xo, po, to, x, p, w, t, g.uid(), swarm, active);
                 trem -= dt;
                 if (coll && r != 0.0 && (!WALL || active)) {
                     const double E = kinenergy(sp, p);
-                    if (E >= cut) {
-                        nev++;
+                    if (E >= cut_of()) {
+                        n_events++;
                         cE = E;
                         pend = true;
                     } else if (MULTI && !WALL && uniform && p.x == po.x && p.y == po.y && p.z == po.z) {
@@ -1196,45 +1163,47 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
             }
         }
         if constexpr (MULTI) {
-            // F. another push round before the collisions: when no lane has one, or when
+            // E. another push round before the collisions: when no lane has one, or when
             //    enough lanes can still reach theirs
             const uint64_t pends = __ballot(pend);
             if (pends == 0) {
                 extra = 0;
                 continue;
             }
-            const bool ready = have && !pend && active && (trem > EPS64 ? ks < K - 1 || trem > tnext : ks < K - 1);
+            const bool ready = have && !pend && active && (trem > EPS64 || ks < K - 1);
             if (extra < MORE_ROUNDS && __popcll(__ballot(ready)) >= MORE_LANES) {
                 extra++;
                 continue;
             }
             extra = 0;
         }
-        // G. the selection; a real collision is finished in I, after the wave's RBEB rejection
-        //    loops (H)
+        // F. the selection; a real collision is finished in H, after the wave's RBEB rejection
+        //    loops (G)
         ull* qc = nullptr;
         uint32_t* qa = nullptr;
         uint32_t qv = 0;
         int qsel = -1;          // collision queued for the sampling kernel
-        int csel = -1;          // collision sampled in I
+        int csel = -1;          // collision sampled in H
         bool rb_wait = false;   // an RBEB collision waiting for the cooperative loop
         double rb_w = -1.0;
         ProcVals cp{0, 0.0, 0.0};  // what the common samplers need of its process
+        g.cblk = half ? (g.draw >> 1) + 1u : 0u;
         if (pend) {
             pend = false;
             double t1, t2;
             bool o;
-            int iv = precheb(cE, kint, xmax, ixmax, two_k1, t1, t2, o);
+            const int iv = grid(cE, t1, t2, o);
             oob |= o;
             double xi = g.next() * r;
-            const int sel = select_process(as_lds(pt_lds) + rate_off + iv * nprocs * 3, nprocs, t1, t2, xi);
+            const int np = LEAN ? sh.sp[sp].nprocs : nprocs, at = LEAN ? sh.sp[sp].rate_off : rate_off;
+            const int sel = select_process(as_lds(pt_lds) + at + iv * np * 3, np, t1, t2, xi);
             if (sel < 0) {
                 if (!(xi >= 0.0)) atomicAdd(&sh.bc.flags[FLAG_RATEBOUND], 1ull);
                 atomicAdd(&sh.bc.counts[sp * NCOUNT], 1ull);
                 new_r = true;  // setr! of the null collision (p unchanged)
                 s = nextcoll(g);
             } else {
-                const DevProc& pr = sh.procs[sp][sel];
+                const DevProc& pr = process(sh, sp, sel);
                 cp.kind = pr.kind;
                 cp.B = pr.B;
                 cp.c0 = pr.c[0];
@@ -1255,7 +1224,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                         J.s.ratio = js.ratio;
                         J.s.iratio = js.iratio;
                         J.first = g.c1;
-                        J.uid = uid;
+                        J.uid = g.uid();
                         J.d0 = g.draw;
                         J.step = g.step;
                         rb_wait = true;
@@ -1263,7 +1232,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                 }
             }
         }
-        // H. every lane of the wave runs the pending RBEB rejection loops
+        // G. every lane of the wave runs the pending RBEB rejection loops
         rbeb_coop(P, wlds, lane, ltmask, rb_wait, rb_w, g);
         // learned samplers: the wave's bremsstrahlung and Moller collisions whose network
         // is in use go through it on the matrix cores, one kind at a time
@@ -1279,7 +1248,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
             for (int which = 0; which < NLEARN; which++)
                 if (__ballot(lnet && lw == which)) learned_pass(P, sh, which, lnet && lw == which, sp, csel, cE, g, ly0, ly1);
         }
-        // I. the sampled collision
+        // H. the sampled collision
         ull sl0 = NO_SLOT, sl1 = NO_SLOT;  // slots of the secondaries it stored
         int cs0 = 0, cs1 = 0;
         // elastic scattering and ionisation are nearly all collisions of electrons: the lanes
@@ -1299,7 +1268,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                 deposit(P, sh.bc, (drop ? cp.B + E2 : cp.B) * w, x.z);
                 if (!drop) {
                     cs1 = PT_ELECTRON;
-                    sl1 = append(P, sh, PT_ELECTRON, x, m1, w, t, s1, uid, g.step, g.draw, 0, swarm, main_pass,
+                    sl1 = append(P, sh, PT_ELECTRON, x, m1, w, t, s1, g.uid(), g.step, g.draw, 0, swarm, main_pass,
                                  (uint32_t)ks);
                 }
             }
@@ -1310,8 +1279,8 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
             const double E = cE;
             const double pn = norm3(p);
             Ev e;
-            if (MLP && lnet) learned_event(sh.procs[sp][csel], sp, E, ly0, ly1, g, e);
-            else sample_event(sh.procs[sp][csel], sp, p, pn, E, P.sb, P.pe, g, e, dropcut);
+            if (MLP && lnet) learned_event(process(sh, sp, csel), sp, E, ly0, ly1, g, e);
+            else sample_event(process(sh, sp, csel), sp, p, pn, E, P.sb, P.pe, g, e, dropcut);
             if (e.err) atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
             if (e.dep != 0.0) deposit(P, sh.bc, e.dep * w, x.z);
             V3 m0, m1;
@@ -1327,14 +1296,18 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
             } else {
                 active = false;
                 cs0 = e.sp0;
-                sl0 = append(P, sh, e.sp0, x, m0, w, t, s0, uid, g.step, dend, 0, swarm, main_pass, (uint32_t)ks);
+                sl0 = append(P, sh, e.sp0, x, m0, w, t, s0, g.uid(), g.step, dend, 0, swarm, main_pass, (uint32_t)ks);
             }
             if (e.ne == 2 && !drop1) {
                 cs1 = e.sp1;
-                sl1 = append(P, sh, e.sp1, x, m1, w, t, s1, uid, g.step, dend, e.keep ? 0 : 1, swarm, main_pass,
+                sl1 = append(P, sh, e.sp1, x, m1, w, t, s1, g.uid(), g.step, dend, e.keep ? 0 : 1, swarm, main_pass,
                              (uint32_t)ks);
             }
         }
+        // what the streams keep between collisions
+        half = (g.draw & 1) && g.cblk == (g.draw >> 1) + 1u;
+        g.c0 = 0.0;
+        g.cblk = 0;
         // the secondaries wait on the wave's stack for its free lanes; those that find it full
         // are left to the passes over the step's secondaries
         if (__ballot(sl0 != NO_SLOT || sl1 != NO_SLOT)) {
@@ -1366,12 +1339,11 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                 L.trem[idx] = trem;
                 L.draw[idx] = g.draw;
                 L.evp[idx] = (uint8_t)qsel;
-                int k = P.q.kq[sp][sh.procs[sp][qsel].kind];
+                int k = P.q.kq[sp][process(sh, sp, qsel).kind];
                 qc = P.q.cnt + QEV(sp, k);
                 qa = P.q.ev[sp][k];
-                qv = (uint32_t)idx | (child ? CHILD_BIT : 0u);
+                qv = idx | (child ? CHILD_BIT : 0u);
                 if (oob) atomicAdd(&sh.bc.flags[FLAG_RANGE], 1ull);
-                n_events += nev;
                 have = false;
             }
             wave_push(qc, qa, qv, lane, ltmask);
@@ -1496,7 +1468,8 @@ __global__ void k_rotate(const Params* __restrict__ Pp) {
 
 // push/select over the step's particles (first round) or the input work queues
 template <int BS, int SRC, bool EVENT, bool WALL = false, bool MLP = false>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_advance(const Params* __restrict__ Pp) {
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS > 512 ? 3 : 2)))
+k_advance(const Params* __restrict__ Pp) {
     __shared__ Shared sh;
     __shared__ int skip;
     const Params& P = *Pp;
@@ -1527,8 +1500,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
     }
     stage(P, sh);
     PT_LDS char* wlds = (PT_LDS char*)pt_lds + P.lds_coop_off + (threadIdx.x >> 6) * COOP_WAVE_BYTES;
-    select_loop<SRC, EVENT, WALL, MLP>(P, sh, wlds, rb, re, &P.clock->cursor, C.step,
-                                       SRC == SRC_RANGE && C.pass == 0, par);
+    select_loop<SRC, EVENT, WALL, MLP, (BS > 512)>(P, sh, wlds, rb, re, &P.clock->cursor, C.step,
+                                                   SRC == SRC_RANGE && C.pass == 0, par);
     flush_counters(P, &sh.bc);
     if constexpr (!EVENT) end_pass(P);
 }
@@ -1616,8 +1589,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) k_
         if (valid) {
             const bool child = (ent & CHILD_BIT) != 0;
             Ev e;
-            if (use_net) learned_event(sh.procs[sp][sel], sp, E, y0, y1, g, e);
-            else sample_event(sh.procs[sp][sel], sp, p, pn, E, P.sb, P.pe, g, e);
+            if (use_net) learned_event(process(sh, sp, sel), sp, E, y0, y1, g, e);
+            else sample_event(process(sh, sp, sel), sp, p, pn, E, P.sb, P.pe, g, e);
             if (e.err) atomicAdd(&sh.bc.flags[FLAG_SAMPLER], 1ull);
             if (e.dep != 0.0) deposit(P, sh.bc, e.dep * w, x.z);
             V3 m0, m1;
@@ -2720,6 +2693,7 @@ struct pt_ctx {
     Clock* dclock = nullptr;
     pt_launch launch{256, 1, 8, 0, 1u << PT_PROC_SB, 2, 0};
     int resident[MAX_KV][3] = {};  // resident workgroups per CU: kernel variant x block 128/256/512
+    int resident_wide = 0;         // and of the wide history pass: 0 where its LDS does not fit
     bool queues = false;      // work and collision queues allocated
     int resident_lds = -1;        // LDS size the residency was computed for
     double* noalloc = nullptr;    // this device's copy of the allocation-free scratch array
@@ -2844,6 +2818,8 @@ static int sync_params(pt_ctx* c) {
         if (c->hp.tab[s].valid) off += (c->hp.tab[s].k + 1) * c->hp.tab[s].nprocs * 3 + SCAN_PAD;
         c->hp.lds_rb_off[s] = off;
         if (c->hp.tab[s].valid && c->hp.rb_in_lds) off += (c->hp.tab[s].k + 1) * 3;
+        c->hp.lds_proc_off[s] = off;
+        if (c->hp.tab[s].valid) off += c->hp.tab[s].nprocs * (int)(sizeof(DevProc) / sizeof(double));
     }
     // several swarms with homogeneous fields: their E and B vectors in LDS (one swarm's
     // field is staged in the static block)
@@ -2866,7 +2842,9 @@ static int sync_params(pt_ctx* c) {
     for (const Field& F : c->hfields) along = along && F.e.v[0] == 0.0 && F.e.v[1] == 0.0;
     c->hp.forcing_off = (c->hp.forcing_off & ~(OFF_NO_B | OFF_E_Z)) | (nob ? OFF_NO_B : 0u) | (along ? OFF_E_Z : 0u);
     c->hp.lds_field_off = off;
-    if (hom) off += 6 * c->cfg.nswarm;
+    if (hom) off += field_doubles(c->hp.forcing_off) * c->cfg.nswarm;
+    c->hp.lds_dose_off = off;  // (zeros in the image)
+    if (c->hp.dose_bins > 0 && c->hp.dose_bins <= DOSE_LDS) off += c->hp.dose_bins + 2;
     off = (off + 1) & ~1;
     c->hp.lds_doubles = off;
     if (sizeof(Staged) + sizeof(double) * (size_t)off > IMAGE_BYTES)
@@ -2925,6 +2903,19 @@ enum {
     // the same push/select kernels with the learned samplers evaluated in place
     KV_RANGE_FULL_MLP = 6, KV_RANGE_EVENT_MLP = 7, KV_QUEUE_EVENT_MLP = 8, KV_QUEUE_FULL_MLP = 9, NKV = 10
 };
+// The history pass of a population that fills the GPU several times over: workgroups of 768
+// threads, three waves per SIMD instead of two (168 registers; a lane then reads its species'
+// constants, its force and its rate bounds from LDS each time).  The pass is bound by
+// instruction issue, and three waves hide more of one another's branches and LDS reads:
+// 24 steps of 10^7 electrons 42.3 -> 35.7 ms, 16 of 1.2 x 10^8 in 256 swarms 330 -> 259.
+// With few electrons per lane the launch is as long as its longest lanes' collisions, and a
+// wave that shares its SIMD with two others takes 1.3 to 1.5 times as long for them: 32 steps
+// of n electrons took (two against three waves, ms) 3.15/3.54 for 3 x 10^5, 4.74/5.61 for
+// 6 x 10^5, 5.77/5.68 for 8 x 10^5, 7.82/7.47 for 1.2 x 10^6 and 11.96/10.68 for 2 x 10^6, so
+// the line lies at four electrons or positrons per lane.  Photons do not count (most only
+// fly): a beam of 2 x 10^6 photons and 10^5 electrons takes 168 against 256 ms.
+constexpr int WIDE = 768;
+constexpr ull WIDE_PER_LANE = 4;
 // the variant of a push/select kernel that evaluates learned samplers in place
 static int with_mlp(int v, bool mlp) { return mlp && v <= KV_QUEUE_FULL ? KV_RANGE_FULL_MLP + v : v; }
 static_assert(NKV <= MAX_KV, "residency table too small for the kernel variants");
@@ -2946,6 +2937,7 @@ static const void* kernel_variant(int v) {
 }
 
 static const void* kernel_of(int v, int bs) {
+    if (bs == WIDE) return (const void*)k_advance<WIDE, SRC_RANGE, false>;
     return bs == 128 ? kernel_variant<128>(v) : bs == 512 ? kernel_variant<512>(v) : kernel_variant<256>(v);
 }
 
@@ -3568,6 +3560,8 @@ static int ensure_residency(pt_ctx* c) {
                                                                    kernel_lds(c, v, bss[bi])));
             c->resident[v][bi] = std::max(nb, 1);
         }
+    HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&c->resident_wide, kernel_of(KV_RANGE_FULL, WIDE), WIDE,
+                                                           kernel_lds(c, KV_RANGE_FULL, WIDE)));
     c->resident_lds = key;
     return PT_OK;
 }
@@ -3595,12 +3589,20 @@ static int ensure_queues(pt_ctx* c) {
     return sync_params(c);
 }
 
+// whether history passes run in wide workgroups: by the electrons and positrons known last,
+// unless the caller asked for small workgroups or the tables leave too little LDS
+static bool wide_now(const pt_ctx* c) {
+    return c->launch.block >= 256 && c->resident_wide > 0 &&
+           c->hn[PT_ELECTRON] + c->hn[PT_POSITRON] >= WIDE_PER_LANE * WIDE * c->ncu;
+}
+
 // full: launch every resident workgroup x grid_mult (captured runs and queue rounds, whose
 // sizes the host does not know); otherwise at most what the last known population needs
 static int launch_kernel_args(pt_ctx* c, int v, bool full) {
     void* args[] = {(void*)&c->dp};
-    const int bs = c->launch.block;
-    ull blocks = (ull)c->resident[v][block_index(bs)] * c->ncu * std::max(1, c->launch.grid_mult);
+    const bool wide = v == KV_RANGE_FULL && wide_now(c);
+    const int bs = wide ? WIDE : c->launch.block;
+    ull blocks = (ull)(wide ? c->resident_wide : c->resident[v][block_index(bs)]) * c->ncu * std::max(1, c->launch.grid_mult);
     if (!full) {
         ull est = c->hn[0] + c->hn[1] + c->hn[2];
         blocks = std::min<ull>(blocks, std::max<ull>((ull)c->ncu, est / (ull)(bs / 64)));
@@ -3943,7 +3945,7 @@ static int capture(pt_ctx* c, int which, int steps, bool compact) {
     if (e != hipSuccess) return fail(c, PT_E_HIP, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
     c->gsteps[which] = steps;
     c->glaunch[which] = c->launch;
-    c->glds[which] = 2 * c->lds_bytes + (mlp_any(c) ? 1 : 0);
+    c->glds[which] = 4 * c->lds_bytes + (mlp_any(c) ? 1 : 0) + (wide_now(c) ? 2 : 0);
     c->ggen[which] = c->params_gen;
     return PT_OK;
 }
@@ -3952,7 +3954,7 @@ static int capture(pt_ctx* c, int which, int steps, bool compact) {
 // layout and no parameter upload since its capture
 static bool graph_current(const pt_ctx* c, int which, int steps) {
     return c->gexec[which] && c->gsteps[which] == steps && same_launch(c->glaunch[which], c->launch) &&
-           c->glds[which] == 2 * c->lds_bytes + (mlp_any(c) ? 1 : 0) && c->ggen[which] == c->params_gen;
+           c->glds[which] == 4 * c->lds_bytes + (mlp_any(c) ? 1 : 0) + (wide_now(c) ? 2 : 0) && c->ggen[which] == c->params_gen;
 }
 
 static int replay(pt_ctx* c, int which) {

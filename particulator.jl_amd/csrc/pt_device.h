@@ -184,6 +184,7 @@ struct PhiloxStream {
         draw = 0;
         cblk = 0;
     }
+    __device__ uint64_t uid() const { return (uint64_t)u1 << 32 | u0; }
     // the same particle's stream of another step
     __device__ __forceinline__ void restart(uint32_t st) {
         step = st;
