@@ -169,9 +169,11 @@ struct Params {
 // doubles of a swarm's homogeneous fields in LDS: E, and B unless there is none
 __host__ __device__ __forceinline__ int field_doubles(uint32_t off) { return (off & OFF_NO_B) ? 3 : 6; }
 
-// zeros after each species' rate table in LDS: the selection scan reads up to three
-// processes past the last one
-constexpr int SCAN_PAD = 9;
+// the selection scan evaluates SCAN_GROUP processes at a time; zeros after each species' rate
+// table in LDS for what it reads past the last one (10^7 electrons, 18 processes: three 34.9 ms,
+// four 35.2, six 35.5; by subtraction, process after process, 35.6)
+constexpr int SCAN_GROUP = 3;
+constexpr int SCAN_PAD = 3 * SCAN_GROUP;
 
 template <typename T>
 using gptr = T PT_GLOBAL*;
@@ -234,23 +236,25 @@ struct Shared : Staged {
 
 constexpr size_t IMAGE_BYTES = 160 * 1024;  // a workgroup's LDS is no larger
 
+constexpr int IMAGE_BLOCKS = 32;  // one workgroup took 28 us, which each of many fields set in a row waits for
 __global__ void __launch_bounds__(256) k_build_image(const Params* __restrict__ Pp) {
     const Params& P = *Pp;
+    const int t0 = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
     Staged& st = *(Staged*)P.image;
     double* const lds = (double*)(&st + 1);
-    for (int q = threadIdx.x; q < MATH_DOUBLES; q += blockDim.x) lds[q] = g_math[q];
+    for (int q = t0; q < MATH_DOUBLES; q += nt) lds[q] = g_math[q];
     if (P.field_lds)
-        for (int q = threadIdx.x, m = field_doubles(P.forcing_off); q < m * P.nswarm; q += blockDim.x) {
+        for (int q = t0, m = field_doubles(P.forcing_off); q < m * P.nswarm; q += nt) {
             const FieldFn& f = (q % m) < 3 ? P.fields[q / m].e : P.fields[q / m].b;
             lds[P.lds_field_off + q] = f.v[q % 3];
         }
     if (P.dose_bins > 0 && P.dose_bins <= DOSE_LDS)
-        for (int q = threadIdx.x; q < P.dose_bins + 2; q += blockDim.x) lds[P.lds_dose_off + q] = 0.0;
-    if (threadIdx.x == 0) st.field0 = P.fields[0];
+        for (int q = t0; q < P.dose_bins + 2; q += nt) lds[P.lds_dose_off + q] = 0.0;
+    if (t0 == 0) st.field0 = P.fields[0];
     for (int s = 0; s < PT_NSPECIES; s++) {
         const DevTable& tb = P.tab[s];
         const SpeciesDev& S = P.sp[s];
-        if (threadIdx.x == 0) {
+        if (threadIdx.x == 0 && blockIdx.x == (s + 1) % gridDim.x) {
             SpLite& L = st.sp[s];
             for (int f = 0; f < PT_NFIELDS; f++) L.f[f] = (gptr<double>)S.f[f];
             L.active = (gptr<uint8_t>)S.active;
@@ -284,15 +288,27 @@ __global__ void __launch_bounds__(256) k_build_image(const Params* __restrict__ 
             st.stored[s] = S.tracked && tb.valid;
         }
         if (!tb.valid) continue;
-        for (int q = threadIdx.x; q < tb.nprocs; q += blockDim.x)
+        for (int q = t0; q < tb.nprocs; q += nt)
             ((DevProc*)(lds + P.lds_proc_off[s]))[q] = tb.procs[q];
         int nr = (tb.k + 1) * tb.nprocs * 3;
         double* dst = lds + P.lds_rate_off[s];
-        for (int q = threadIdx.x; q < nr + SCAN_PAD; q += blockDim.x) dst[q] = q < nr ? tb.rate[q] : 0.0;
+        // the coefficients of the cumulative rates: sums over the row's processes so far, with
+        // the rounding error of each addition carried along
+        for (int q = t0; q < (tb.k + 1) * 3; q += nt) {
+            double sum = 0.0, err = 0.0;
+            for (int j = 0; j < tb.nprocs; j++) {
+                const int at = ((q / 3) * tb.nprocs + j) * 3 + q % 3;
+                const double v = tb.rate[at], n = sum + v, b = n - sum;
+                err += (sum - (n - b)) + (v - b);
+                sum = n;
+                dst[at] = err == err ? sum + err : sum;  // (an infinite sum has no error)
+            }
+        }
+        for (int q = nr + t0; q < nr + SCAN_PAD; q += nt) dst[q] = 0.0;
         if (P.rb_in_lds) {
             int nb = (tb.k + 1) * 3;
             double* d2 = lds + P.lds_rb_off[s];
-            for (int q = threadIdx.x; q < nb; q += blockDim.x) d2[q] = tb.ratebound[q];
+            for (int q = t0; q < nb; q += nt) d2[q] = tb.ratebound[q];
         }
     }
 }
@@ -342,37 +358,39 @@ __device__ __forceinline__ double setr(const SpLite& L, double E, int swarm, boo
 }
 
 // The selection scan of do_one_collision! (src/collisions.jl:160-186): the first process j
-// whose rate exceeds what is left of xi after subtracting the rates of processes 0..j-1; -1
-// for a null collision, xi then holding the remainder.  Rates are evaluated four at a time,
-// branch-free within a group, and the next group's coefficients are read before a group is
-// tested, so that their LDS reads overlap; a group may run past the row's last process into
-// the next row or the table's padding (SCAN_PAD).  A scan that arrives at the row's end there
-// stops as if process `np` had been found.
-__device__ __forceinline__ int select_process(const PT_LDS double* rt, int np, double t1, double t2, double& xi) {
-    int sel = -1;
-    double c[12];
+// whose rate exceeds what is left of xi after subtracting the rates of processes 0..j-1, that
+// is, the first whose cumulative rate exceeds xi; np or more for a null collision.  The row
+// holds the coefficients of the cumulative rates, so a process costs two FMAs, a comparison
+// and a selection, and nothing is carried from one to the next.  A group may run past the
+// row's end into the next row or the table's padding (SCAN_PAD): what it finds there stands
+// for the null collision.
+__device__ __forceinline__ int select_process(const PT_LDS double* rt, int np, double t1, double t2, double xi) {
+    constexpr int G = SCAN_GROUP;
+    int sel = np;
+    double c[3 * G];
 #pragma unroll
-    for (int u = 0; u < 12; u++) c[u] = rt[u];
-    for (int j = 0; j < np; j += 4) {
-        double nu[4], x[5];
-        x[0] = xi;
+    for (int u = 0; u < 3 * G; u++) c[u] = rt[u];
+    for (int j = 0; j < np; j += G) {
+        double cu[G];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            nu[u] = (c[3 * u] * 1.0 + c[3 * u + 1] * t1) + c[3 * u + 2] * t2;
-            x[u + 1] = x[u] - nu[u];
-        }
-        const PT_LDS double* nx = rt + (j + 4 < np ? 3 * (j + 4) : 0);
+        for (int u = 0; u < G; u++) cu[u] = (c[3 * u] + c[3 * u + 1] * t1) + c[3 * u + 2] * t2;
+        const PT_LDS double* nx = rt + (j + G < np ? 3 * (j + G) : 0);
 #pragma unroll
-        for (int u = 0; u < 12; u++) c[u] = nx[u];
+        for (int u = 0; u < 3 * G; u++) c[u] = nx[u];
+        bool any = false;
 #pragma unroll
-        for (int u = 3; u >= 0; u--) {
-            const bool hit = nu[u] > x[u] || (u > 0 && j + u == np);
+        for (int u = G - 1; u >= 0; u--) {
+            const bool hit = cu[u] > xi;
+            any = any || hit;
             sel = hit ? j + u : sel;
-            xi = hit ? x[u] : u == 3 ? x[4] : xi;
         }
-        if (sel >= 0) break;
+        if (any) break;
     }
-    return sel < np ? sel : -1;
+    return sel;
+}
+// whether a null collision's remainder of xi is a number
+__device__ __forceinline__ bool null_remains(const PT_LDS double* rt, int np, double t1, double t2, double xi) {
+    return np == 0 ? xi >= 0.0 : cheb3(rt + 3 * (np - 1), t1, t2) <= xi;
 }
 
 __device__ void flush_counters(const Params& P, BlockCounters* bc) {
@@ -1194,11 +1212,12 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
             bool o;
             const int iv = grid(cE, t1, t2, o);
             oob |= o;
-            double xi = g.next() * r;
+            const double xi = g.next() * r;
             const int np = LEAN ? sh.sp[sp].nprocs : nprocs, at = LEAN ? sh.sp[sp].rate_off : rate_off;
-            const int sel = select_process(as_lds(pt_lds) + at + iv * np * 3, np, t1, t2, xi);
-            if (sel < 0) {
-                if (!(xi >= 0.0)) atomicAdd(&sh.bc.flags[FLAG_RATEBOUND], 1ull);
+            const PT_LDS double* const row = as_lds(pt_lds) + at + iv * np * 3;
+            const int sel = select_process(row, np, t1, t2, xi);
+            if (sel >= np) {
+                if (!null_remains(row, np, t1, t2, xi)) atomicAdd(&sh.bc.flags[FLAG_RATEBOUND], 1ull);
                 atomicAdd(&sh.bc.counts[sp * NCOUNT], 1ull);
                 new_r = true;  // setr! of the null collision (p unchanged)
                 s = nextcoll(g);
@@ -2554,6 +2573,7 @@ __global__ void __launch_bounds__(256) k_dbg_select(const Params* __restrict__ P
     int iv = precheb(E[i], L.k, L.xmax, L.ixmax, L.two_k1, t1, t2, o);
     double xi = u[i] * r;
     int sel = select_process(as_lds(pt_lds) + L.rate_off + iv * L.nprocs * 3, L.nprocs, t1, t2, xi);
+    if (sel >= L.nprocs) sel = -1;
     interval[i] = o ? -1 : iv;
     proc[i] = sel;
     rbound[i] = r;
@@ -2852,7 +2872,7 @@ static int sync_params(pt_ctx* c) {
     c->lds_bytes = off * (int)sizeof(double);
     c->hp.lds_coop_off = (c->lds_bytes + 15) & ~15;
     HIPCHK(c, hipMemcpyAsync(c->dp, &c->hp, sizeof(Params), hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_build_image, dim3(1), dim3(256), 0, c->stream, c->dp);
+    hipLaunchKernelGGL(k_build_image, dim3(IMAGE_BLOCKS), dim3(256), 0, c->stream, c->dp);
     HIPCHK(c, hipGetLastError());
     c->dirty = false;
     // a captured step bakes in host-side choices made from these parameters (the kernel
