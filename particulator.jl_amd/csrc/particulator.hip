@@ -3609,20 +3609,31 @@ static int ensure_queues(pt_ctx* c) {
     return sync_params(c);
 }
 
-// whether history passes run in wide workgroups: by the electrons and positrons known last,
-// unless the caller asked for small workgroups or the tables leave too little LDS
-static bool wide_now(const pt_ctx* c) {
-    return c->launch.block >= 256 && c->resident_wide > 0 &&
-           c->hn[PT_ELECTRON] + c->hn[PT_POSITRON] >= WIDE_PER_LANE * WIDE * c->ncu;
+// The shape of a history pass, by the numbers known last.
+// SHAPE_WIDE: by electrons and positrons (see WIDE), unless the caller asked for small
+// workgroups or the tables leave too little LDS.
+// SHAPE_LONE: one wave per SIMD where that gives a lane at most one particle.  Such a launch
+// is as long as its longest lane's chain of collisions, and a wave that shares its SIMD goes
+// through that more slowly: 32 steps of n electrons took (two waves against one, ms)
+// 1.78/1.62 for 2 x 10^4 and 1.90/1.78 for 6 x 10^4, one step a launch 1.20/1.00; 8 x 10^4
+// electrons, with a second round for some lanes, 1.96/2.07.  Not in captured runs (`full`),
+// which may grow without the host knowing.
+enum { SHAPE_FULL = 0, SHAPE_WIDE = 1, SHAPE_LONE = 2 };
+static int pass_shape(const pt_ctx* c, bool full) {
+    const ull electrons = c->hn[PT_ELECTRON] + c->hn[PT_POSITRON];
+    if (c->launch.block >= 256 && c->resident_wide > 0 && electrons >= WIDE_PER_LANE * WIDE * c->ncu) return SHAPE_WIDE;
+    return !full && c->launch.grid_mult == 1 && electrons + c->hn[PT_PHOTON] <= 256ull * c->ncu ? SHAPE_LONE : SHAPE_FULL;
 }
 
 // full: launch every resident workgroup x grid_mult (captured runs and queue rounds, whose
 // sizes the host does not know); otherwise at most what the last known population needs
 static int launch_kernel_args(pt_ctx* c, int v, bool full) {
     void* args[] = {(void*)&c->dp};
-    const bool wide = v == KV_RANGE_FULL && wide_now(c);
-    const int bs = wide ? WIDE : c->launch.block;
-    ull blocks = (ull)(wide ? c->resident_wide : c->resident[v][block_index(bs)]) * c->ncu * std::max(1, c->launch.grid_mult);
+    const int shape = v == KV_RANGE_FULL ? pass_shape(c, full) : SHAPE_FULL;
+    const int bs = shape == SHAPE_WIDE ? WIDE : c->launch.block;
+    const int per_cu = shape == SHAPE_WIDE ? c->resident_wide : c->resident[v][block_index(bs)];
+    ull blocks = (ull)per_cu * c->ncu * std::max(1, c->launch.grid_mult);
+    if (shape == SHAPE_LONE) blocks = std::min<ull>(blocks, (ull)c->ncu * std::max(1, 256 / bs));
     if (!full) {
         ull est = c->hn[0] + c->hn[1] + c->hn[2];
         blocks = std::min<ull>(blocks, std::max<ull>((ull)c->ncu, est / (ull)(bs / 64)));
@@ -3965,7 +3976,7 @@ static int capture(pt_ctx* c, int which, int steps, bool compact) {
     if (e != hipSuccess) return fail(c, PT_E_HIP, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
     c->gsteps[which] = steps;
     c->glaunch[which] = c->launch;
-    c->glds[which] = 4 * c->lds_bytes + (mlp_any(c) ? 1 : 0) + (wide_now(c) ? 2 : 0);
+    c->glds[which] = 4 * c->lds_bytes + (mlp_any(c) ? 1 : 0) + 2 * pass_shape(c, true);
     c->ggen[which] = c->params_gen;
     return PT_OK;
 }
@@ -3974,7 +3985,8 @@ static int capture(pt_ctx* c, int which, int steps, bool compact) {
 // layout and no parameter upload since its capture
 static bool graph_current(const pt_ctx* c, int which, int steps) {
     return c->gexec[which] && c->gsteps[which] == steps && same_launch(c->glaunch[which], c->launch) &&
-           c->glds[which] == 4 * c->lds_bytes + (mlp_any(c) ? 1 : 0) + (wide_now(c) ? 2 : 0) && c->ggen[which] == c->params_gen;
+           c->glds[which] == 4 * c->lds_bytes + (mlp_any(c) ? 1 : 0) + 2 * pass_shape(c, true) &&
+           c->ggen[which] == c->params_gen;
 }
 
 static int replay(pt_ctx* c, int which) {
@@ -4027,6 +4039,11 @@ int pt_run_graph(pt_ctx* c, double t0, double dt, int nsteps, int check_every) {
             since = 0;
             if ((rc = read_state(c))) return rc;
             if ((rc = check_flags(c, nullptr))) {
+                c->step += (uint32_t)done;
+                return rc;
+            }
+            // (the population may have come to need the other shape)
+            if (k + 1 < full && !graph_current(c, 0, ce) && (rc = capture(c, 0, ce, true))) {
                 c->step += (uint32_t)done;
                 return rc;
             }

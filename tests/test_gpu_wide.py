@@ -91,3 +91,20 @@ def test_wide_workgroups_equal_small_ones(form, n, steps, mode):
     # the bins are sums of at most a few 10^5 positive terms in any order (n eps/2 each way)
     assert np.allclose(a["dose"][0], b["dose"][0], rtol=1e-10, atol=0.0)
     assert np.allclose(a["dose"][1:], b["dose"][1:], rtol=1e-9, atol=0.0)
+
+
+@pytest.mark.parametrize("n", [256 * 256 - 1, 256 * 256, 256 * 256 + 1])
+@pytest.mark.parametrize("block", [128, 256, 512])
+def test_one_wave_per_simd_equals_the_full_launch(n, block):
+    """Particles of all species up to one per lane of a single wave per SIMD (65,536): the
+    launches of pt_run against those of a captured run, which always fill the GPU."""
+    m = n - n // 17  # (run() adds n // 16 photons)
+    a = run("uniform", m, 6, "run", block)
+    b = run("uniform", m, 6, "graph", block)
+    assert a["work"] == b["work"] and a["work"][1] > 0
+    for sp in range(3):
+        assert np.array_equal(a["counts"][sp], b["counts"][sp])
+        x, y = a["pop"][sp], b["pop"][sp]
+        assert np.array_equal(x["uid"], y["uid"])
+        for f in ("x", "p", "w", "t", "s", "r", "swarm"):
+            assert np.array_equal(x[f], y[f]), (sp, f)
