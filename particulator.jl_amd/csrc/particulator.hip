@@ -541,8 +541,11 @@ __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, cons
 //
 // Lanes reach their next collision at different times: of a wave's 64, about 40 end a push in
 // a collision and 24 at the end of a step.  When enough lanes could still reach theirs, they
-// push once more before the wave goes through the collision code (MORE_LANES; 10^7 electrons:
-// 2.39 -> 2.33 ms a step with 12 to 20 lanes, 2.45 with 28).
+// push once more before the wave goes through the collision code: in wide workgroups (WIDE),
+// 10^7 electrons 36.6 -> 35.0 ms with 12 to 20 lanes, 37.4 with 28.  Smaller populations do
+// without: they are as long as their longest chain of collisions, and asking alone costs it
+// 2 to 4% (a beam of 2 x 10^6 photons 153 -> 147 ms, 10^4 electrons 9.4 -> 9.1; 3.2 x 10^5
+// electrons, the other way, 19.6 -> 19.9).
 // EVENT = true (collision rounds): a selected real collision of a sampler kind in
 // P.defer_mask is not sampled here; the particle is written back with its time left and
 // stream position and queued for that sampler kind (wave-aggregated appends), and the
@@ -794,6 +797,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
     // range passes with every collision in place advance their particles through several
     // steps; the others through one
     constexpr bool MULTI = SRC == SRC_RANGE && !EVENT;
+    constexpr bool MORE = MULTI && LEAN;
     const int K = MULTI ? sh.nsub : 1;
     const ull n0 = re[0] - rb[0], n1 = re[1] - rb[1], n2 = re[2] - rb[2];
     const ull total = n0 + n1 + n2;
@@ -949,7 +953,7 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
         settle();
     };
     for (;;) {
-        const bool first = !MULTI || extra == 0;
+        const bool first = !MORE || extra == 0;
         // A. the end of a particle's step: droplow!'s cut, then its next step, or back to memory
         if (have && !pend && (!(trem > EPS64) || !active)) {
             // droplow!: the energy is computed only where |p|^2 does not settle the test
@@ -1183,11 +1187,12 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
         if constexpr (MULTI) {
             // E. another push round before the collisions: when no lane has one, or when
             //    enough lanes can still reach theirs
-            const uint64_t pends = __ballot(pend);
-            if (pends == 0) {
+            if (__ballot(pend) == 0) {
                 extra = 0;
                 continue;
             }
+        }
+        if constexpr (MORE) {
             const bool ready = have && !pend && active && (trem > EPS64 || ks < K - 1);
             if (extra < MORE_ROUNDS && __popcll(__ballot(ready)) >= MORE_LANES) {
                 extra++;
@@ -3616,13 +3621,21 @@ static int ensure_queues(pt_ctx* c) {
 // is as long as its longest lane's chain of collisions, and a wave that shares its SIMD goes
 // through that more slowly: 32 steps of n electrons took (two waves against one, ms)
 // 1.78/1.62 for 2 x 10^4 and 1.90/1.78 for 6 x 10^4, one step a launch 1.20/1.00; 8 x 10^4
-// electrons, with a second round for some lanes, 1.96/2.07.  Not in captured runs (`full`),
+// electrons, with a second round for some lanes, 1.96/2.07.  Photons with few electrons are
+// such a case too, as most photons only fly and what takes long are the chains of the
+// electrons that a few set free: 10 steps of a beam of n photons took 154/141 for 5 x 10^5,
+// 187/152 for 2 x 10^6, 175/162 for 4 x 10^6 and (7 steps) 99/88 for 8 x 10^6; with 1.5
+// photons per lane, where their electrons crowd in half as many waves, 106/121, and with
+// 1500 per lane (10^8), where flying counts, 114/164 (3 steps).  Not in captured runs (`full`),
 // which may grow without the host knowing.
 enum { SHAPE_FULL = 0, SHAPE_WIDE = 1, SHAPE_LONE = 2 };
 static int pass_shape(const pt_ctx* c, bool full) {
     const ull electrons = c->hn[PT_ELECTRON] + c->hn[PT_POSITRON];
     if (c->launch.block >= 256 && c->resident_wide > 0 && electrons >= WIDE_PER_LANE * WIDE * c->ncu) return SHAPE_WIDE;
-    return !full && c->launch.grid_mult == 1 && electrons + c->hn[PT_PHOTON] <= 256ull * c->ncu ? SHAPE_LONE : SHAPE_FULL;
+    if (full || c->launch.grid_mult != 1) return SHAPE_FULL;
+    const ull lanes = 256ull * c->ncu, photons = c->hn[PT_PHOTON];
+    const bool beam = photons >= 4 * lanes && photons <= 128 * lanes && electrons <= std::min(photons / 8, 4 * lanes);
+    return beam || electrons + photons <= lanes ? SHAPE_LONE : SHAPE_FULL;
 }
 
 // full: launch every resident workgroup x grid_mult (captured runs and queue rounds, whose

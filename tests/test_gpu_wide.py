@@ -108,3 +108,27 @@ def test_one_wave_per_simd_equals_the_full_launch(n, block):
         assert np.array_equal(x["uid"], y["uid"])
         for f in ("x", "p", "w", "t", "s", "r", "swarm"):
             assert np.array_equal(x[f], y[f]), (sp, f)
+
+
+@pytest.mark.parametrize("photons", [4 * 65536 - 1, 4 * 65536, 300_001])
+def test_a_beam_on_one_wave_per_simd_equals_the_full_launch(photons):
+    """Photons with few electrons run on one wave per SIMD from four per lane on; a launch of
+    two workgroups per resident one (grid_mult 2) never does."""
+    out = []
+    for mult in (1, 2):
+        te, tg, tp = H.tables()
+        mp = H.make_device(te, tg, tp, 3, caps=(1 << 17, 1 << 19, 1 << 15))
+        soa, uid, _ = H.soa_of(O.init_swarm(photons, 1, 7, e1=2e4, e2=5e6, loguniform=True))
+        mp.add_soa(1, soa, uid=uid, swarm=np.zeros(photons, np.int32))
+        mp.init()
+        mp.set_launch(**dict(mp.get_launch(), grid_mult=mult))
+        mp.run_steps(0.0, 2e-11, 6, compact_every=3, check_every=6)
+        out.append([H.by_uid(mp.download(sp)) for sp in range(3)] + [mp.collision_counts(sp) for sp in range(3)])
+        mp.close()
+    a, b = out
+    assert a[0].size > 0 and a[1].size < photons
+    for sp in range(3):
+        assert np.array_equal(a[3 + sp], b[3 + sp])
+        assert np.array_equal(a[sp]["uid"], b[sp]["uid"])
+        for f in ("x", "p", "w", "t", "s", "r", "swarm"):
+            assert np.array_equal(a[sp][f], b[sp][f]), (sp, f)
