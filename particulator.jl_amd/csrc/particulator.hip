@@ -2442,14 +2442,19 @@ __global__ void __launch_bounds__(256) k_stats(const Params* __restrict__ Pp, in
 // they belong to one swarm (they mostly do: swarms are laid out one after the other), then
 // once into LDS (up to SWARM_LDS swarms; beyond that into global memory directly), and the
 // workgroup adds what it found to the output.  (With an LDS atomic per particle the 64 lanes of
-// a wave met on one address four times over: 2 x 10^6 particles 89 us, now 31.)
+// a wave met on one address four times over.)
 // out[4*i + 3] holds max E as the bit pattern of a non-negative double (ordered like the value).
 constexpr int SWARM_LDS = 1024;
 // With `host` (pinned memory) the last workgroup copies the sums there and clears `out` for the
-// next call.
+// next call; the workgroups then add into `copies` arrays by turns, since atomics on one
+// address, from eight XCDs, are done one after the other.  A call for 2 x 10^6 particles in 64
+// swarms took 109 us with 2048 workgroups on one array, 77 with 512, 48 with 512 on 8 arrays
+// (reading the records once takes 33 us); fewer than 128 workgroups use one array.
+constexpr int SWARM_COPIES = 8;
 __global__ void __launch_bounds__(256) k_swarm_stats(const Params* __restrict__ Pp, int sp, int nswarm,
-                                                     double* __restrict__ out, double* __restrict__ host,
-                                                     ull* __restrict__ ticket) {
+                                                     double* __restrict__ sums, int copies,
+                                                     double* __restrict__ host, ull* __restrict__ ticket) {
+    double* const out = sums + (size_t)(blockIdx.x % copies) * 4 * nswarm;
     __shared__ bool last;
     __shared__ double acc[3 * SWARM_LDS];
     __shared__ ull emax[SWARM_LDS];
@@ -2528,8 +2533,16 @@ __global__ void __launch_bounds__(256) k_swarm_stats(const Params* __restrict__ 
     __syncthreads();
     if (!last) return;
     for (int q = threadIdx.x; q < 4 * nswarm; q += blockDim.x) {
-        to_host(&host[q], agent_load(&out[q]));
-        agent_store(&out[q], 0.0);
+        double u[SWARM_COPIES];
+#pragma unroll
+        for (int k = 0; k < SWARM_COPIES; k++) u[k] = k < copies ? agent_load(&sums[(size_t)k * 4 * nswarm + q]) : 0.0;
+        double v = 0.0;
+#pragma unroll
+        for (int k = 0; k < SWARM_COPIES; k++) {
+            v = (q & 3) == 3 ? fmax(v, u[k]) : v + u[k];
+            if (k < copies) agent_store(&sums[(size_t)k * 4 * nswarm + q], 0.0);
+        }
+        to_host(&host[q], v);
     }
     if (threadIdx.x == 0) *ticket = 0;
 }
@@ -4217,14 +4230,16 @@ int pt_swarm_stats(pt_ctx* c, int sp, int nswarm, double* out) {
     int rc = sync_params(c);
     if (rc) return rc;
     const size_t bytes = sizeof(double) * 4 * (size_t)c->cfg.nswarm;
+    const int most = c->cfg.nswarm <= SWARM_LDS ? SWARM_COPIES : 1;
     if (!c->swarm_part) {
-        if ((rc = dalloc(c, (void**)&c->swarm_part, bytes))) return rc;
-        HIPCHK(c, hipMemsetAsync(c->swarm_part, 0, bytes, c->stream));
+        if ((rc = dalloc(c, (void**)&c->swarm_part, most * bytes))) return rc;
+        HIPCHK(c, hipMemsetAsync(c->swarm_part, 0, most * bytes, c->stream));
     }
     rc = read_counts(c);
     if (rc) return rc;
-    int blocks = (int)std::min<ull>((ull)c->grid, std::max<ull>(1, (c->hn[sp] + 255) / 256));
-    hipLaunchKernelGGL(k_swarm_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, nswarm, c->swarm_part,
+    int blocks = (int)std::min<ull>(2 * c->ncu, std::max<ull>(1, (c->hn[sp] + 255) / 256));
+    const int copies = blocks >= 16 * most ? most : 1;
+    hipLaunchKernelGGL(k_swarm_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, nswarm, c->swarm_part, copies,
                        c->swarm_host, (ull*)(c->stat_part + NSTAT * STAT_BLOCKS));
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -4247,8 +4262,9 @@ int pt_swarm_stats_noalloc(pt_ctx* c, int sp, int nswarm, double* out) {
     const int n4 = 4 * nswarm;
     hipLaunchKernelGGL(k_zero_doubles, dim3((n4 + 255) / 256), dim3(256), 0, c->stream, c->noalloc, n4);
     HIPCHK(c, hipGetLastError());
-    int blocks = (int)std::min<ull>((ull)c->grid, std::max<ull>(1, (c->hn[sp] + 255) / 256));
-    hipLaunchKernelGGL(k_swarm_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, nswarm, c->noalloc, (double*)nullptr, (ull*)nullptr);
+    int blocks = (int)std::min<ull>(2 * c->ncu, std::max<ull>(1, (c->hn[sp] + 255) / 256));
+    hipLaunchKernelGGL(k_swarm_stats, dim3(blocks), dim3(256), 0, c->stream, c->dp, sp, nswarm, c->noalloc, 1,
+                       (double*)nullptr, (ull*)nullptr);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(out, c->noalloc, sizeof(double) * (size_t)n4, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
