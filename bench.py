@@ -12,8 +12,9 @@ Metric: particle-steps/s = sum over timed steps of the active particles at step 
 divided by the wall time of the timed loop (inputs resident in HBM, tables uploaded).
 
 Prints one JSON line.  `roofline` prices the main advance kernel with the algorithmic HBM
-bytes of its launches (165 B per particle-step + 93 B per appended secondary) over its
-average launch duration measured with HIP events on the library's stream.  `cpu_baseline`
+bytes of its launches (165 B per particle-step + 93 B per appended secondary; a launch takes
+its particles through several steps and moves their state once) over its average launch
+duration measured with HIP events on the library's stream.  `cpu_baseline`
 times the CPU restatement of the reference step (oracle/, OpenMP over the host cores) on a
 bounded sample of the same workload.
 """
@@ -236,6 +237,7 @@ def main():
                      "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic["bytes"] if traffic else None,
                      "kernel": "k_advance (in-place collisions)", "avg_launch_ms": adv_avg_ms,
                      "algorithmic_bytes_per_launch": adv_bytes,
+                     "steps_per_launch": args.steps / max(w.advance_launches, 1),
                      "traffic_source": traffic},
     }
     mp.close()
@@ -285,7 +287,7 @@ def pmc_pass(args, counters):
     exe = shutil.which("rocprofv3") or "/opt/rocm/bin/rocprofv3"
     d = tempfile.mkdtemp(prefix="pt_pmc_", dir="/tmp")
     cmd = [exe, "--pmc"] + list(counters) + ["-d", d, "-o", "p", "--", sys.executable, os.path.abspath(__file__),
-                                             "--workload", args.workload, "--steps", "3", "--warmup", "1",
+                                             "--workload", args.workload, "--steps", "16", "--warmup", "8",
                                              "--no-learned", "--no-cpu-baseline", "--no-traffic", "--no-horizon",
                                              "--no-sweep"]
     cmd += ["--n", str(args.n)] if args.n else []
@@ -323,9 +325,11 @@ def pmc_traffic(args):
     out = {"bytes": fetch + write, "fetch_bytes": fetch, "write_bytes": write,
            "fetch_kib_raw": kib["FETCH_SIZE"][0], "write_kib_raw": kib["WRITE_SIZE"][0],
            "dispatches": kib["FETCH_SIZE"][1], "scale": {"FETCH_SIZE": FETCH_SCALE, "WRITE_SIZE": WRITE_SCALE},
-           "note": "counter passes of a 3-step run of the same workload"}
+           "note": "counter passes of a run of 24 steps of the same workload, several to a launch"}
     try:
-        v = {k: x[0] for k, x in pmc_pass(args, VALU_COUNTERS).items()}
+        v = pmc_pass(args, VALU_COUNTERS)
+        steps_per_launch = 24.0 / v["SQ_INSTS_VALU"][1]
+        v = {k: x[0] for k, x in v.items()}
         n0 = args.n or WORKLOADS[args.workload]["n"]
         import torch
         simds = 4 * torch.cuda.get_device_properties(0).multi_processor_count
@@ -334,12 +338,12 @@ def pmc_traffic(args):
         # that many times the pass's length
         waves_per_simd = v["SQ_WAVES"] / simds
         out["valu"] = {"wave_instructions_per_launch": v["SQ_INSTS_VALU"],
-                       "wave_instructions_per_particle_step": v["SQ_INSTS_VALU"] / n0,
+                       "wave_instructions_per_particle_step": v["SQ_INSTS_VALU"] / (n0 * steps_per_launch),
                        "lane_utilisation": v["SQ_THREAD_CYCLES_VALU"] / (64.0 * v["SQ_ACTIVE_INST_VALU"]),
                        "wait_fraction": v["SQ_WAIT_ANY"] / v["SQ_WAVE_CYCLES"],
                        "waves_per_simd": waves_per_simd,
                        "simd_valu_busy": v["SQ_ACTIVE_INST_VALU"] * waves_per_simd / v["SQ_WAVE_CYCLES"],
-                       "note": "the main passes of the same 3-step run: SQ_THREAD_CYCLES_VALU / "
+                       "note": "the main passes of the same 24-step run: SQ_THREAD_CYCLES_VALU / "
                                "(64 SQ_ACTIVE_INST_VALU), SQ_WAIT_ANY / SQ_WAVE_CYCLES; simd_valu_busy = "
                                "share of each SIMD's time its vector unit issues = SQ_ACTIVE_INST_VALU x "
                                "waves per SIMD / SQ_WAVE_CYCLES"}

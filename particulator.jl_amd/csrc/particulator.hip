@@ -6,14 +6,17 @@
 // arrays: every wave reads 64 consecutive doubles per field, fully coalesced).  A device
 // counter n holds the slots in use; secondaries are appended at n with an atomic claim.
 //
-// One step (pt_advance):
-//   k_snapshot   -- pass range [0, n) of every species (the advance_init!/iup state)
-//   k_advance    -- one thread per particle, grid-stride over all three species: ratebound,
+// One step (pt_advance), or up to MAX_SUB steps of a run in one launch:
+//   k_snapshot   -- pass range [0, n) of every species (the advance_init!/iup state) and the
+//                   final times of the launch's steps
+//   k_advance    -- lanes take particles of all three species one after another: ratebound,
 //                   then the reference's `while trem > eps` loop of push / null-collision
-//                   selection / sampling, appending secondaries; finally droplow!'s
-//                   energy cut.  Rate tables live in LDS.
-//   k_tail       -- one workgroup advances the secondaries created in this step (the
-//                   reference's further advance1! passes) until no new particle appears.
+//                   selection / sampling, appending secondaries, which the wave's free lanes
+//                   take up at once; droplow!'s energy cut at the end of each step.  Rate
+//                   tables live in LDS.
+//   k_advance again and k_tail -- only when secondaries found no room: whole-grid passes over
+//                   them, then one workgroup until no new particle appears (the reference's
+//                   further advance1! passes).
 // Compaction (pt_compact) fills holes below the active count with active particles from
 // above it (repack!), found by wave-ballot prefix sums over the active flags.
 #include <hip/hip_runtime.h>
@@ -2144,11 +2147,12 @@ __global__ void __launch_bounds__(256) k_split(const Params* __restrict__ Pp, in
 // of each chunk and, in the last workgroup of a species, the prefix sums; list the k-th hole
 // below the active count and the k-th active above it; move.  Counts are read on the device,
 // so that the launches can be captured; a workgroup without a chunk in use ends at once.
-// (One launch per kernel and species, with a grid over the whole capacity: 52 us for three
-// nearly empty species of 2^27 slots, now 11.)
+// (One launch per kernel and species, with a grid over the whole capacity, and a copy of the
+// counts: a call took 118 us for three species of 2^27 slots, whatever they held; now 17 us up
+// to 16384 slots, 22 for 10^6.)
 constexpr int CH = 4096;  // slots per chunk: one 16-byte read of flags per thread of a workgroup
-// chunks that one workgroup compacts alone, in one launch (16384 slots: 14 us, with three
-// launches 17; with twice as many the one workgroup takes longer)
+// chunks that one workgroup compacts alone, in one launch (16384 slots: a call 17 us, with
+// three launches 20; one launch of 10^3 slots 6.4 us of GPU time, three 13)
 constexpr int CMP_SMALL = 4;
 struct Compaction {
     SpeciesDev sp[PT_NSPECIES];
@@ -2354,8 +2358,8 @@ __global__ void __launch_bounds__(256) k_copy_ranges(const Copies c) {
 // sums over active particles: count, w, w*E, w*x, w*y, w*z, w*|x|^2, and max E; each workgroup
 // leaves its part and the last one adds them up and reports them.  Bound by memory (a record's
 // first 64 bytes: the whole line): every lane reads its particle with 16-byte loads, two
-// particles at a time.  2 x 10^6 particles: 49 -> 33 us (with the host's sum of the parts, which
-// this saves, 85 -> 40).
+// particles at a time.  2 x 10^6 particles: 38 us (160 MB in whole lines take 33 at the rate of a
+// copy); a call 79 -> 48 us without the host's sum of the parts, of 10^4 particles 44 -> 17.
 __device__ __forceinline__ double agent_load(const double* p) {
     return __longlong_as_double(
         (long long)__hip_atomic_load((const ull*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
@@ -3598,8 +3602,14 @@ static int ensure_residency(pt_ctx* c) {
                                                                    kernel_lds(c, v, bss[bi])));
             c->resident[v][bi] = std::max(nb, 1);
         }
-    HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&c->resident_wide, kernel_of(KV_RANGE_FULL, WIDE), WIDE,
-                                                           kernel_lds(c, KV_RANGE_FULL, WIDE)));
+    // (tables that leave no room for it are no error)
+    c->resident_wide = 0;
+    if (kernel_lds(c, KV_RANGE_FULL, WIDE) + sizeof(Shared) <= IMAGE_BYTES &&
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&c->resident_wide, kernel_of(KV_RANGE_FULL, WIDE), WIDE,
+                                                     kernel_lds(c, KV_RANGE_FULL, WIDE)) != hipSuccess) {
+        (void)hipGetLastError();
+        c->resident_wide = 0;
+    }
     c->resident_lds = key;
     return PT_OK;
 }
@@ -3900,7 +3910,7 @@ static int save_state(pt_ctx* c, const ull n[PT_NSPECIES], bool back) {
 // therefore copied aside first (a few us for the populations that gain by it, up to SAVE_MAX
 // particles that fill no more than half their slots); if anything did not fit, the window is
 // taken back and run with the compactions it asked for, so that it fails only where it did.
-// 10^4 electrons with compaction in each step: 152 -> 16 us a step.
+// 200 steps of 10^4 electrons with compaction in each: 33.8 -> 10.6 ms.
 static int run_window(pt_ctx* c, double& t, double dt, int q, int end, int every) {
     const ull all = c->hn[0] + c->hn[1] + c->hn[2];
     bool late = every > 0 && every < steps_per_launch(c) && end - end % every > q + every && !c->hp.wall.on &&
