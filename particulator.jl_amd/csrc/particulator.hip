@@ -2958,6 +2958,10 @@ enum {
 // fly): a beam of 2 x 10^6 photons and 10^5 electrons takes 168 against 256 ms.
 constexpr int WIDE = 768;
 constexpr ull WIDE_PER_LANE = 4;
+// (a launch of one step has no chains that long: from 1.5 per lane on, 8 such launches for
+// 3 x 10^5 electrons 1.62 -> 1.57 ms, 4 x 10^5 2.12 -> 1.72, 6 x 10^5 2.75 -> 1.97; 2 x 10^5
+// 1.32 -> 1.55)
+constexpr ull WIDE_PER_LANE_2 = 3;  // half a lane's electrons
 // the variant of a push/select kernel that evaluates learned samplers in place
 static int with_mlp(int v, bool mlp) { return mlp && v <= KV_QUEUE_FULL ? KV_RANGE_FULL_MLP + v : v; }
 static_assert(NKV <= MAX_KV, "residency table too small for the kernel variants");
@@ -3652,9 +3656,10 @@ static int ensure_queues(pt_ctx* c) {
 // 1500 per lane (10^8), where flying counts, 114/164 (3 steps).  Not in captured runs (`full`),
 // which may grow without the host knowing.
 enum { SHAPE_FULL = 0, SHAPE_WIDE = 1, SHAPE_LONE = 2 };
-static int pass_shape(const pt_ctx* c, bool full) {
+static int pass_shape(const pt_ctx* c, bool full, int steps = 0) {
     const ull electrons = c->hn[PT_ELECTRON] + c->hn[PT_POSITRON];
-    if (c->launch.block >= 256 && c->resident_wide > 0 && electrons >= WIDE_PER_LANE * WIDE * c->ncu) return SHAPE_WIDE;
+    const ull line = (!full && steps == 1 ? WIDE_PER_LANE_2 : 2 * WIDE_PER_LANE) * WIDE * c->ncu / 2;
+    if (c->launch.block >= 256 && c->resident_wide > 0 && electrons >= line) return SHAPE_WIDE;
     if (full || c->launch.grid_mult != 1) return SHAPE_FULL;
     const ull lanes = 256ull * c->ncu, photons = c->hn[PT_PHOTON];
     const bool beam = photons >= 4 * lanes && photons <= 128 * lanes && electrons <= std::min(photons / 8, 4 * lanes);
@@ -3663,9 +3668,9 @@ static int pass_shape(const pt_ctx* c, bool full) {
 
 // full: launch every resident workgroup x grid_mult (captured runs and queue rounds, whose
 // sizes the host does not know); otherwise at most what the last known population needs
-static int launch_kernel_args(pt_ctx* c, int v, bool full) {
+static int launch_kernel_args(pt_ctx* c, int v, bool full, int steps = 0) {
     void* args[] = {(void*)&c->dp};
-    const int shape = v == KV_RANGE_FULL ? pass_shape(c, full) : SHAPE_FULL;
+    const int shape = v == KV_RANGE_FULL ? pass_shape(c, full, steps) : SHAPE_FULL;
     const int bs = shape == SHAPE_WIDE ? WIDE : c->launch.block;
     const int per_cu = shape == SHAPE_WIDE ? c->resident_wide : c->resident[v][block_index(bs)];
     ull blocks = (ull)per_cu * c->ncu * std::max(1, c->launch.grid_mult);
@@ -3716,7 +3721,7 @@ static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int ns
     if (prof && (rc = mark(c, &e0))) return rc;
     const int in_place = wall ? KV_RANGE_WALL : with_mlp(KV_RANGE_FULL, mlp);
     if (R == 0) {
-        if ((rc = launch_kernel_args(c, in_place, clocked))) return rc;
+        if ((rc = launch_kernel_args(c, in_place, clocked, nsub))) return rc;
     } else {
         const bool mlp_ev = mlp_in_rounds(c);
         if ((rc = launch_kernel_args(c, with_mlp(KV_RANGE_EVENT, mlp_ev), clocked))) return rc;

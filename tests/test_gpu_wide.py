@@ -4,7 +4,7 @@ uid), collision counters and work counters must be equal, bit for bit, and the d
 to the order of its sums.
 
 Sizes lie on both sides of the rule (four electrons and positrons per lane of a launch of 256
-CUs: 786,432) and are ragged; the forms are those whose values the wide kernel reads from LDS
+CUs, 786,432; 1.5 in launches of one step) and are ragged; the forms are those whose values the wide kernel reads from LDS
 or memory instead of registers: one swarm's force, several swarms' forces and rate bounds, a
 magnetic field, functors, continuum loss, and electrons with positrons and photons."""
 import numpy as np
@@ -74,7 +74,8 @@ def run(form, n, steps, mode, block, seed=31, dt=1e-12):
 
 
 @pytest.mark.parametrize("form,n,steps,mode", [
-    ("uniform", LINE - 1, 3, "steps"), ("uniform", LINE, 3, "steps"), ("uniform", LINE + 12345, 8, "run"),
+    ("uniform", LINE * 3 // 8 - 1, 3, "steps"), ("uniform", LINE * 3 // 8, 3, "steps"),
+    ("uniform", LINE - 1, 3, "run"), ("uniform", LINE, 3, "run"), ("uniform", LINE + 12345, 8, "run"),
     ("uniform", LINE + 1, 9, "graph"), ("swarms", LINE + 77, 5, "run"), ("swarms, E across", LINE + 63, 3, "run"),
     ("swarms with B", LINE + 65, 3, "run"), ("swarms of functors", LINE + 7, 2, "run"),
     ("layer and loss", LINE + 129, 3, "graph"), ("no force on electrons", LINE + 5, 5, "run")])
