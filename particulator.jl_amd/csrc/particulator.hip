@@ -1472,7 +1472,7 @@ __global__ void k_tick(const Params* __restrict__ Pp) {
 // after a sampling round: its output queue becomes the input of the next push/select
 // round; the consumed input and the collision queues are emptied.  The secondary passes
 // that follow the rounds start where the step's secondaries start (the mark k_snapshot
-// set): a secondary stored when its lane's list was full, in any round, is advanced there;
+// set): a secondary stored when its wave's stack was full, in any round, is advanced there;
 // the others have reached the end of the step and are skipped.
 __global__ void k_rotate(const Params* __restrict__ Pp) {
     const Params& P = *Pp;
@@ -2949,7 +2949,8 @@ enum {
 // threads, three waves per SIMD instead of two (168 registers; a lane then reads its species'
 // constants, its force and its rate bounds from LDS each time).  The pass is bound by
 // instruction issue, and three waves hide more of one another's branches and LDS reads:
-// 24 steps of 10^7 electrons 42.3 -> 35.7 ms, 16 of 1.2 x 10^8 in 256 swarms 330 -> 259.
+// 24 steps of 10^7 electrons 44.9 -> 35.1 ms (42.3 in small workgroups with the second push
+// round), 48 of 10^6 10.7 -> 9.1, 16 of 1.2 x 10^8 in 256 swarms 333 -> 255.
 // With few electrons per lane the launch is as long as its longest lanes' collisions, and a
 // wave that shares its SIMD with two others takes 1.3 to 1.5 times as long for them: 32 steps
 // of n electrons took (two against three waves, ms) 3.15/3.54 for 3 x 10^5, 4.74/5.61 for
