@@ -811,8 +811,13 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
     const ull nwaves = (ull)gridDim.x * (blockDim.x >> 6);
     const int lanes = lanes_used(total, nwaves);
     const ull least = lanes < LEAST_CHUNK ? lanes : LEAST_CHUNK;
-    // (the first one fills the wave's lanes at once: each further claim is a round trip)
-    ull chunk = total / nwaves > 64 ? claim_chunk(4 * total, nwaves, least) : (ull)lanes;
+    // The first one fills the wave's lanes.  With one step a launch it is more, up to the wave's
+    // share, as each further claim is a round trip (2 x 10^5 electrons 6.8 -> 6.5 ms for 24
+    // such launches); an item of several steps takes far longer than that, and the waves end
+    // closer together if little is given out beforehand (32 swarms of 10^4 electrons 20.1 ->
+    // 18.9 ms, 1.2 x 10^6 7.3 -> 7.0; a beam of 2 x 10^6 photons, whose electrons no longer
+    // crowd in a wave's first items, 147 -> 124).
+    ull chunk = K == 1 && total / nwaves > 64 ? claim_chunk(4 * total, nwaves, least) : (ull)lanes;
     ull cbeg = 0, cend = 0;
     bool drained = false;
     // the wave's next chunk of items; false when they are all claimed
