@@ -3656,10 +3656,11 @@ static int ensure_queues(pt_ctx* c) {
 // 1.78/1.62 for 2 x 10^4 and 1.90/1.78 for 6 x 10^4, one step a launch 1.20/1.00; 8 x 10^4
 // electrons, with a second round for some lanes, 1.96/2.07.  Photons with few electrons are
 // such a case too, as most photons only fly and what takes long are the chains of the
-// electrons that a few set free: 10 steps of a beam of n photons took 154/141 for 5 x 10^5,
-// 187/152 for 2 x 10^6, 175/162 for 4 x 10^6 and (7 steps) 99/88 for 8 x 10^6; with 1.5
-// photons per lane, where their electrons crowd in half as many waves, 106/121, and with
-// 1500 per lane (10^8), where flying counts, 114/164 (3 steps).  Not in captured runs (`full`),
+// electrons that a few set free: 10 steps of a beam of n photons took 128/112 for 3 x 10^5,
+// 131/123 for 10^6, 139/125 for 2 x 10^6, 145/135 for 4 x 10^6 and (7 steps) 93/88 for
+// 8 x 10^6; with 1.5 photons per lane (10^5), where their electrons crowd in half as many
+// waves, 106/121, and with 1500 per lane (10^8), where flying counts, 114/164 (3 steps).
+// Not in captured runs (`full`),
 // which may grow without the host knowing.
 enum { SHAPE_FULL = 0, SHAPE_WIDE = 1, SHAPE_LONE = 2 };
 static int pass_shape(const pt_ctx* c, bool full, int steps = 0) {
