@@ -496,6 +496,11 @@ int pt_debug_collide(pt_ctx* ctx, int species, int proc, size_t n,
                      const double* u, int stride, int32_t* out_kind, int32_t* out_draws,
                      double* out_states, int32_t* out_species, uint64_t* out_uid);
 
+/* what the library chose by itself: out[0], out[1] threads and number of workgroups of the last
+ * main pass launched or captured with every collision in place, out[2] windows of pt_run that
+ * compacted late, out[3] how many of those were taken back and repeated */
+int pt_debug_choices(pt_ctx* ctx, int64_t out[4]);
+
 /* one forward/backward pass of the training kernels on a batch: loss and the gradient of
  * the FP32 parameters (X: B x 16 inputs, Y: B x 2 targets, output weights w0, w1) */
 int pt_debug_mlp_grad(pt_ctx* ctx, const float* params, const float* X, const float* Y, int B, float w0,

@@ -2770,6 +2770,9 @@ struct pt_ctx {
     int glds[2] = {0, 0};
     uint64_t ggen[2] = {0, 0};  // params_gen at capture
     uint64_t params_gen = 0;    // bumped by every upload of changed parameters
+    // for pt_debug_choices
+    int main_block = 0, main_grid = 0;
+    int64_t late_windows = 0, windows_back = 0;
     bool profile = false;
     hipEvent_t ev[8] = {};
     std::vector<hipEvent_t> evq;  // event pool of the profiling spans
@@ -3686,6 +3689,10 @@ static int launch_kernel_args(pt_ctx* c, int v, bool full, int steps = 0) {
         ull est = c->hn[0] + c->hn[1] + c->hn[2];
         blocks = std::min<ull>(blocks, std::max<ull>((ull)c->ncu, est / (ull)(bs / 64)));
     }
+    if (steps > 0) {
+        c->main_block = bs;
+        c->main_grid = (int)std::max<ull>(blocks, 1);
+    }
     HIPCHK(c, hipLaunchKernel(kernel_of(v, bs), dim3((unsigned)std::max<ull>(blocks, 1)), dim3(bs), args,
                               kernel_lds(c, v, bs), c->stream));
     return PT_OK;
@@ -3931,6 +3938,7 @@ static int run_window(pt_ctx* c, double& t, double dt, int q, int end, int every
     int rc;
     ull n[PT_NSPECIES] = {c->hn[0], c->hn[1], c->hn[2]};
     if (late && save_state(c, n, false) != PT_OK) late = false;  // no room for the copy
+    if (late) c->late_windows++;
     const double t1 = t;
     const uint32_t step1 = c->step;
     if ((rc = run_steps(c, t, dt, q, end, every, late))) return rc;
@@ -3939,6 +3947,7 @@ static int run_window(pt_ctx* c, double& t, double dt, int q, int end, int every
     rc = check_flags(c, nullptr);
     if (rc != PT_E_CAPACITY) return rc;
     if ((rc = save_state(c, n, true))) return rc;
+    c->windows_back++;
     t = t1;
     c->step = step1;
     if ((rc = run_steps(c, t, dt, q, end, every, false))) return rc;
@@ -4424,6 +4433,14 @@ int pt_debug_philox(pt_ctx* c, const uint32_t* ctr, const uint32_t key[2], uint3
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     HIPCHK(c, hipMemcpy(out, dout.p, sizeof(uint32_t) * 4 * n, hipMemcpyDeviceToHost));
+    return PT_OK;
+}
+
+int pt_debug_choices(pt_ctx* c, int64_t out[4]) {
+    if (!c) return PT_E_ARG;
+    if (!out) return fail(c, PT_E_ARG, "bad arguments");
+    const int64_t v[4] = {c->main_block, c->main_grid, c->late_windows, c->windows_back};
+    for (int q = 0; q < 4; q++) out[q] = v[q];
     return PT_OK;
 }
 

@@ -186,6 +186,7 @@ SIGNATURES = {
     "pt_synchronize": (C.c_int, [VP]),
     "pt_debug_philox": (C.c_int, [VP, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32),
                                   C.POINTER(C.c_uint32), C.c_size_t]),
+    "pt_debug_choices": (C.c_int, [VP, C.POINTER(C.c_int64)]),
     "pt_debug_uniforms": (C.c_int, [VP, C.c_uint64, C.c_uint32, DP, C.c_size_t]),
     "pt_debug_select": (C.c_int, [VP, C.c_int, C.c_size_t, DP, DP, C.POINTER(C.c_int32),
                                   C.POINTER(C.c_int32), C.POINTER(C.c_int32), DP]),
