@@ -3663,14 +3663,14 @@ static int ensure_queues(pt_ctx* c) {
 // 131/123 for 10^6, 139/125 for 2 x 10^6, 145/135 for 4 x 10^6 and (7 steps) 93/88 for
 // 8 x 10^6; with 1.5 photons per lane (10^5), where their electrons crowd in half as many
 // waves, 106/121, and with 1500 per lane (10^8), where flying counts, 114/164 (3 steps).
-// Not in captured runs (`full`),
-// which may grow without the host knowing.
+// Not in captured runs (`full`), which may grow without the host knowing, and not where the
+// caller asked for workgroups of 512 threads, which are two waves per SIMD each.
 enum { SHAPE_FULL = 0, SHAPE_WIDE = 1, SHAPE_LONE = 2 };
 static int pass_shape(const pt_ctx* c, bool full, int steps = 0) {
     const ull electrons = c->hn[PT_ELECTRON] + c->hn[PT_POSITRON];
     const ull line = (!full && steps == 1 ? WIDE_PER_LANE_2 : 2 * WIDE_PER_LANE) * WIDE * c->ncu / 2;
     if (c->launch.block >= 256 && c->resident_wide > 0 && electrons >= line) return SHAPE_WIDE;
-    if (full || c->launch.grid_mult != 1) return SHAPE_FULL;
+    if (full || c->launch.grid_mult != 1 || c->launch.block > 256) return SHAPE_FULL;
     const ull lanes = 256ull * c->ncu, photons = c->hn[PT_PHOTON];
     const bool beam = photons >= 4 * lanes && photons <= 128 * lanes && electrons <= std::min(photons / 8, 4 * lanes);
     return beam || electrons + photons <= lanes ? SHAPE_LONE : SHAPE_FULL;
@@ -3684,7 +3684,7 @@ static int launch_kernel_args(pt_ctx* c, int v, bool full, int steps = 0) {
     const int bs = shape == SHAPE_WIDE ? WIDE : c->launch.block;
     const int per_cu = shape == SHAPE_WIDE ? c->resident_wide : c->resident[v][block_index(bs)];
     ull blocks = (ull)per_cu * c->ncu * std::max(1, c->launch.grid_mult);
-    if (shape == SHAPE_LONE) blocks = std::min<ull>(blocks, (ull)c->ncu * std::max(1, 256 / bs));
+    if (shape == SHAPE_LONE) blocks = std::min<ull>(blocks, (ull)c->ncu * (256 / bs));
     if (!full) {
         ull est = c->hn[0] + c->hn[1] + c->hn[2];
         blocks = std::min<ull>(blocks, std::max<ull>((ull)c->ncu, est / (ull)(bs / 64)));

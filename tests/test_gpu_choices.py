@@ -55,6 +55,21 @@ def test_large_populations_run_in_wide_workgroups(mode, eighths, block):
         mp.close()
 
 
+@pytest.mark.parametrize("block", [128, 256, 512])
+def test_small_populations_run_on_one_wave_per_simd(block):
+    """A particle per lane of four waves on each CU or fewer; not beyond, not in captured runs,
+    and not in workgroups of 512 threads, eight waves each.  (The wide rule lies far above.)"""
+    line = 256 * cus()
+    for n in (1000, line, line + 1):
+        mp = electrons(n, block)
+        mp.run_steps(0.0, 1e-12, 2, check_every=2)
+        one = choices(mp)["waves"]
+        assert (one <= 4 * cus()) == (n <= line and block != 512), n
+        mp.run_graph(0.0, 1e-12, 8, check_every=8)
+        assert choices(mp)["waves"] > 4 * cus()
+        mp.close()
+
+
 def late(cap, n, dt, every, steps):
     cut = 600.0 * co.eV
     te, tg, tp = H.tables(dt=dt, cut=cut)
