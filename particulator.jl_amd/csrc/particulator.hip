@@ -2733,6 +2733,8 @@ struct pt_ctx {
     double* dtally = nullptr;
     double* ddose = nullptr;
     uint32_t step = 0;
+    double last_t = 0.0;      // final time of the step launched last
+    double lowest_rate = 0.0; // of an electron's collisions, over the intervals above the cut
     uint64_t next_uid = 0;
     int grid = 0;         // workgroups of the grid-stride utility kernels
     int ncu = 0;          // compute units
@@ -3252,6 +3254,15 @@ int pt_upload_table(pt_ctx* c, int sp, const pt_table_desc* t) {
             d.c[2] = 1.0 / d.B;
         }
     }
+    if (sp == PT_ELECTRON) {
+        c->lowest_rate = 0.0;
+        for (int i = 1; i <= k; i++) {
+            if (std::ldexp(t->xmax, i - k - 1) < t->energy_cut) continue;  // (the interval's lower end)
+            double rate = 0.0;  // the mean over the interval
+            for (int j = 0; j < t->nprocs; j++) rate += t->rate[((size_t)i * t->nprocs + j) * 3];
+            if (c->lowest_rate == 0.0 || rate < c->lowest_rate) c->lowest_rate = rate;
+        }
+    }
     // one collision queue per sampler kind present in the table
     Queues& Q = c->hp.q;
     for (int k = 0; k < 16; k++) Q.kq[sp][k] = -1;
@@ -3659,28 +3670,38 @@ static int ensure_queues(pt_ctx* c) {
 // 1.78/1.62 for 2 x 10^4 and 1.90/1.78 for 6 x 10^4, one step a launch 1.20/1.00; 8 x 10^4
 // electrons, with a second round for some lanes, 1.96/2.07.  Photons with few electrons are
 // such a case too, as most photons only fly and what takes long are the chains of the
-// electrons that a few set free: 10 steps of a beam of n photons took 128/112 for 3 x 10^5,
-// 131/123 for 10^6, 139/125 for 2 x 10^6, 145/135 for 4 x 10^6 and (7 steps) 93/88 for
-// 8 x 10^6; with 1.5 photons per lane (10^5), where their electrons crowd in half as many
-// waves, 106/121, and with 1500 per lane (10^8), where flying counts, 114/164 (3 steps).
+// electrons that a few set free.  From 4 photons per lane on (with 1.5, where their electrons
+// crowd in half as many waves, 10 steps of 1 ns took 106/121 ms) to 16 whatever the step (16
+// steps of 10^6 photons of 10 MeV: 0.76/0.68 of 1 ps, 2.4/2.3 of 10 ps, 38.1/38.1 of 100 ps, 8
+// of 1 ns 867/821), and to 128 if a step has room for many collisions: where the photons mostly
+// fly, the launch waits for memory and needs the waves.  Of 4 x 10^6 photons, 16 steps of 1 ps
+// took 1.52/1.90, of 10 ps 3.6/3.8, of 100 ps 42.5/42.0, 8 of 300 ps 109/105, of 600 ps 403/364, of
+// 1 ns 1033/942; of 8 x 10^6 2.5/3.5, 4.2/5.2, 45.6/45.0, 124/113, 437/391 and 1147/1025; of
+// 1.6 x 10^7, beyond the line, 4.3/6.6, 6.5/9.3, 50.9/59.2, 138/130, 488/441 and 1262/1216; 3 steps of
+// 10^8 114/164.  An electron collides 1.5 times a ps in air where its rate is lowest, so the
+// line lies at 200 collisions a step, 130 ps.  (Photons of 100 keV, whose electrons stop
+// early, gain less: 8 steps of 1 ns took 52.9/48.2 for 10^6, 64.1/65.0 for 4 x 10^6, 76/87 for
+// 8 x 10^6.)
 // Not in captured runs (`full`), which may grow without the host knowing, and not where the
 // caller asked for workgroups of 512 threads, which are two waves per SIMD each.
 enum { SHAPE_FULL = 0, SHAPE_WIDE = 1, SHAPE_LONE = 2 };
-static int pass_shape(const pt_ctx* c, bool full, int steps = 0) {
+constexpr double BEAM_COLLISIONS = 200.0;
+static int pass_shape(const pt_ctx* c, bool full, int steps = 0, double dt = 0.0) {
     const ull electrons = c->hn[PT_ELECTRON] + c->hn[PT_POSITRON];
     const ull line = (!full && steps == 1 ? WIDE_PER_LANE_2 : 2 * WIDE_PER_LANE) * WIDE * c->ncu / 2;
     if (c->launch.block >= 256 && c->resident_wide > 0 && electrons >= line) return SHAPE_WIDE;
     if (full || c->launch.grid_mult != 1 || c->launch.block > 256) return SHAPE_FULL;
     const ull lanes = 256ull * c->ncu, photons = c->hn[PT_PHOTON];
-    const bool beam = photons >= 4 * lanes && photons <= 128 * lanes && electrons <= std::min(photons / 8, 4 * lanes);
+    const ull most = dt * c->lowest_rate >= BEAM_COLLISIONS ? 128 * lanes : 16 * lanes;
+    const bool beam = photons >= 4 * lanes && photons <= most && electrons <= std::min(photons / 8, 4 * lanes);
     return beam || electrons + photons <= lanes ? SHAPE_LONE : SHAPE_FULL;
 }
 
 // full: launch every resident workgroup x grid_mult (captured runs and queue rounds, whose
 // sizes the host does not know); otherwise at most what the last known population needs
-static int launch_kernel_args(pt_ctx* c, int v, bool full, int steps = 0) {
+static int launch_kernel_args(pt_ctx* c, int v, bool full, int steps = 0, double dt = 0.0) {
     void* args[] = {(void*)&c->dp};
-    const int shape = v == KV_RANGE_FULL ? pass_shape(c, full, steps) : SHAPE_FULL;
+    const int shape = v == KV_RANGE_FULL ? pass_shape(c, full, steps, dt) : SHAPE_FULL;
     const int bs = shape == SHAPE_WIDE ? WIDE : c->launch.block;
     const int per_cu = shape == SHAPE_WIDE ? c->resident_wide : c->resident[v][block_index(bs)];
     ull blocks = (ull)per_cu * c->ncu * std::max(1, c->launch.grid_mult);
@@ -3735,7 +3756,7 @@ static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int ns
     if (prof && (rc = mark(c, &e0))) return rc;
     const int in_place = wall ? KV_RANGE_WALL : with_mlp(KV_RANGE_FULL, mlp);
     if (R == 0) {
-        if ((rc = launch_kernel_args(c, in_place, clocked, nsub))) return rc;
+        if ((rc = launch_kernel_args(c, in_place, clocked, nsub, dt))) return rc;
     } else {
         const bool mlp_ev = mlp_in_rounds(c);
         if ((rc = launch_kernel_args(c, with_mlp(KV_RANGE_EVENT, mlp_ev), clocked))) return rc;
@@ -3759,6 +3780,7 @@ static int launch_step(pt_ctx* c, bool clocked, double tfinal, double dt, int ns
         HIPCHK(c, hipGetLastError());
     } else {
         c->step += (uint32_t)nsub;
+        c->last_t = tfinal + (nsub - 1) * dt;
     }
     return PT_OK;
 }
@@ -3797,7 +3819,7 @@ int pt_advance(pt_ctx* c, double tfinal) {
     if (rc) return rc;
     // the main pass reports counts, flags and whether it left secondaries to further passes:
     // only then are those launched
-    rc = launch_step(c, false, tfinal, 0.0, 1, false);
+    rc = launch_step(c, false, tfinal, tfinal - c->last_t, 1, false);
     if (rc) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (c->report->left) {

@@ -11,7 +11,7 @@ import torch
 import helpers as H
 import oracle as O
 import particulator_hip as P
-from particulator_hip import co
+from particulator_hip import air, co
 from particulator_hip._lib import check, lib
 
 pytestmark = pytest.mark.gpu
@@ -68,6 +68,28 @@ def test_small_populations_run_on_one_wave_per_simd(block):
         mp.run_graph(0.0, 1e-12, 8, check_every=8)
         assert choices(mp)["waves"] > 4 * cus()
         mp.close()
+
+
+@pytest.mark.parametrize("mode", ["run", "advance"])
+@pytest.mark.parametrize("per_lane,more,dt,thin,one", [
+    (4, -1, 1e-9, 1.0, False), (4, 0, 1e-12, 1.0, True), (16, 0, 1e-12, 1.0, True), (16, 1, 1e-12, 1.0, False),
+    (16, 1, 1e-10, 1.0, False), (16, 1, 1e-9, 1.0, True), (16, 1, 1e-9, 1e-2, False), (128, 0, 1e-9, 1.0, True),
+    (128, 1, 1e-9, 1.0, False)])
+def test_beams_run_on_one_wave_per_simd(mode, per_lane, more, dt, thin, one):
+    """Photons and no electrons: from 4 per lane to 16 whatever the step, to 128 with long steps
+    in dense air"""
+    n = per_lane * 256 * cus() + more
+    comp = {k: v * thin for k, v in air.composition().items()}
+    te, tg, tp = H.tables(efield=0.0, dt=dt, comp=comp)
+    mp = H.make_device(te, tg, tp, 3, caps=(1 << 18, n + n // 16, 1 << 16))
+    mp.init_beam(1, n, 1e5 * co.eV)
+    mp.init()
+    if mode == "advance":
+        mp.advance(dt)
+    else:
+        mp.run_steps(0.0, dt, 2, check_every=2)
+    assert (choices(mp)["waves"] <= 4 * cus()) == one
+    mp.close()
 
 
 def late(cap, n, dt, every, steps):
