@@ -535,7 +535,7 @@ __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, cons
 // way to memory and back, the launches between steps and the wait for the step's slowest
 // wave.  10^7 electrons, 8 steps a launch: 2.50 -> 2.36 ms a step; 41,000 electrons: 253 ->
 // 168 us; a pencil beam of 2 x 10^6 photons, where the wait is for the electron with the most
-// collisions: 75 -> 26 ms (with the repeated pushes of D).
+// collisions: 75 -> 26 ms.
 //
 // Collisions are sampled in the lane.  The secondaries it stores go on a stack in LDS that
 // the wave's free lanes take from before new items; those that find it full are left to the
@@ -1140,7 +1140,6 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                 const V3 xo = x, po = p;
                 const double to = t;
                 V3 dx{0, 0, 0}, dp{0, 0, 0};
-                bool uniform;  // the force does not depend on the position
                 if (ffree) {
                     if constexpr (LEAN) {
                         const PT_LDS double* e = as_lds(pt_lds) + P.lds_field_off + field_doubles(P.forcing_off) * swarm;
@@ -1149,18 +1148,14 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                         F = V3{none || falong ? 0.0 : q * e[0], none || falong ? 0.0 : q * e[1], none ? 0.0 : q * e[2]};
                     }
                     push_uniform(sp, F, falong, p, dt, dx, dp);
-                    uniform = true;
                 } else if (P.field_lds) {
                     const PT_LDS double* fv = as_lds(pt_lds) + P.lds_field_off + field_doubles(P.forcing_off) * swarm;
                     const HomField hf{{fv}, {fv + 3}, {{nullptr, nullptr}}};
                     push_delta(sp, hf, x, p, dt, foff, dx, dp);
-                    uniform = true;
                 } else if (P.nswarm == 1) {
                     push_delta(sp, sh.field0, x, p, dt, foff, dx, dp);
-                    uniform = sp == PT_PHOTON;
                 } else {
                     push_delta(sp, as_global(P.fields)[swarm], x, p, dt, foff, dx, dp);
-                    uniform = sp == PT_PHOTON;
                 }
                 if (foff & off_push(sp)) {
                     dx = V3{0, 0, 0};  // only its time advances
@@ -1177,17 +1172,6 @@ __device__ __forceinline__ void select_loop(const Params& P, Shared& sh, PT_LDS 
                         n_events++;
                         cE = E;
                         pend = true;
-                    } else if (MULTI && !WALL && uniform && p.x == po.x && p.y == po.y && p.z == po.z) {
-                        // Below the cut a particle moves on in pushes of s / r until the step
-                        // ends (s is not drawn again, src/collisions.jl:151).  This push left
-                        // its momentum as it was and depends on nothing else, so the next
-                        // ones repeat it.
-                        while (trem > tnext && iters < ITER_LIMIT) {
-                            iters++;
-                            x = V3{x.x + dx.x, x.y + dx.y, x.z + dx.z};
-                            t = t + dt;
-                            trem -= dt;
-                        }
                     }
                 }
             }
