@@ -237,7 +237,16 @@ struct Shared : Staged {
     int nsub, pad;
 };
 
-constexpr size_t IMAGE_BYTES = 160 * 1024;  // a workgroup's LDS is no larger
+// what is staged in the dynamic LDS at most: the math table, three species' rates and process
+// records, and either one swarm's rate bounds and fields or the fields of many; the dose bins
+constexpr size_t table_doubles(int bounds, int swarms) {
+    return MATH_DOUBLES +
+           PT_NSPECIES * (MAX_INTERVALS * (MAX_PROCS * 3 + bounds) + SCAN_PAD + MAX_PROCS * sizeof(DevProc) / sizeof(double)) +
+           6 * swarms + DOSE_LDS + 2 + 2;
+}
+constexpr size_t MAX_TABLE_BYTES = sizeof(double) * std::max(table_doubles(3, 1), table_doubles(0, MAX_LDS_FIELDS));
+constexpr size_t IMAGE_BYTES = sizeof(Staged) + MAX_TABLE_BYTES;
+constexpr size_t LDS_BYTES = 160 * 1024;  // of a CU, and what a workgroup may have
 
 constexpr int IMAGE_BLOCKS = 32;  // one workgroup took 28 us, which each of many fields set in a row waits for
 __global__ void __launch_bounds__(256) k_build_image(const Params* __restrict__ Pp) {
@@ -2725,8 +2734,9 @@ struct pt_ctx {
     int lds_bytes = 0;
     Clock* dclock = nullptr;
     pt_launch launch{256, 1, 8, 0, 1u << PT_PROC_SB, 2, 0};
-    int resident[MAX_KV][3] = {};  // resident workgroups per CU: kernel variant x block 128/256/512
-    int resident_wide = 0;         // and of the wide history pass: 0 where its LDS does not fit
+    int resident[MAX_KV][3] = {};  // resident workgroups per CU: kernel variant x block 128/256/512 (0: no room)
+    int resident_wide = 0;         // and of the wide history pass
+    int tail_block = 512;          // threads of the one-workgroup passes
     bool queues = false;      // work and collision queues allocated
     int resident_lds = -1;        // LDS size the residency was computed for
     double* noalloc = nullptr;    // this device's copy of the allocation-free scratch array
@@ -2883,8 +2893,6 @@ static int sync_params(pt_ctx* c) {
     if (c->hp.dose_bins > 0 && c->hp.dose_bins <= DOSE_LDS) off += c->hp.dose_bins + 2;
     off = (off + 1) & ~1;
     c->hp.lds_doubles = off;
-    if (sizeof(Staged) + sizeof(double) * (size_t)off > IMAGE_BYTES)
-        return fail(c, PT_E_ARG, "the tables (%zu bytes) do not fit a workgroup's LDS", sizeof(double) * (size_t)off);
     c->lds_bytes = off * (int)sizeof(double);
     c->hp.lds_coop_off = (c->lds_bytes + 15) & ~15;
     HIPCHK(c, hipMemcpyAsync(c->dp, &c->hp, sizeof(Params), hipMemcpyHostToDevice, c->stream));
@@ -3591,6 +3599,19 @@ static bool mlp_in_rounds(const pt_ctx* c) {
            (c->hp.mlp[LEARN_MOLLER].on && !((dm >> PT_PROC_MOLLER) & 1u));
 }
 
+// A workgroup of 256 threads has room for the largest tables; one of 512 may have none, and the
+// kernel then runs with 256.  The runtime compares the dynamic LDS alone with a CU's: what
+// passes that and does not fit with the static LDS faults in the launch, so that every launch
+// beyond 256 threads goes by lds_fits.
+static_assert(MAX_TABLE_BYTES + (256 / 64) * COOP_WAVE_BYTES + sizeof(Shared) + 1024 <= LDS_BYTES,
+              "a workgroup of 256 threads takes every table that can be uploaded");
+static int lds_fits(pt_ctx* c, const void* kernel, size_t dynamic, bool* fits) {
+    hipFuncAttributes a;
+    HIPCHK(c, hipFuncGetAttributes(&a, kernel));
+    *fits = a.sharedSizeBytes + dynamic <= LDS_BYTES;
+    return PT_OK;
+}
+
 // dynamic LDS of a kernel variant: the rate tables (and for the push/select kernels the
 // per-wave RBEB job areas); the learned samplers' inference needs none
 static size_t kernel_lds(const pt_ctx* c, int v, int bs) {
@@ -3599,24 +3620,44 @@ static size_t kernel_lds(const pt_ctx* c, int v, int bs) {
     return (size_t)c->hp.lds_coop_off + (size_t)(bs / 64) * COOP_WAVE_BYTES;
 }
 
+// the one-workgroup passes over secondaries: plain, with walls, with learned samplers
+static const void* tail_kernel(int q) {
+    return q == 1 ? (const void*)k_tail<true, false> : q == 2 ? (const void*)k_tail<false, true>
+                                                              : (const void*)k_tail<false, false>;
+}
+static size_t tail_lds(const pt_ctx* c, int bs) {
+    return (size_t)c->hp.lds_coop_off + (size_t)(bs / 64) * COOP_WAVE_BYTES;
+}
+
 static int ensure_residency(pt_ctx* c) {
     const int key = 2 * c->lds_bytes + (mlp_any(c) ? 1 : 0);
     if (c->resident_lds == key) return PT_OK;
     const int bss[3] = {128, 256, 512};
+    int rc;
+    bool fits;
     for (int v = 0; v < NKV; v++)
         for (int bi = 0; bi < 3; bi++) {
+            const void* f = kernel_of(v, bss[bi]);
+            const size_t lds = kernel_lds(c, v, bss[bi]);
             int nb = 0;
-            HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel_of(v, bss[bi]), bss[bi],
-                                                                   kernel_lds(c, v, bss[bi])));
+            c->resident[v][bi] = 0;
+            if ((rc = lds_fits(c, f, lds, &fits))) return rc;
+            if (!fits) continue;
+            HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, bss[bi], lds));
             c->resident[v][bi] = std::max(nb, 1);
         }
-    // (tables that leave no room for it are no error)
     c->resident_wide = 0;
-    if (kernel_lds(c, KV_RANGE_FULL, WIDE) + sizeof(Shared) <= IMAGE_BYTES &&
+    if ((rc = lds_fits(c, kernel_of(KV_RANGE_FULL, WIDE), kernel_lds(c, KV_RANGE_FULL, WIDE), &fits))) return rc;
+    if (fits &&
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&c->resident_wide, kernel_of(KV_RANGE_FULL, WIDE), WIDE,
                                                      kernel_lds(c, KV_RANGE_FULL, WIDE)) != hipSuccess) {
         (void)hipGetLastError();
         c->resident_wide = 0;
+    }
+    c->tail_block = 512;
+    for (int q = 0; q < 3; q++) {
+        if ((rc = lds_fits(c, tail_kernel(q), tail_lds(c, 512), &fits))) return rc;
+        if (!fits) c->tail_block = 256;
     }
     c->resident_lds = key;
     return PT_OK;
@@ -3686,7 +3727,8 @@ static int pass_shape(const pt_ctx* c, bool full, int steps = 0, double dt = 0.0
 static int launch_kernel_args(pt_ctx* c, int v, bool full, int steps = 0, double dt = 0.0) {
     void* args[] = {(void*)&c->dp};
     const int shape = v == KV_RANGE_FULL ? pass_shape(c, full, steps, dt) : SHAPE_FULL;
-    const int bs = shape == SHAPE_WIDE ? WIDE : c->launch.block;
+    const int asked = c->launch.block == 512 && !c->resident[v][block_index(512)] ? 256 : c->launch.block;
+    const int bs = shape == SHAPE_WIDE ? WIDE : asked;
     const int per_cu = shape == SHAPE_WIDE ? c->resident_wide : c->resident[v][block_index(bs)];
     ull blocks = (ull)per_cu * c->ncu * std::max(1, c->launch.grid_mult);
     if (shape == SHAPE_LONE) blocks = std::min<ull>(blocks, (ull)c->ncu * (256 / bs));
@@ -3711,11 +3753,10 @@ static int launch_tail(pt_ctx* c) {
     const int in_place = wall ? KV_RANGE_WALL : with_mlp(KV_RANGE_FULL, mlp);
     for (int q = 0; q < c->launch.tail_passes; q++)
         if ((rc = launch_kernel_args(c, in_place, true))) return rc;
-    const size_t tail_lds = (size_t)c->hp.lds_coop_off + (size_t)(512 / 64) * COOP_WAVE_BYTES;
-    if (wall) hipLaunchKernelGGL((k_tail<true, false>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
-    else if (mlp) hipLaunchKernelGGL((k_tail<false, true>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
-    else hipLaunchKernelGGL((k_tail<false, false>), dim3(1), dim3(512), tail_lds, c->stream, c->dp, 100000);
-    HIPCHK(c, hipGetLastError());
+    int passes = 100000;
+    void* args[] = {(void*)&c->dp, (void*)&passes};
+    HIPCHK(c, hipLaunchKernel(tail_kernel(wall ? 1 : mlp ? 2 : 0), dim3(1), dim3(c->tail_block), args,
+                              tail_lds(c, c->tail_block), c->stream));
     return PT_OK;
 }
 
@@ -4019,6 +4060,7 @@ static int capture(pt_ctx* c, int which, int steps, bool compact) {
     int rc = ensure_residency(c);
     if (rc) return rc;
     if (c->launch.rounds > 0 && (rc = ensure_queues(c))) return rc;
+    if ((rc = ensure_residency(c))) return rc;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int lrc = PT_OK;
     for (int q = 0; q < steps && lrc == PT_OK;) {
