@@ -2708,15 +2708,11 @@ struct pt_ctx {
     Compaction cmp{};
     int cmp_blocks = 1;
     // a copy of the state at the start of a run's window (see run_window), kept from one
-    // window to the next and freed with the context
-    struct Saved {
-        double* f[PT_NSPECIES] = {};
-        uint8_t* active[PT_NSPECIES] = {};
-        uint64_t* uid[PT_NSPECIES] = {};
-        int32_t* swarm[PT_NSPECIES] = {};
-        ull cap[PT_NSPECIES] = {};  // particles each copy has room for
-        void* counters = nullptr;
-    } saved;
+    // window to the next, given back when another allocation needs the room, and freed with
+    // the context
+    char* saved = nullptr;
+    size_t saved_bytes = 0;
+    bool saved_live = false;  // a window may yet be taken back
     double* stat_part = nullptr;
     // counters
     ull* dcounts = nullptr;
@@ -2825,14 +2821,27 @@ static int noalloc_scratch(pt_ctx* c) {
     return PT_OK;
 }
 
-// device memory of its own, freed with the context
-static int dalloc_own(pt_ctx* c, void** p, size_t bytes) {
+// device memory; a window's copy of the state (see run_window) gives way to it
+static hipError_t dev_malloc(pt_ctx* c, void** p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes ? bytes : 8);
+    if (e != hipSuccess && c->saved && !c->saved_live) {
+        (void)hipGetLastError();
+        (void)hipFree(c->saved);  // (waits for the work that uses it)
+        c->saved = nullptr;
+        c->saved_bytes = 0;
+        e = hipMalloc(p, bytes ? bytes : 8);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();  // reported here: a later launch's check must not find it
         *p = nullptr;
-        return fail(c, PT_E_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     }
+    return e;
+}
+
+// device memory of its own, freed with the context
+static int dalloc_own(pt_ctx* c, void** p, size_t bytes) {
+    hipError_t e = dev_malloc(c, p, bytes);
+    if (e != hipSuccess) return fail(c, PT_E_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     c->allocs.push_back(*p);
     return PT_OK;
 }
@@ -2932,11 +2941,8 @@ struct Scratch {
 
 template <class T>
 static int dscratch(pt_ctx* c, Scratch<T>& s, size_t count) {
-    hipError_t e = hipMalloc((void**)&s.p, sizeof(T) * (count ? count : 1));
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
+    if (dev_malloc(c, (void**)&s.p, sizeof(T) * count) != hipSuccess)
         return fail(c, PT_E_NOMEM, "scratch allocation of %zu bytes failed", sizeof(T) * count);
-    }
     return PT_OK;
 }
 
@@ -3003,6 +3009,7 @@ void pt_destroy(pt_ctx* c) {
     for (auto& g : c->gexec)
         if (g) (void)hipGraphExecDestroy(g);
     for (void* p : c->allocs) (void)hipFree(p);
+    if (c->saved) (void)hipFree(c->saved);
     if (c->report) (void)hipHostFree(c->report);
     for (auto& e : c->ev)
         if (e) (void)hipEventDestroy(e);
@@ -3921,49 +3928,49 @@ static int run_steps(pt_ctx* c, double& t, double dt, int q, int end, int every,
 }
 
 // The state (particles, counters, tallies) copied aside, or back.
-constexpr ull SAVE_MAX = 1ull << 21;  // particles: 195 MB at most
+constexpr ull SAVE_MAX = 1ull << 21;  // particles of all species: their 93 bytes make 195 MB
 static int save_state(pt_ctx* c, const ull n[PT_NSPECIES], bool back) {
-    pt_ctx::Saved& v = c->saved;
-    int rc;
     Copies cp{};
-    auto add = [&](void* copy, void* live, size_t bytes) {
+    void* live[MAX_COPIES];
+    size_t at[MAX_COPIES], off = 0;  // places in the copy, 16-byte aligned
+    auto add = [&](void* p, size_t bytes) {
         if (!bytes) return;
-        cp.dst[cp.n] = back ? live : copy;
-        cp.src[cp.n] = back ? copy : live;
+        live[cp.n] = p;
+        at[cp.n] = off;
         cp.bytes[cp.n++] = bytes;
+        off += (bytes + 15) & ~(size_t)15;
     };
+    ull all = 0;
     for (int s = 0; s < PT_NSPECIES; s++) {
-        if (n[s] == 0) continue;
-        if (v.cap[s] < n[s]) {
-            const ull room = std::min<ull>(c->cfg.capacity[s], std::max<ull>(2 * n[s], 4096));
-            void** old[4] = {(void**)&v.f[s], (void**)&v.active[s], (void**)&v.uid[s], (void**)&v.swarm[s]};
-            const size_t size[4] = {sizeof(double) * PT_NFIELDS, 1, sizeof(uint64_t), sizeof(int32_t)};
-            v.cap[s] = 0;
-            for (int q = 0; q < 4; q++) {
-                if (*old[q]) {
-                    auto it = std::find(c->allocs.begin(), c->allocs.end(), *old[q]);
-                    if (it != c->allocs.end()) c->allocs.erase(it);
-                    HIPCHK(c, hipFree(*old[q]));
-                    *old[q] = nullptr;
-                }
-                if ((rc = dalloc_own(c, old[q], size[q] * room))) return rc;
-            }
-            v.cap[s] = room;
-        }
         const SpeciesDev& S = c->hp.sp[s];
-        add(v.f[s], S.f[0], sizeof(double) * PT_NFIELDS * n[s]);
-        add(v.active[s], S.active, n[s]);
-        add(v.uid[s], S.uid, sizeof(uint64_t) * n[s]);
-        add(v.swarm[s], S.swarm, sizeof(int32_t) * n[s]);
+        all += n[s];
+        add(S.f[0], sizeof(double) * PT_NFIELDS * n[s]);
+        add(S.active, n[s]);
+        add(S.uid, sizeof(uint64_t) * n[s]);
+        add(S.swarm, sizeof(int32_t) * n[s]);
     }
-    const size_t bytes[6] = {sizeof(ull) * PT_NSPECIES, sizeof(ull) * PT_NSPECIES * NCOUNT, sizeof(ull) * NFLAGS,
-                             sizeof(ull) * NWORK, sizeof(double) * PT_NSPECIES * (c->hp.tally_bins + 2),
-                             sizeof(double) * (c->hp.dose_bins + 3)};
-    void* live[6] = {c->dn, c->dcounts, c->dflags, c->dwork, c->dtally, c->ddose};
-    size_t off[7] = {0};
-    for (int q = 0; q < 6; q++) off[q + 1] = off[q] + ((bytes[q] + 15) & ~(size_t)15);
-    if (!v.counters && (rc = dalloc(c, &v.counters, off[6]))) return rc;
-    for (int q = 0; q < 6; q++) add((char*)v.counters + off[q], live[q], bytes[q]);
+    add(c->dn, sizeof(ull) * PT_NSPECIES);
+    add(c->dcounts, sizeof(ull) * PT_NSPECIES * NCOUNT);
+    add(c->dflags, sizeof(ull) * NFLAGS);
+    add(c->dwork, sizeof(ull) * NWORK);
+    add(c->dtally, sizeof(double) * PT_NSPECIES * (c->hp.tally_bins + 2));
+    add(c->ddose, sizeof(double) * (c->hp.dose_bins + 3));
+    if (c->saved_bytes < off) {
+        // room for half as many particles again, within the bound
+        const size_t room = off + 93 * (size_t)std::min<ull>(std::max<ull>(all / 2, 4096), SAVE_MAX - all);
+        if (c->saved) {
+            HIPCHK(c, hipFree(c->saved));
+            c->saved = nullptr;
+            c->saved_bytes = 0;
+        }
+        if (dev_malloc(c, (void**)&c->saved, room) != hipSuccess)
+            return fail(c, PT_E_NOMEM, "no room for a copy of %zu bytes", room);
+        c->saved_bytes = room;
+    }
+    for (int q = 0; q < cp.n; q++) {
+        cp.dst[q] = back ? live[q] : c->saved + at[q];
+        cp.src[q] = back ? c->saved + at[q] : live[q];
+    }
     hipLaunchKernelGGL(k_copy_ranges, dim3(c->grid), dim3(256), 0, c->stream, cp);
     HIPCHK(c, hipGetLastError());
     return PT_OK;
@@ -3986,6 +3993,11 @@ static int run_window(pt_ctx* c, double& t, double dt, int q, int end, int every
     ull n[PT_NSPECIES] = {c->hn[0], c->hn[1], c->hn[2]};
     if (late && save_state(c, n, false) != PT_OK) late = false;  // no room for the copy
     if (late) c->late_windows++;
+    c->saved_live = late;
+    struct Release {
+        bool& live;
+        ~Release() { live = false; }
+    } release{c->saved_live};
     const double t1 = t;
     const uint32_t step1 = c->step;
     if ((rc = run_steps(c, t, dt, q, end, every, late))) return rc;
@@ -4461,11 +4473,8 @@ int pt_synchronize(pt_ctx* c) {
 #define SCRATCH(c, var, T, count)                                                             \
     Scratch<T> var;                                                                           \
     do {                                                                                      \
-        hipError_t e_ = hipMalloc((void**)&var.p, sizeof(T) * ((count) ? (count) : 1));      \
-        if (e_ != hipSuccess) {                                                               \
-            (void)hipGetLastError();                                                          \
+        if (dev_malloc((c), (void**)&var.p, sizeof(T) * (count)) != hipSuccess)               \
             return fail((c), PT_E_NOMEM, "scratch allocation failed");                        \
-        }                                                                                     \
     } while (0)
 
 int pt_debug_philox(pt_ctx* c, const uint32_t* ctr, const uint32_t key[2], uint32_t* out, size_t n) {
