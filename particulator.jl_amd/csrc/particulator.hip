@@ -3141,16 +3141,15 @@ int pt_create(const pt_config* cfg, pt_ctx** out) {
     for (int s = 0; s < PT_NSPECIES; s++) {
         const size_t cap = c->cfg.capacity[s], chunks = (cap + CH - 1) / CH + 1;
         c->cmp.sp[s] = P.sp[s];
-        const size_t size[5] = {chunks, chunks, chunks, cap / 2 + 1, cap / 2 + 1};
-        unsigned** part[5] = {&c->cmp.cnt[s], &c->cmp.hole[s], &c->cmp.tail[s], &c->cmp.hpos[s], &c->cmp.tpos[s]};
-        size_t words = 0;
-        for (size_t v : size) words += (v + 63) & ~(size_t)63;
+        unsigned** part[3] = {&c->cmp.cnt[s], &c->cmp.hole[s], &c->cmp.tail[s]};
+        const size_t words = (chunks + 63) & ~(size_t)63;
         unsigned* base = nullptr;
-        TRY(dalloc(c, (void**)&base, sizeof(unsigned) * words));
-        for (int q = 0; q < 5; q++) {
-            *part[q] = base;
-            base += (size[q] + 63) & ~(size_t)63;
-        }
+        TRY(dalloc(c, (void**)&base, 3 * sizeof(unsigned) * words));
+        for (int q = 0; q < 3; q++) *part[q] = base + q * words;
+        // the lists of positions lie in the column of times left, which is in use only within a
+        // step of collision rounds
+        c->cmp.hpos[s] = (unsigned*)P.sp[s].trem;
+        c->cmp.tpos[s] = c->cmp.hpos[s] + cap / 2 + 1;
         most = std::max(most, chunks);
     }
     TRY(dalloc(c, (void**)&c->cmp.info, sizeof(ull) * 4 * PT_NSPECIES));
