@@ -283,9 +283,18 @@ __device__ __forceinline__ uint64_t child_uid(uint64_t seed, uint64_t uid, uint3
     return ((uint64_t)b << 32) | a;
 }
 
+// -log(u) of a draw: a stream's are in (0, 1), an injected one may be zero
+template <class G>
+__device__ __forceinline__ double neg_log(double u, G& g) {
+    return -log_tab(u, g.tab());
+}
+__device__ __forceinline__ double neg_log(double u, InjectedStream& g) {
+    return u == 0.0 ? __builtin_inf() : -log_tab(u, g.tab());
+}
+
 template <class G>
 __device__ __forceinline__ double nextcoll(G& g) {  // src/util.jl:17
-    return -log_tab(g.next(), g.tab());
+    return neg_log(g.next(), g);
 }
 
 // ---------------------------------------------------------------- kinematics
@@ -1146,8 +1155,8 @@ __device__ __forceinline__ void finish_event(const V3& p, double pnorm, const Ev
     const bool need1 = e.ne == 2 && !drop1 && stored(e.sp1, m1);
     double q0, q1;
     g.next12(e.ne == 2 ? 2 : 1, q0, q1);  // both draws at one place
-    s0 = need0 ? -log_tab(q0, g.tab()) : 0.0;  // nextcoll(), src/util.jl:17
-    s1 = need1 ? -log_tab(q1, g.tab()) : 0.0;
+    s0 = need0 ? neg_log(q0, g) : 0.0;  // nextcoll(), src/util.jl:17
+    s1 = need1 ? neg_log(q1, g) : 0.0;
 }
 
 // What the common event needs of its process record, in registers.

@@ -82,3 +82,13 @@ def test_azimuth():
         # (np.longdouble's sine and cosine are good to 2^-63; beside their zeros what counts is
         # the argument, exact here)
         assert np.max(np.abs(got - want) / np.maximum(np.abs(want), L(2) ** -60)) <= 4 * 2.0 ** -53
+
+
+def test_zero_draws_as_ieee_has_them():
+    """An injected uniform of zero (a stream never yields one): no interval to the next
+    collision is finite; the smallest numbers have theirs."""
+    tiny = np.array([0.0, 5e-324, 1e-310, 2.3e-308])
+    s = elastic(uniforms(tiny.size, last=tiny))[:, 8]
+    assert s[0] == np.inf
+    want = -np.log(tiny[1:].astype(L))
+    assert np.allclose(s[1:].astype(L), want, rtol=1e-15, atol=0.0)
