@@ -4238,8 +4238,11 @@ int pt_autotune(pt_ctx* c, double t0, double dt, int trial_steps, pt_tune_trial*
         }
         c->launch = top;
     }
+    // (a block that leads to the launches of a smaller one, as 512 does to those of 256 for a
+    // large population, is not chosen over it: what differs is noise)
     double top_rate = -1.0;
     const int blocks[3] = {128, 256, 512}, mults[3] = {1, 2, 4};
+    std::vector<std::pair<int, int>> shapes;
     for (int bi = 0; bi < 3 && rc == PT_OK; bi++)
         for (int mi = 0; mi < 3 && rc == PT_OK; mi++) {
             c->launch.block = blocks[bi];
@@ -4249,7 +4252,10 @@ int pt_autotune(pt_ctx* c, double t0, double dt, int trial_steps, pt_tune_trial*
             if (rc) break;
             if (trials && nt < max_trials) trials[nt] = pt_tune_trial{c->launch, r};
             nt++;
-            if (r > top_rate) {
+            const std::pair<int, int> shape{c->main_block, c->main_grid};
+            const bool seen = c->launch.rounds == 0 && std::find(shapes.begin(), shapes.end(), shape) != shapes.end();
+            shapes.push_back(shape);
+            if (r > top_rate && !seen) {
                 top_rate = r;
                 top = c->launch;
             }

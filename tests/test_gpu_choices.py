@@ -92,6 +92,16 @@ def test_beams_run_on_one_wave_per_simd(mode, per_lane, more, dt, thin, one):
     mp.close()
 
 
+def test_autotuner_keeps_the_smaller_of_equal_launches():
+    """A large population runs the same wide workgroups for 256 and 512: the trials of 512 are
+    repetitions, and none of their rates, differing by noise, is chosen."""
+    mp = electrons(4 * 768 * cus() + 100_000, 256)
+    best, trials, _ = mp.autotune(0.0, 1e-13, trial_steps=2)
+    assert [t["block"] for t in trials[4:13]] == [128] * 3 + [256] * 3 + [512] * 3
+    assert best["block"] != 512 or best["rounds"] > 0
+    mp.close()
+
+
 def late(cap, n, dt, every, steps):
     cut = 600.0 * co.eV
     te, tg, tp = H.tables(dt=dt, cut=cut)
