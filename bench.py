@@ -11,10 +11,12 @@ null-collision selection, sampling, secondary append and the secondaries' own pa
 Metric: particle-steps/s = sum over timed steps of the active particles at step start,
 divided by the wall time of the timed loop (inputs resident in HBM, tables uploaded).
 
-Prints one JSON line.  `roofline` prices the main advance kernel with the algorithmic HBM
-bytes of its launches (165 B per particle-step + 93 B per appended secondary; a launch takes
-its particles through several steps and moves their state once) over its average launch
-duration measured with HIP events on the library's stream.  `cpu_baseline`
+Prints one JSON line.  `roofline` names what bounds the main advance kernel, the issue of
+vector instructions: those it issues per second (counted by rocprofv3 over a short run of the
+same workload) against one wave instruction per SIMD in four cycles.  Its `hbm` entry gives
+the bytes the launches cannot do without (a launch takes its particles through several steps
+and moves each one's state once, 165 B, and writes 93 B per appended secondary) over the
+average launch duration measured with HIP events on the library's stream.  `cpu_baseline`
 times the CPU restatement of the reference step (oracle/, OpenMP over the host cores) on a
 bounded sample of the same workload.
 """
@@ -28,12 +30,35 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(ROOT, "particulator.jl_amd"))
 
 HBM_PEAK_GBPS = 8000.0
-# a particle-step reads the particle (10 FP64, uid, swarm, active flag: 93 B) and writes
-# back position, momentum, t, s and r (9 FP64: 72 B); an appended secondary writes a whole
-# particle (93 B)
-BYTES_PER_PSTEP = 165.0
+# a launch reads each particle (10 FP64, uid, swarm, active flag: 93 B) and writes back
+# position, momentum, t, s and r (9 FP64: 72 B), however many steps it advances it; an
+# appended secondary writes a whole particle (93 B)
+BYTES_PER_PARTICLE = 165.0
 BYTES_PER_SECONDARY = 93.0
-BYTES_PER_MOVE = 186.0
+# one FP64 vector instruction of a wave takes a SIMD four cycles; 4 SIMDs a CU, 2.4 GHz at most
+CLOCK_GHZ, CYCLES_PER_INSTRUCTION = 2.4, 4.0
+
+
+def launch_bytes(psteps, secondaries, steps, launches):
+    """bytes that the average of `launches` launches over `steps` steps has to move, with
+    `psteps` particle-steps and `secondaries` in all"""
+    return BYTES_PER_PARTICLE * psteps / max(steps, 1) + BYTES_PER_SECONDARY * secondaries / max(launches, 1)
+
+
+def roofline(psteps, secondaries, steps, launches, avg_launch_ms, rate, traffic):
+    valu = (traffic or {}).get("valu") or {}
+    per_pstep, simds = valu.get("wave_instructions_per_particle_step"), valu.get("simds")
+    nbytes = launch_bytes(psteps, secondaries, steps, launches)
+    gbps = nbytes / (avg_launch_ms * 1e-3) / 1e9
+    peak = simds * CLOCK_GHZ / CYCLES_PER_INSTRUCTION if simds else None
+    achieved = per_pstep * rate / 1e9 if per_pstep else None
+    return {"bound": "vector instruction issue", "achieved": achieved, "peak": peak,
+            "unit": "1e9 wave instructions/s", "frac": achieved / peak if achieved and peak else None,
+            "traffic": traffic["bytes"] if traffic else None, "kernel": "k_advance (in-place collisions)",
+            "avg_launch_ms": avg_launch_ms, "steps_per_launch": steps / max(launches, 1),
+            "hbm": {"algorithmic_bytes_per_launch": nbytes, "achieved": gbps, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
+                    "frac": gbps / HBM_PEAK_GBPS},
+            "traffic_source": traffic}
 
 WORKLOADS = {
     "avalanche": dict(n=10_000_000, e1=1e5, e2=1e7, loguniform=True, efield=1e6, dt=1e-12,
@@ -212,8 +237,6 @@ def main():
     psteps = w.particle_steps
     value = psteps / el
     adv_avg_ms = w.advance_ms / max(w.advance_launches, 1)
-    adv_bytes = (BYTES_PER_PSTEP * psteps + BYTES_PER_SECONDARY * w.main_secondaries) / max(w.advance_launches, 1)
-    achieved = adv_bytes / (adv_avg_ms * 1e-3) / 1e9
     log("timed %d steps in %.3f s: %.4g particle-steps/s; advance %.3f ms/launch, tail %.3f ms, "
         "compact %.3f ms total; populations %s; events/pstep %.2f; secondaries %d"
         % (args.steps, el, value, adv_avg_ms, w.tail_ms / max(w.advance_launches, 1), w.compact_ms,
@@ -233,12 +256,7 @@ def main():
         "data": "synthetic (device-generated initial particles from a seeded Philox stream)",
         "config": {"workload": wl["name"], "initial_particles": n, "seed": args.seed,
                    "population_end": counts, "events_per_particle_step": w.events / max(psteps, 1)},
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic["bytes"] if traffic else None,
-                     "kernel": "k_advance (in-place collisions)", "avg_launch_ms": adv_avg_ms,
-                     "algorithmic_bytes_per_launch": adv_bytes,
-                     "steps_per_launch": args.steps / max(w.advance_launches, 1),
-                     "traffic_source": traffic},
+        "roofline": roofline(psteps, w.main_secondaries, args.steps, w.advance_launches, adv_avg_ms, value, traffic),
     }
     mp.close()
     nets = {}
@@ -341,7 +359,7 @@ def pmc_traffic(args):
                        "wave_instructions_per_particle_step": v["SQ_INSTS_VALU"] / (n0 * steps_per_launch),
                        "lane_utilisation": v["SQ_THREAD_CYCLES_VALU"] / (64.0 * v["SQ_ACTIVE_INST_VALU"]),
                        "wait_fraction": v["SQ_WAIT_ANY"] / v["SQ_WAVE_CYCLES"],
-                       "waves_per_simd": waves_per_simd,
+                       "simds": simds, "waves_per_simd": waves_per_simd,
                        "simd_valu_busy": v["SQ_ACTIVE_INST_VALU"] * waves_per_simd / v["SQ_WAVE_CYCLES"],
                        "note": "the main passes of the same 24-step run: SQ_THREAD_CYCLES_VALU / "
                                "(64 SQ_ACTIVE_INST_VALU), SQ_WAIT_ANY / SQ_WAVE_CYCLES; simd_valu_busy = "
