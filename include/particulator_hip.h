@@ -155,7 +155,7 @@ typedef struct {
 typedef struct {
     uint64_t particle_steps;     /* active particles at step start, summed over steps */
     uint64_t secondaries;        /* particles appended to a population */
-    uint64_t moved;              /* particles moved by compaction */
+    uint64_t moved;              /* particles moved by the compactions that ran (pt_run) */
     uint64_t events;             /* real + null collision events */
     uint64_t steps;
     uint64_t tail_particles;     /* secondaries advanced within their birth step */
@@ -288,7 +288,14 @@ int pt_init(pt_ctx* ctx);
  * of the random streams advances by one. */
 int pt_advance(pt_ctx* ctx, double tfinal);
 /* `nsteps` calls of pt_advance at t0 + dt, t0 + 2dt, ..., with pt_compact every
- * `compact_every` steps (0: never) and error checks every `check_every` steps. */
+ * `compact_every` steps (0: never) and error checks every `check_every` steps.
+ * Up to 16 steps run in one launch; where several compactions fall among the steps of a
+ * launch, one at its end may stand for them.  The particles are the same, and a population
+ * fails to fit only where it would with every compaction in its place; but the slots that
+ * particles have (their order in pt_download) and pt_work.moved follow the compactions that
+ * ran.  The context keeps a copy of the state for that (of at most 2^21 particles that fill no
+ * more than half their slots: up to 195 MB, and the tallies) and runs the steps since the
+ * last check again, compacting as asked, if something did not fit. */
 int pt_run(pt_ctx* ctx, double t0, double dt, int nsteps, int compact_every, int check_every);
 /* repack! (src/population.jl:229-259): fill holes below the active count with active
  * particles from the end (not order preserving, as in the reference). */

@@ -1,10 +1,10 @@
 // particulator.hip -- kernels and C ABI of the null-collision Monte Carlo step on
 // MI355X (gfx950).
 //
-// Data layout in HBM (per species): ten FP64 columns x,y,z,px,py,pz,w,t,s,r, a u8 active
-// column, a u64 uid column and an i32 swarm column, each `capacity` long (structure of
-// arrays: every wave reads 64 consecutive doubles per field, fully coalesced).  A device
-// counter n holds the slots in use; secondaries are appended at n with an atomic claim.
+// Data layout in HBM (per species): records of ten FP64 fields x,y,z,px,py,pz,w,t,s,r (80
+// bytes a slot), and columns of a u8 active flag, a u64 uid and an i32 swarm, each `capacity`
+// long.  A device counter n holds the slots in use; secondaries are appended at n with an
+// atomic claim.
 //
 // One step (pt_advance), or up to MAX_SUB steps of a run in one launch:
 //   k_snapshot   -- pass range [0, n) of every species (the advance_init!/iup state) and the
@@ -372,10 +372,12 @@ __device__ __forceinline__ double setr(const SpLite& L, double E, int swarm, boo
 // The selection scan of do_one_collision! (src/collisions.jl:160-186): the first process j
 // whose rate exceeds what is left of xi after subtracting the rates of processes 0..j-1, that
 // is, the first whose cumulative rate exceeds xi; np or more for a null collision.  The row
-// holds the coefficients of the cumulative rates, so a process costs two FMAs, a comparison
-// and a selection, and nothing is carried from one to the next.  A group may run past the
-// row's end into the next row or the table's padding (SCAN_PAD): what it finds there stands
-// for the null collision.
+// holds the coefficients of the cumulative rates, so a process costs two multiplications, two
+// additions, a comparison and a selection, and nothing is carried from one to the next.  A
+// group may run past the row's end into the next row or the table's padding (SCAN_PAD): what
+// it finds there stands for the null collision.  (The sums differ from those of subtracting
+// one rate after another by rounding: a draw within that of a cumulative rate may fall on
+// the other side.)
 __device__ __forceinline__ int select_process(const PT_LDS double* rt, int np, double t1, double t2, double xi) {
     constexpr int G = SCAN_GROUP;
     int sel = np;
@@ -564,8 +566,8 @@ __device__ __forceinline__ ull append(const Params& P, Shared& sh, int sp2, cons
 // lane moves on.  The sampling kernel then runs each queued kind with whole waves of the
 // same kind (no divergence between samplers; the learned samplers need it).
 // Items a wave claims at a time: 128 in workgroups of up to 256 threads, 256 in larger ones
-// (the faster size for each launch shape the autotuner picks: the avalanche's 256-thread
-// and the sweep's 512-thread workgroups), and a quarter of the wave's share of what is left
+// (512, and the 768 of large populations; 64 and 128 there: 16.35 and 19.2 ms against 16.1 for
+// 8 launches of one step of 10^7 electrons), and a quarter of the wave's share of what is left
 // when that is less, so that the waves end together.
 constexpr ull LEAST_CHUNK = 16;
 __device__ __forceinline__ ull claim_chunk(ull left, ull nwaves, ull least) {

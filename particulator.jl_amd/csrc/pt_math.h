@@ -77,8 +77,10 @@ PT_HD double flip_sign(double x, uint32_t signbit) {
 }
 #endif
 
-// sqrt(x): one Goldschmidt step from the hardware's 1/sqrt(x), then two corrections of the
-// root by its exact remainder
+// sqrt(x): one step of Goldschmidt's iteration from the hardware's 1/sqrt(x), then two
+// corrections of the root by its exact remainder (P. Markstein, "Software division and square
+// root using Goldschmidt's algorithms", Proc. 6th Conf. on Real Numbers and Computers (2004)
+// 146-157)
 PT_HD double qsqrt(double x) {
     const double y = approx_rsq(x);
     double g = x * y, h = 0.5 * y;

@@ -2,10 +2,11 @@
 
 Flags: -ffp-contract=off keeps the reference's unfused multiply/add order on the selection
 and push paths; packed-FP32 instructions are disabled.  Machine LICM is disabled: in the
-step kernel it hoists the 64-bit polynomial constants of log and sincos out of the
-particle loop into vector registers, which then spill to scratch (256 VGPRs and 84 B of
-spills per lane, reloaded on every collision); without it the kernel needs 187 VGPRs and no
-scratch, and the step runs about 9% faster.  The max-ILP machine scheduler adds about 1%.
+step kernel it hoists 64-bit constants and table offsets out of the particle loop into vector
+registers, which then spill to scratch and are reloaded on every collision.  Without it the
+kernel of two waves per SIMD takes 199 VGPRs and spills none (67 SGPRs go to VGPR lanes); that
+of three takes all of its 168, with 6 VGPRs spilled to scratch and 82 SGPRs to lanes.  The
+max-ILP machine scheduler adds about 1%.
 """
 import os
 import subprocess
