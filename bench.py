@@ -403,7 +403,7 @@ def run_beam(args):
     counts = [mp.count(s) for s in range(3)]
     value = w.particle_steps / el
     log("beam: %d steps in %.3f s: %.4g particle-steps/s, %.4g collision events/s; populations %s; "
-        "dose %.4g J; photon births %d; advance %.1f ms/step, last-workgroup tail %.1f ms/step, secondaries "
+        "dose %.4g J; photon births %d; advance %.1f ms/launch, last-workgroup tail %.1f ms/launch, secondaries "
         "advanced in their birth step %d" % (steps, el, value, w.events / el, counts, total, c1,
                                              w.advance_ms / max(w.advance_launches, 1),
                                              w.tail_ms / max(w.advance_launches, 1), w.tail_particles))
